@@ -1194,6 +1194,7 @@ struct evp1d_handle {
   // fused form: tiling and its device tables (owned here, replaced on relayout)
   int tile_w = 64, tile_h = 16, tile_block = 512, tile_xcd = 1;
   bool tiling_auto = true;         // choose the tile from the domain size (until evp1d_set_tiling)
+  bool crowded_checked = false;    // the chosen tile needs no look at its busiest tile's level-2 points
   evp1d::GridCoords coords;        // grid coordinates of the current lists
   bool coords_ok = false;
   evp1d::TileIds tile_cache;       // tile of every point for the current lists and tile size
@@ -1541,26 +1542,46 @@ static int relayout_impl(evp1d_handle *h) {
     h->tile_cache_ok = false;
   }
   if (h->tiling_auto && !h->tile_cache_ok) {
-    // one subcycle per launch: enough tiles to fill the GPU, the largest
-    // tile of the ladder that still gives min_tiles tiles (256 CUs); the
-    // pair form: 31x19 cells, the tuner's choice from 84k to 5.4M points
-    // (at most 640 level-2 stress points per tile: one 512- or 1024-thread
-    // workgroup; one subcycle per launch on the same tiles where the pair
-    // tables do not fit)
-    struct Rung { int w, h, block, min_tiles; };
-    static const Rung ladder[3] = {{64, 16, 512, 1024}, {32, 8, 256, 512}, {16, 8, 128, 0}};
-    static const Rung pair_rung = {31, 19, 512, 0};
-    const Rung *rungs = h->fused_depth == 2 ? &pair_rung : ladder;
-    const int nrungs = h->fused_depth == 2 ? 1 : 3;
+    // The first rung of a ladder that gives at most `most` tiles, or at least
+    // `least`.
+    // Pair form: a tile's time is its chain of four phases, whatever runs
+    // beside it, until the 256 CUs are full.  So with at most one tile per CU
+    // the smallest tile is the fastest: in 15x11 every phase is one pass of
+    // 256 threads (18x14 cells at level 1), in 22x16 one of 512.  Measured,
+    // 31x19 / chosen, us per subcycle: 64x48 5.3 / 4.0, 200x150 6.2 / 4.1,
+    // 300x220 6.9 / 5.9, 520x400 11.1 / 10.3 (31x15).  Beyond two tiles per
+    // CU the border's extra work counts: 31x19.
+    // One subcycle per launch: the largest tile that still fills the GPU.
+    struct Rung { int w, h, block, most, least; };
+    constexpr int kCus = 256;
+    static const Rung ladder[3] = {{64, 16, 512, 0, 1024}, {32, 8, 256, 0, 512}, {16, 8, 128, 0, 0}};
+    static const Rung pairs[5] = {{15, 11, 256, kCus, 0}, {22, 16, 512, kCus, 0}, {31, 19, 512, kCus, 0},
+                                  {31, 15, 512, 2 * kCus, 0}, {31, 19, 512, 0, 0}};
+    const Rung *rungs = h->fused_depth == 2 ? pairs : ladder;
+    const int nrungs = h->fused_depth == 2 ? 5 : 3;
     for (int k = 0; k < nrungs; ++k) {
       const Rung &r = rungs[k];
+      if (r.most > 0 && na / (r.w * r.h) > r.most) continue;
       h->tile_cache = evp1d::tile_ids(h->coords, r.w, r.h, h->tile_order);
       h->tile_w = r.w;
       h->tile_h = r.h;
       h->tile_block = r.block;
-      if (h->tile_cache.ntiles >= r.min_tiles) break;
+      const int n = h->tile_cache.ntiles;
+      if (r.most > 0 ? n <= r.most : n >= r.least) break;
     }
     h->tile_cache_ok = true;
+    h->crowded_checked = h->fused_depth != 2 || h->tile_w != 31 || h->tile_h != 19 || h->tile_cache.ntiles <= kCus;
+  }
+  // 31x19 where its busiest tile has more than 512 level-2 stress points
+  // (contiguous ice: 32x20) takes workgroups of 1024 threads, one per CU,
+  // which nothing overlaps: 31x15 then (at most 512, two per CU).  1280x1520
+  // in contiguous ice 75.4 / 61.2 us per subcycle, 733x517 17.9 / 15.4.  Once
+  // chosen it stays for these lists, so that changing flags do not alternate.
+  if (h->tiling_auto && !h->crowded_checked && all && h->tile_cache.ntiles > 0 &&
+      evp1d::max_level2(na, idx, h->skip_host.data(), h->tile_cache) > 512) {
+    h->tile_h = 15;
+    h->tile_cache = evp1d::tile_ids(h->coords, h->tile_w, h->tile_h, h->tile_order);
+    h->crowded_checked = true;
   }
   if (!h->tile_cache_ok || h->tile_cache.tile_w != h->tile_w || h->tile_cache.tile_h != h->tile_h ||
       h->tile_cache.order != h->tile_order) {

@@ -323,6 +323,29 @@ struct TileWork {
 
 }  // namespace
 
+// T point q is read by the stepu points ee(q), ne(q) and se(q) (as their nw,
+// sw and sse neighbour): it is a halo entry of the other tiles among theirs.
+int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids) {
+  std::vector<int32_t> n((size_t)std::max(ids.ntiles, 1), 0);
+  par_chunks(na, 1 << 15, [&](int64_t lo, int64_t hi, int) {
+    for (int64_t q = lo; q < hi; ++q) {
+      if (point_class(skip[q]) > 1) continue;
+      int32_t seen[4] = {ids.tid[(size_t)q], -1, -1, -1};
+      int m = 1;
+      for (int k : {0, 1, 2}) {
+        const int32_t r = idx[k][q];
+        if (r < 0 || r >= na) continue;
+        const int c = point_class(skip[r]);
+        if (c != 1 && c != 2) continue;
+        const int32_t t = ids.tid[(size_t)r];
+        if (std::find(seen, seen + m, t) == seen + m) seen[m++] = t;
+      }
+      for (int i = 0; i < m; ++i) __atomic_fetch_add(&n[(size_t)seen[i]], 1, __ATOMIC_RELAXED);
+    }
+  });
+  return *std::max_element(n.begin(), n.end());
+}
+
 // The plan is a pure function of the lists, the flags and the tile ids; the
 // work is split over host threads, and every part is computed in an order
 // that does not depend on the number of threads, so the plan does not either.

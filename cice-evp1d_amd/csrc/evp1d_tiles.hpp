@@ -132,6 +132,10 @@ struct TileIds {
 TileIds tile_ids(const GridCoords &c, int tile_w, int tile_h, int order = 0);
 TileIds tile_ids(int na, int navel, const int32_t *const idx[6], int tile_w, int tile_h);
 
+// The largest number of stress points that a tile owns or evaluates as halo
+// (its level-2 entries in the pair form, one thread each) for these flags.
+int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids);
+
 // idx: ee, ne, se, nw, sw, sse as 0-based caller positions (values in
 // [0, navel); positions >= na are ghost slots).  skip: bit0 skipT, bit1 skipU.
 // idx may be null (no tiling, class order only).

@@ -1,0 +1,33 @@
+"""The tile that the library chooses for the pair form, at the edges of its
+ladder (at most one tile per CU of 15x11, 22x16, 31x19; two of 31x15; 31x19;
+31x15 again where contiguous ice crowds the 31x19 tiles): the choice, and the
+state after a run bit for bit against the oracle."""
+import pytest
+
+from gpu_common import assert_state_bitexact, fetch_state, make_engine, oracle_params, synthetic_state
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nx,ny,ice,tile,threads", [
+    (1, 1, 1.0, (15, 11), 256),
+    (240, 176, 1.0, (15, 11), 256),     # 16 x 16 tiles: 256
+    (241, 176, 1.0, (22, 16), 512),
+    (352, 256, 0.7, (22, 16), 512),     # 16 x 16 tiles of 22x16
+    (352, 257, 1.0, (31, 19), 1024),
+    (497, 304, 0.7, (31, 15), 512),     # 17 x 16 tiles of 31x19
+    (620, 480, 0.7, (31, 19), 512),     # 20 x 32 tiles of 31x15
+    (620, 480, 1.0, (31, 15), 512),     # 640 level-2 points in a 31x19 tile
+])
+def test_chosen_tile(gpu, nx, ny, ice, tile, threads):
+    st = synthetic_state(nx, ny, seed=5, land_frac=0.0, ice_prob=ice)
+    nsub = 4
+    with make_engine(st, nsub) as eng:
+        t, d = eng.get_tiling(), eng.get_fused_depth()
+        assert (t["tile_w"], t["tile_h"]) == tile and d["active"] and d["block"] == threads
+        eng.run(nsub)
+        got = fetch_state(eng, st)
+    lib, p = oracle_params(st, nsub)
+    want = st.copy()
+    lib.run(p, want, nsub)
+    assert_state_bitexact(got, want)
