@@ -44,6 +44,7 @@
 #include "evp1d_tiles.hpp"
 #include "evp1d_point.hpp"
 #include "evp1d_cache.hpp"
+#include "evp1d_pair.hpp"
 #include "evp1d_xcd.hpp"
 
 #ifndef EVP1D_FMA
@@ -351,50 +352,6 @@ __global__ __launch_bounds__(B) void k_fused(DevView d, FusedView f, int last) {
   }
 }
 
-// ---------------------------------------------------------------------------
-// two subcycles per workgroup ("pair" form)
-// ---------------------------------------------------------------------------
-// Level 1 runs stress on the tile's T1 entries (owned, halo, T1-only) from the
-// input state d.vel / d.sig, then stepu on its U1 entries into an LDS
-// velocity table; level 2 runs stress on the owned and halo entries from
-// those velocities and the level-1 stresses, then stepu on the owned U
-// points, and writes the state two subcycles on to vel_out / sig_out (two
-// buffers each).  Every point computes exactly what the one-subcycle kernels
-// compute, so results are bit-identical; neighbour tiles evaluate the border
-// rings again instead of exchanging them, which halves the loads and stores
-// of the state and the constant fields per subcycle.  Level-2 stress entry k
-// is thread k (the plan guarantees at most B of them), so its level-1
-// stresses stay in that thread's registers.  The 20 constant fields come
-// from a copy packed in pairs at the start of the run (k_pack_const), the
-// stresses live during the run in pairs too (k_pack_sig / k_unpack_sig): one
-// 16-byte load per pair, since the kernel's time follows its load
-// instructions.  Each level-1 stress entry's slot and ee, ne, se neighbour
-// slots come from one per-tile int4 (PairPlan::tnbr), so a halo or T1-only
-// entry reaches its velocities after two dependent loads, not three.
-struct PairView {
-  const evp1d::PairTile *tiles;
-  const int32_t *hlist, *xlist, *elist;
-  const uint2 *uloc;        // per U1 entry: own | nw << 16, sse | sw << 16 (str table entries)
-  const uint2 *vloc;        // per T2 entry: cc | ee << 16, ne | se << 16 (velocity table entries)
-  const double2 *cstr;      // [4][nk]: s15, s27, s36, s48 of the constant entries
-  const int *cnz;
-  long nk;
-  double2 *vel_out;
-  int cap;                  // entries of the str table (the velocity table follows it)
-  const double2 *pc;        // [kPairConst][lp]: the constant fields in pairs (k_pack_const)
-  long lp;
-  const double2 *sg_in;     // [6][ls]: stresses in pairs (p1 p2, p3 p4, m1 m2, m3 m4, 12_1 12_2, 12_3 12_4)
-  double2 *sg_out;
-  long ls;
-  const int4 *tnbr;         // per level-1 stress entry (PairTile::n0 + k): slot, ee, ne, se
-  const int32_t *fix;       // fixed copy-list sources of level-2 ghost reads (PairPlan::fix)
-  // gradient trajectory (k_pair<.., TRAJ>): the velocities of the stepu
-  // slots after the launch's first subcycle (tr_mid) and after its second
-  // (tr_end, null when the handle's own buffer is the only copy wanted),
-  // indexed by slot - u_begin
-  double2 *tr_mid, *tr_end;
-};
-
 // the stresses of the stress slots [0, n) into pairs, and back
 __global__ void k_pack_sig(double2 *p, long ls, const double *sig, long ldsig, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -421,7 +378,7 @@ __global__ void k_pack_nbr(DevView d, int4 *nbr, long n) {
 // The constant fields in pairs, one double2 array each: (dxT, dyT), (hte,
 // htn), (htem1, htnm1), (cw, aiu), (uocn, vocn), (waterx, watery), (forcex,
 // forcey), (umassdti, fm), (uarear, tbu), (uvel_init, vvel_init).
-constexpr int kPairConst = 10;
+constexpr int kPairConst = kPairT<false> + kPairU;
 __global__ void k_pack_const(DevView d, double2 *pc, long lp) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= d.na) return;
@@ -435,253 +392,6 @@ __global__ void k_pack_const(DevView d, double2 *pc, long lp) {
   pc[7 * lp + i] = make_double2(d.umassdti[i], d.fm[i]);
   pc[8 * lp + i] = make_double2(d.uarear[i], d.tbu[i]);
   pc[9 * lp + i] = make_double2(d.uvel_init[i], d.vvel_init[i]);
-}
-
-// the buffers that alternate between launches: input velocities and
-// stresses, output velocities and stresses
-struct PairBufs {
-  const double2 *vel;
-  double2 *vel_out;
-  const double2 *sg_in;
-  double2 *sg_out;
-};
-
-// At most 128 VGPRs (4 waves per SIMD): workgroups of 256, 512 or 1024
-// threads then fill 16 waves per CU.  TRAJ: the gradient's forward sweep,
-// which also stores both subcycles' stepu-slot velocities (f.tr_mid,
-// f.tr_end); the values computed are the same.
-//
-// Each barrier waits for LDS only, so global loads issued before it stay in
-// flight across it: every thread loads the memory inputs of its first entry
-// of the next phase (level-1 stepu, level-2 stress, level-2 stepu) before
-// the barrier that ends the current phase, and that phase starts on values
-// already in registers instead of one memory round trip after the barrier.
-//
-// NT: the cache hints (evp1d_cache.hpp).  The streams a launch reads or
-// writes once (stresses in and out, the T points' constant fields,
-// velocities and trajectory written) become non-temporal loads and stores,
-// so that the cache can keep what every launch reads again (the U points'
-// constant fields, velocities, tables).
-template <int B, bool TRAJ, bool FIX, bool NT>
-__device__ __forceinline__ void pair_tile(const DevView &d, const PairView &f, PairBufs bf, int last, int tix) {
-  extern __shared__ double2 lds[];
-  const int cap = f.cap;
-  double2 *vt = lds + 4 * cap;
-  const evp1d::PairTile pt = f.tiles[tix];
-  const evp1d::TileDesc &t = pt.t;
-  const int nA = t.a1 - t.a0, nB = t.b1 - t.b0, nO = nA + nB, nS = nO + t.nh, nT = nS + pt.nx, nE = nT + pt.nq;
-  const int nUo = nB + (t.c1 - t.c0), nU = nUo + pt.ne;
-  const bool cz = *f.cnz == 0;
-  auto tslot = [&](int k) {
-    return k < nA ? t.a0 + k : k < nO ? t.b0 + (k - nA) : k < nS ? f.hlist[t.h0 + (k - nO)] : f.xlist[pt.x0 + (k - nS)];
-  };
-  auto uslot = [&](int k) { return k < nB ? t.b0 + k : k < nUo ? t.c0 + (k - nB) : f.elist[pt.e0 + (k - nUo)]; };
-  auto put = [&](int k, const evp1d::StressOut &o) {
-    lds[k] = make_double2(o.str[0], o.str[4]);
-    lds[cap + k] = make_double2(o.str[1], o.str[6]);
-    lds[2 * cap + k] = make_double2(o.str[2], o.str[5]);
-    lds[3 * cap + k] = make_double2(o.str[3], o.str[7]);
-  };
-  const double2 *pc = f.pc;
-  const long lp = f.lp;
-  // memory inputs of one stepu evaluation: its str table entries and the
-  // seven packed constant pairs of slot q
-  struct UIn {
-    uint2 w;
-    double2 c[7];
-  };
-  auto uload = [&](int k, int q) {
-    UIn u;
-    u.w = f.uloc[pt.u0 + k];
-#pragma unroll
-    for (int c = 0; c < 7; ++c) u.c[c] = pc[(3 + c) * lp + q];
-    return u;
-  };
-  auto stepu = [&](const UIn &u, double2 v, evp1d::StepuOut &o) {
-    const double2 a = lds[u.w.x & 0xffffu];
-    const double2 b = lds[cap + (u.w.x >> 16)];
-    const double2 c = lds[2 * cap + (u.w.y & 0xffffu)];
-    const double2 e = lds[3 * cap + (u.w.y >> 16)];
-    const double2 *k = u.c;
-    evp1d::stepu_point(d.s, v.x, v.y, k[0].x, k[0].y, k[1].x, k[1].y, k[2].x, k[2].y, k[3].x, k[3].y, k[4].x,
-                       k[4].y, k[5].x, k[6].x, k[6].y, k[5].y, a.x, b.x, c.x, e.x, a.y, c.y, b.y, e.y, o);
-  };
-  const int me = threadIdx.x;
-  double sg[12];   // level-1 stresses of entry `me` when me < nS
-  // entry `me`'s metric pairs and strength, loaded at level 1 and used again
-  // at level 2 (the same slot)
-  double2 m2[3];
-  double st2 = 0.0;
-  // level 1, stress (or constants) of entry k
-  auto level1 = [&](int k) {
-    if (k < nT) {
-      const int4 n = f.tnbr[pt.n0 + k];   // slot and ee, ne, se of the entry
-      const int g = k < nO ? tslot(k) : n.x;
-      double sig[12];
-#pragma unroll
-      for (int c = 0; c < 6; ++c) {
-        const double2 v = in2<NT>(bf.sg_in + (c * f.ls + g));
-        sig[2 * c] = v.x;
-        sig[2 * c + 1] = v.y;
-      }
-      const double2 a0 = in2<NT>(pc + g), a1 = in2<NT>(pc + (lp + g)), a2 = in2<NT>(pc + (2 * lp + g));
-      const double st = in1<NT>(d.strength + g);
-      evp1d::StressOut o;
-      const double2 cc = bf.vel[g], ve = bf.vel[n.y], vn = bf.vel[n.z], vs = bf.vel[n.w];
-      evp1d::stress_point(d.s, cc.x, cc.y, ve.x, ve.y, vs.x, vs.y, vn.x, vn.y, a0.x, a0.y, st, a1.x, a1.y, a2.x,
-                          a2.y, sig, o);
-      if (k == me) {
-        m2[0] = a0;
-        m2[1] = a1;
-        m2[2] = a2;
-        st2 = st;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          sg[c] = o.sp[c];
-          sg[4 + c] = o.sm[c];
-          sg[8 + c] = o.s12[c];
-        }
-      }
-      put(k, o);
-    } else {
-      double2 p15, p27, p36, p48;
-      if (cz) {
-        p15 = p27 = p36 = p48 = make_double2(0.0, 0.0);
-      } else {
-        const long j = pt.q0 + (k - nT);
-        p15 = f.cstr[j];
-        p27 = f.cstr[f.nk + j];
-        p36 = f.cstr[2 * f.nk + j];
-        p48 = f.cstr[3 * f.nk + j];
-      }
-      lds[k] = p15;
-      lds[cap + k] = p27;
-      lds[2 * cap + k] = p36;
-      lds[3 * cap + k] = p48;
-    }
-  };
-  // entries me + B, me + 2B, ... first and entry me (kept for level 2) last,
-  // so no other evaluation overlaps the lifetime of its stresses
-  for (int k = me + B; k < nE; k += B) level1(k);
-  if (me < nE) level1(me);
-  // level 1, stepu, entry me: inputs loaded before the barrier
-  int q1 = 0;
-  UIn u1;
-  double2 v1;
-  if (me < nU) {
-    q1 = uslot(me);
-    u1 = uload(me, q1);
-    v1 = bf.vel[q1];
-  }
-  __syncthreads();
-  // level 1, stepu: every U1 entry into the velocity table
-  if (me < nU) {
-    evp1d::StepuOut o;
-    stepu(u1, v1, o);
-    vt[me] = make_double2(o.uvel, o.vvel);
-    if (TRAJ && me < nUo) out2<NT>(f.tr_mid + (q1 - d.u_begin), vt[me]);
-  }
-  for (int k = me + B; k < nU; k += B) {
-    const int q = uslot(k);
-    const UIn u = uload(k, q);
-    evp1d::StepuOut o;
-    stepu(u, bf.vel[q], o);
-    vt[k] = make_double2(o.uvel, o.vvel);
-    if (TRAJ && k < nUo) out2<NT>(f.tr_mid + (q - d.u_begin), vt[k]);
-  }
-  // level 2, stress of entry me: memory inputs loaded before the barrier
-  // (velocities that are no U1 entry never change, kNoEntry: from memory)
-  // (velocities that are no U1 entry never change, kNoEntry: from memory;
-  // a ghost on the copy list whose source is no U1 entry: kFixBase + j, the
-  // source's unchanging velocity or zero)
-  constexpr unsigned kNo = evp1d::PairPlan::kNoEntry, kFix = evp1d::PairPlan::kFixBase;
-  int g2 = 0;
-  uint2 w2 = make_uint2(0u, 0u);
-  double2 c2[4];
-  if (me < nS) {
-    const int4 n = f.tnbr[pt.n0 + me];
-    g2 = me < nO ? tslot(me) : n.x;
-    w2 = f.vloc[pt.v0 + me];
-    c2[0] = bf.vel[g2];
-    if (!FIX) {   // no copy list: every entry is a table entry or kNoEntry
-      if ((w2.x >> 16) == kNo || (w2.y & 0xffffu) == kNo || (w2.y >> 16) == kNo) {
-        c2[1] = bf.vel[n.y];
-        c2[2] = bf.vel[n.z];
-        c2[3] = bf.vel[n.w];
-      }
-    } else {
-      const unsigned e[3] = {w2.x >> 16, w2.y & 0xffffu, w2.y >> 16};
-      const int ns[3] = {n.y, n.z, n.w};
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        if (e[c] == kNo) {
-          c2[1 + c] = bf.vel[ns[c]];
-        } else if (e[c] >= kFix) {
-          const int s = f.fix[pt.f0 + (int)(e[c] - kFix)];
-          c2[1 + c] = s < 0 ? make_double2(0.0, 0.0) : bf.vel[s];
-        }
-      }
-    }
-  }
-  __syncthreads();
-  // level 2, stress: owned and halo entries, one per thread
-  if (me < nS) {
-    const unsigned e0 = w2.x & 0xffffu, e1 = w2.x >> 16, e2 = w2.y & 0xffffu, e3 = w2.y >> 16;
-    const double2 cc = e0 >= kFix ? c2[0] : vt[e0];
-    const double2 ve = e1 >= kFix ? c2[1] : vt[e1];
-    const double2 vn = e2 >= kFix ? c2[2] : vt[e2];
-    const double2 vs = e3 >= kFix ? c2[3] : vt[e3];
-    evp1d::StressOut o;
-    evp1d::stress_point(d.s, cc.x, cc.y, ve.x, ve.y, vs.x, vs.y, vn.x, vn.y, m2[0].x, m2[0].y, st2, m2[1].x,
-                        m2[1].y, m2[2].x, m2[2].y, sg, o);
-    const int g = g2;
-    if (me < nO) {
-      out2<NT>(bf.sg_out + g, make_double2(o.sp[0], o.sp[1]));
-      out2<NT>(bf.sg_out + (f.ls + g), make_double2(o.sp[2], o.sp[3]));
-      out2<NT>(bf.sg_out + (2 * f.ls + g), make_double2(o.sm[0], o.sm[1]));
-      out2<NT>(bf.sg_out + (3 * f.ls + g), make_double2(o.sm[2], o.sm[3]));
-      out2<NT>(bf.sg_out + (4 * f.ls + g), make_double2(o.s12[0], o.s12[1]));
-      out2<NT>(bf.sg_out + (5 * f.ls + g), make_double2(o.s12[2], o.s12[3]));
-      if (last) {
-        out2<NT>(d.s15 + g, make_double2(o.str[0], o.str[4]));
-        out2<NT>(d.s27 + g, make_double2(o.str[1], o.str[6]));
-        out2<NT>(d.s36 + g, make_double2(o.str[2], o.str[5]));
-        out2<NT>(d.s48 + g, make_double2(o.str[3], o.str[7]));
-      }
-    }
-    put(me, o);
-  }
-  // level 2, stepu of entry me: inputs loaded before the barrier
-  int q2 = 0;
-  UIn u2;
-  if (me < nUo) {
-    q2 = uslot(me);
-    u2 = uload(me, q2);
-  }
-  __syncthreads();
-  // level 2, stepu: the owned U points
-  auto level2u = [&](int k, int q, const UIn &u) {
-    evp1d::StepuOut o;
-    stepu(u, vt[k], o);
-    out2<NT>(bf.vel_out + q, make_double2(o.uvel, o.vvel));
-    if (TRAJ && f.tr_end) out2<NT>(f.tr_end + (q - d.u_begin), make_double2(o.uvel, o.vvel));
-    if (last) {
-      out1<NT>(d.strintx + q, o.strintx);
-      out1<NT>(d.strinty + q, o.strinty);
-      out1<NT>(d.cb + q, o.Cb);
-    }
-  };
-  if (me < nUo) level2u(me, q2, u2);
-  for (int k = me + B; k < nUo; k += B) {
-    const int q = uslot(k);
-    level2u(k, q, uload(k, q));
-  }
-}
-
-template <int B, bool X, bool TRAJ = false, bool FIX = false, bool NT = false>
-__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4))) void k_pair(DevView d, PairView f, int last) {
-  pair_tile<B, TRAJ, FIX, NT>(d, f, PairBufs{d.vel, f.vel_out, f.sg_in, f.sg_out}, last,
-                              tile_of(blockIdx.x, gridDim.x, X));
 }
 
 // The pair launches j0..L of a run (numbered as issue_fused numbers them) in
@@ -699,29 +409,28 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4))) void k_p
 // launch j uses row j mod 2 and clears the other row for launch j + 1.
 constexpr int kCntPad = 64;   // ints from one tile counter to the next
 struct PersistArgs {
-  double2 *vy, *sg0, *sg1;
+  double2 *vx, *vy, *sg0, *sg1;
   int *cnt;
-  int j0, L, ntiles;
+  int j0, L, ntiles, nhalo;
+  const int32_t *halo_dst, *halo_src;
 };
 
-template <int B, bool X, bool FIX>
-__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4))) void k_pair_persistent(DevView d, PairView f,
+template <int B, bool FIX>
+__global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4))) void k_pair_persistent(PairView f,
                                                                                              PersistArgs a) {
   cg::grid_group grid = cg::this_grid();
-  // The arguments are read in place in the kernel-argument segment (d at
-  // offset 0, f and a after it, each at its alignment), through a pointer
+  // The arguments are read in place in the kernel-argument segment (f at
+  // offset 0, a after it at its alignment), through a pointer
   // that an empty asm statement makes opaque once per tile: their fields are
   // then loaded where the tile body uses them, as in k_pair, instead of
   // being hoisted out of the loops and held in registers for the whole
   // launch (which spilled).
   typedef const __attribute__((address_space(4))) char *ArgP;
-  constexpr size_t kOffF = (sizeof(DevView) + alignof(PairView) - 1) / alignof(PairView) * alignof(PairView);
-  constexpr size_t kOffA =
-      (kOffF + sizeof(PairView) + alignof(PersistArgs) - 1) / alignof(PersistArgs) * alignof(PersistArgs);
+  constexpr size_t kOffA = (sizeof(PairView) + alignof(PersistArgs) - 1) / alignof(PersistArgs) * alignof(PersistArgs);
   ArgP ka = (ArgP)__builtin_amdgcn_kernarg_segment_ptr();
   const int j0 = a.j0, L = a.L, ntiles = a.ntiles;
   // this workgroup's group x and the group's tiles [t0, t0 + nt)
-  const int P = (X && gridDim.x >= kXcds && gridDim.x % kXcds == 0) ? kXcds : 1;
+  const int P = (f.xcd != 0 && gridDim.x >= kXcds && gridDim.x % kXcds == 0) ? kXcds : 1;
   const int x = blockIdx.x % P;
   const int q = ntiles / P, r = ntiles % P;
   const int t0 = x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q, nt = q + (x < r ? 1 : 0);
@@ -739,19 +448,18 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(4))) void k_p
       const int k = grab;   // read by every thread before the tile's first barrier
       if (k >= nt) break;
       asm volatile("" : "+s"(ka));
-      const DevView &dv = *(const DevView *)(const __attribute__((address_space(4))) DevView *)ka;
-      const PairView &fv = *(const PairView *)(const __attribute__((address_space(4))) PairView *)(ka + kOffF);
+      const PairView &fv = *(const PairView *)(const __attribute__((address_space(4))) PairView *)ka;
       const PersistArgs &av =
           *(const PersistArgs *)(const __attribute__((address_space(4))) PersistArgs *)(ka + kOffA);
-      const PairBufs bf{to_x ? av.vy : dv.vel, to_x ? dv.vel : av.vy, odd ? av.sg1 : av.sg0, odd ? av.sg0 : av.sg1};
-      pair_tile<B, false, FIX, false>(dv, fv, bf, j == L ? 1 : 0, t0 + k);
+      const PairBufs bf{to_x ? av.vy : av.vx, to_x ? av.vx : av.vy, odd ? av.sg1 : av.sg0, odd ? av.sg0 : av.sg1};
+      pair_tile<B, false, false, FIX, false>(fv, bf, j == L ? 1 : 0, t0 + k);
       __syncthreads();   // the next tile rewrites the LDS tables and grab
     }
     grid.sync();
-    if (d.nhalo > 0) {   // the copy after the launch's second subcycle
-      double2 *out = to_x ? d.vel : a.vy;
-      for (int k = blockIdx.x * B + threadIdx.x; k < d.nhalo; k += gridDim.x * B) {
-        const int dst = d.halo_dst[k], src = d.halo_src[k];
+    if (a.nhalo > 0) {   // the copy after the launch's second subcycle
+      double2 *out = to_x ? a.vx : a.vy;
+      for (int k = blockIdx.x * B + threadIdx.x; k < a.nhalo; k += gridDim.x * B) {
+        const int dst = a.halo_dst[k], src = a.halo_src[k];
         out[dst] = src >= 0 ? out[src] : make_double2(0.0, 0.0);
       }
       grid.sync();
@@ -793,13 +501,6 @@ __global__ void k_fill_const(DevView d, const int32_t *klist, double2 *cstr, lon
 
 constexpr int kFusedMaxEntries = 2560;   // 160 KiB of LDS per workgroup (gfx950)
 constexpr int kFusedMinSub = 4;          // evp1d_run in AUTO mode: fused from this many subcycles
-// pair form: block sizes (one level-2 stress per thread) and LDS limit
-constexpr int kNumPairBlocks = 3;
-constexpr int kPairBlocks[kNumPairBlocks] = {256, 512, 1024};
-constexpr int kPairMaxLds = 160 * 1024;
-// LDS of a pair launch: str table and velocity table
-static size_t pair_lds(int cap, int capv) { return (size_t)(4 * cap + capv) * sizeof(double2); }
-
 // launch configurations the autotuner chooses from
 constexpr int kNumBlocks = 5;
 constexpr int kBlocks[kNumBlocks] = {64, 128, 256, 512, 1024};
@@ -1194,7 +895,6 @@ struct evp1d_handle {
   // fused form: tiling and its device tables (owned here, replaced on relayout)
   int tile_w = 64, tile_h = 16, tile_block = 512, tile_xcd = 1;
   bool tiling_auto = true;         // choose the tile from the domain size (until evp1d_set_tiling)
-  bool crowded_checked = false;    // the chosen tile needs no look at its busiest tile's level-2 points
   evp1d::GridCoords coords;        // grid coordinates of the current lists
   bool coords_ok = false;
   evp1d::TileIds tile_cache;       // tile of every point for the current lists and tile size
@@ -1542,47 +1242,27 @@ static int relayout_impl(evp1d_handle *h) {
     h->tile_cache_ok = false;
   }
   if (h->tiling_auto && !h->tile_cache_ok) {
-    // The first rung of a ladder that gives at most `most` tiles, or at least
-    // `least`.
-    // Pair form: a tile's time is its chain of four phases, whatever runs
-    // beside it, until the 256 CUs are full.  So with at most one tile per CU
-    // the smallest tile is the fastest: in 15x11 every phase is one pass of
-    // 256 threads (18x14 cells at level 1), in 22x16 one of 512.  Measured,
-    // 31x19 / chosen, us per subcycle: 64x48 5.3 / 4.0, 200x150 6.2 / 4.1,
-    // 300x220 6.9 / 5.9, 520x400 11.1 / 10.3 (31x15).  Beyond two tiles per
-    // CU the border's extra work counts: 31x19.
-    // One subcycle per launch: the largest tile that still fills the GPU.
-    struct Rung { int w, h, block, most, least; };
-    constexpr int kCus = 256;
-    static const Rung ladder[3] = {{64, 16, 512, 0, 1024}, {32, 8, 256, 0, 512}, {16, 8, 128, 0, 0}};
-    static const Rung pairs[5] = {{15, 11, 256, kCus, 0}, {22, 16, 512, kCus, 0}, {31, 19, 512, kCus, 0},
-                                  {31, 15, 512, 2 * kCus, 0}, {31, 19, 512, 0, 0}};
-    const Rung *rungs = h->fused_depth == 2 ? pairs : ladder;
-    const int nrungs = h->fused_depth == 2 ? 5 : 3;
-    for (int k = 0; k < nrungs; ++k) {
-      const Rung &r = rungs[k];
-      if (r.most > 0 && na / (r.w * r.h) > r.most) continue;
-      h->tile_cache = evp1d::tile_ids(h->coords, r.w, r.h, h->tile_order);
-      h->tile_w = r.w;
-      h->tile_h = r.h;
-      h->tile_block = r.block;
-      const int n = h->tile_cache.ntiles;
-      if (r.most > 0 ? n <= r.most : n >= r.least) break;
+    if (h->fused_depth == 2) {
+      h->tile_cache = evp1d::pair_tiles(h->coords, h->tile_order, &h->tile_block);
+    } else {
+      // one subcycle per launch: the largest tile that still fills the GPU
+      struct Rung { int w, h, block, least; };
+      static const Rung ladder[3] = {{64, 16, 512, 1024}, {32, 8, 256, 512}, {16, 8, 128, 0}};
+      for (const Rung &r : ladder) {
+        h->tile_cache = evp1d::tile_ids(h->coords, r.w, r.h, h->tile_order);
+        h->tile_block = r.block;
+        if (h->tile_cache.ntiles >= r.least) break;
+      }
     }
+    h->tile_w = h->tile_cache.tile_w;
+    h->tile_h = h->tile_cache.tile_h;
     h->tile_cache_ok = true;
-    h->crowded_checked = h->fused_depth != 2 || h->tile_w != 31 || h->tile_h != 19 || h->tile_cache.ntiles <= kCus;
   }
-  // 31x19 where its busiest tile has more than 512 level-2 stress points
-  // (contiguous ice: 32x20) takes workgroups of 1024 threads, one per CU,
-  // which nothing overlaps: 31x15 then (at most 512, two per CU).  1280x1520
-  // in contiguous ice 75.4 / 61.2 us per subcycle, 733x517 17.9 / 15.4.  Once
-  // chosen it stays for these lists, so that changing flags do not alternate.
-  if (h->tiling_auto && !h->crowded_checked && all && h->tile_cache.ntiles > 0 &&
-      evp1d::max_level2(na, idx, h->skip_host.data(), h->tile_cache) > 512) {
-    h->tile_h = 15;
-    h->tile_cache = evp1d::tile_ids(h->coords, h->tile_w, h->tile_h, h->tile_order);
-    h->crowded_checked = true;
-  }
+  // Once uncrowded the tile stays for these lists, so that changing flags do
+  // not make it alternate.
+  if (h->tiling_auto && h->fused_depth == 2 && all &&
+      evp1d::pair_uncrowd(h->coords, na, idx, h->skip_host.data(), h->tile_cache))
+    h->tile_h = h->tile_cache.tile_h;
   if (!h->tile_cache_ok || h->tile_cache.tile_w != h->tile_w || h->tile_cache.tile_h != h->tile_h ||
       h->tile_cache.order != h->tile_order) {
     h->tile_cache = evp1d::tile_ids(h->coords, h->tile_w, h->tile_h, h->tile_order);
@@ -1719,38 +1399,24 @@ static const FusedFn kFusedFns[4][2] = {{k_fused<64, false>, k_fused<64, true>},
                                         {k_fused<512, false>, k_fused<512, true>}};
 static const FusedFn kFusedSplitFns[4] = {k_fused<64, true, true>, k_fused<128, true, true>,
                                          k_fused<256, true, true>, k_fused<512, true, true>};
-typedef void (*PairFn)(DevView, PairView, int);
-// [workgroup size][XCD-aware order][cache hints]
-#define PAIR_ROW(B, FIX)                                                                      \
-  {{k_pair<B, false, false, FIX, false>, k_pair<B, false, false, FIX, true>},                 \
-   {k_pair<B, true, false, FIX, false>, k_pair<B, true, false, FIX, true>}}
-static const PairFn kPairFns[kNumPairBlocks][2][2] = {PAIR_ROW(256, false), PAIR_ROW(512, false),
-                                                      PAIR_ROW(1024, false)};
-// with a ghost copy list (level-2 reads of listed ghosts through PairPlan::fix)
-static const PairFn kPairFixFns[kNumPairBlocks][2][2] = {PAIR_ROW(256, true), PAIR_ROW(512, true),
-                                                         PAIR_ROW(1024, true)};
+typedef void (*PairFn)(PairView, PairBufs, int);
+enum PairKind { kPairPlain, kPairFix, kPairTraj };
+// [workgroup size][plain, with a ghost copy list (level-2 reads of listed
+// ghosts through PairPlan::fix), the gradient sweep's trajectory-storing
+// form][cache hints]
+#define PAIR_ROW(B)                                                                \
+  {{k_pair<B, false>, k_pair<B, false, false, false, true>},                       \
+   {k_pair<B, false, false, true>, k_pair<B, false, false, true, true>},           \
+   {k_pair<B, false, true>, k_pair<B, false, true, false, true>}}
+static const PairFn kPairFns[kNumPairBlocks][3][2] = {PAIR_ROW(256), PAIR_ROW(512), PAIR_ROW(1024)};
 #undef PAIR_ROW
-// the gradient sweep's trajectory-storing form (XCD-aware tile order only),
-// [workgroup size][cache hints]
-static const PairFn kPairTrajFns[kNumPairBlocks][2] = {
-    {k_pair<256, true, true, false, false>, k_pair<256, true, true, false, true>},
-    {k_pair<512, true, true, false, false>, k_pair<512, true, true, false, true>},
-    {k_pair<1024, true, true, false, false>, k_pair<1024, true, true, false, true>}};
 // one cooperative launch for the pair launches of a run (evp1d_run in
 // EVP1D_MODE_PERSISTENT with the pair form selected)
-typedef void (*PairPersistFn)(DevView, PairView, PersistArgs);
-static const PairPersistFn kPairPersistFns[kNumPairBlocks][2][2] = {
-    {{k_pair_persistent<256, false, false>, k_pair_persistent<256, false, true>},
-     {k_pair_persistent<256, true, false>, k_pair_persistent<256, true, true>}},
-    {{k_pair_persistent<512, false, false>, k_pair_persistent<512, false, true>},
-     {k_pair_persistent<512, true, false>, k_pair_persistent<512, true, true>}},
-    {{k_pair_persistent<1024, false, false>, k_pair_persistent<1024, false, true>},
-     {k_pair_persistent<1024, true, false>, k_pair_persistent<1024, true, true>}}};
-static int pair_block_index(int b) {
-  for (int i = 0; i < kNumPairBlocks; ++i)
-    if (kPairBlocks[i] == b) return i;
-  return -1;
-}
+typedef void (*PairPersistFn)(PairView, PersistArgs);
+static const PairPersistFn kPairPersistFns[kNumPairBlocks][2] = {
+    {k_pair_persistent<256, false>, k_pair_persistent<256, true>},
+    {k_pair_persistent<512, false>, k_pair_persistent<512, true>},
+    {k_pair_persistent<1024, false>, k_pair_persistent<1024, true>}};
 // the pair form runs when selected and planned
 static bool pair_form(const evp1d_handle *h) { return h->fused_depth == 2 && h->pair_ok; }
 
@@ -1786,14 +1452,10 @@ static int ensure_fused_buffers(evp1d_handle *h) {
     for (FusedFn fn : kFusedSplitFns)
       HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   kFusedMaxEntries * 4 * (int)sizeof(double2)));
-    for (const auto *tab : {&kPairFns, &kPairFixFns})
-      for (const auto &row : *tab)
-        for (const auto &pair : row)
-          for (PairFn fn : pair)
-            HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
-    for (const auto &row : kPairTrajFns)
-      for (PairFn fn : row)
-        HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
+    for (const auto &size : kPairFns)
+      for (const auto &kind : size)
+        for (PairFn fn : kind)
+          HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
   }
   if (!h->vel_alt) HIP_TRY(hipMalloc((void **)&h->vel_alt, (size_t)h->navel * sizeof(double2)));
   if ((!h->fused_inplace || pair_form(h)) && !h->sig_alt)
@@ -1865,7 +1527,7 @@ static void fused_step(evp1d_handle *h, FusedView &f, int k) {
 static int launch_pair_persistent(evp1d_handle *h, const DevView &x, PairView pv, double2 *sg0, double2 *sg1,
                                   int j0, int L, size_t lds) {
   const int b = pair_block_index(h->pair_block);
-  const PairPersistFn fn = kPairPersistFns[b][h->tile_xcd ? 1 : 0][h->v.nhalo > 0 ? 1 : 0];
+  const PairPersistFn fn = kPairPersistFns[b][h->v.nhalo > 0 ? 1 : 0];
   int per_cu = 0, cus = 0;
   HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, h->pair_block, lds));
   HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device));
@@ -1875,9 +1537,8 @@ static int launch_pair_persistent(evp1d_handle *h, const DevView &x, PairView pv
   const size_t cnt_bytes = (size_t)2 * kXcds * kCntPad * sizeof(int);
   if (!h->pcnt_dev) HIP_TRY(hipMalloc((void **)&h->pcnt_dev, cnt_bytes));
   HIP_TRY(hipMemsetAsync(h->pcnt_dev, 0, cnt_bytes, h->stream));
-  DevView d = x;
-  PersistArgs a{h->vel_alt, sg0, sg1, h->pcnt_dev, j0, L, h->fused_ntiles};
-  void *args[] = {&d, &pv, &a};
+  PersistArgs a{x.vel, h->vel_alt, sg0, sg1, h->pcnt_dev, j0, L, h->fused_ntiles, x.nhalo, x.halo_dst, x.halo_src};
+  void *args[] = {&pv, &a};
   HIP_TRY(hipLaunchCooperativeKernel((const void *)fn, dim3(grid), dim3(h->pair_block), args, lds, h->stream));
   return EVP1D_OK;
 }
@@ -1914,9 +1575,33 @@ static int issue_fused(evp1d_handle *h, int nsub, double2 *traj = nullptr, bool 
   FusedView f;
   RC_TRY(fused_prologue(h, X, f, ip, fills));
   const long t_end = h->v.t_end;
-  PairView pv{h->ptiles_dev, h->hlist_dev, h->pxlist_dev, h->pelist_dev, h->puloc_dev, h->pvloc_dev,
-              h->pcstr_dev,  h->cnz_dev,   h->pk_total,   nullptr,       h->pair_cap,  h->pconst,
-              (long)h->na,   nullptr,      nullptr,       h->ldsig,      h->ptnbr_dev,  h->pfix_dev};
+  PairView pv{};
+  pv.s = X.s;
+  pv.tiles = h->ptiles_dev;
+  pv.hlist = h->hlist_dev;
+  pv.xlist = h->pxlist_dev;
+  pv.elist = h->pelist_dev;
+  pv.uloc = h->puloc_dev;
+  pv.vloc = h->pvloc_dev;
+  pv.cstr = h->pcstr_dev;
+  pv.cnz = h->cnz_dev;
+  pv.nk = h->pk_total;
+  pv.cap = h->pair_cap;
+  pv.xcd = h->tile_xcd;
+  pv.pc = h->pconst;
+  pv.lp = h->na;
+  pv.strength = X.strength;
+  pv.ls = h->ldsig;
+  pv.tnbr = h->ptnbr_dev;
+  pv.fix = h->pfix_dev;
+  pv.u_begin = X.u_begin;
+  pv.s15 = X.s15;
+  pv.s27 = X.s27;
+  pv.s36 = X.s36;
+  pv.s48 = X.s48;
+  pv.strintx = X.strintx;
+  pv.strinty = X.strinty;
+  pv.cb = X.cb;
   if (pair && h->na > 0 && !h->pconst_fresh) {
     hipLaunchKernelGGL(k_pack_const, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, X, h->pconst, (long)h->na);
     HIP_TRY(hipGetLastError());
@@ -1951,20 +1636,17 @@ static int issue_fused(evp1d_handle *h, int nsub, double2 *traj = nullptr, bool 
         pin = (pin + (L - j + 1)) % 2;
         break;
       }
-      pv.vel_out = out.vel;
-      pv.sg_in = P[pin];
-      pv.sg_out = P[1 - pin];
+      const PairBufs bufs{in.vel, out.vel, P[pin], P[1 - pin]};
       pin = 1 - pin;
-      const int nt = pair_hints(h) ? 1 : 0;
-      PairFn fn = (h->v.nhalo > 0 ? kPairFixFns : kPairFns)[pair_block_index(h->pair_block)][h->tile_xcd ? 1 : 0][nt];
+      const PairKind kind = traj ? kPairTraj : h->v.nhalo > 0 ? kPairFix : kPairPlain;
+      const PairFn fn = kPairFns[pair_block_index(h->pair_block)][kind][pair_hints(h) ? 1 : 0];
       if (traj) {
         const int before = odd_first ? 2 * j - 3 : 2 * j - 2;   // subcycles done before this launch
         pv.tr_mid = traj + (size_t)(before + 1) * nu;
         pv.tr_end = before + 2 < nsub ? traj + (size_t)(before + 2) * nu : nullptr;
-        fn = kPairTrajFns[pair_block_index(h->pair_block)][nt];
       }
       if (h->fused_ntiles > 0) {
-        hipLaunchKernelGGL(fn, dim3(h->fused_ntiles), dim3(h->pair_block), lds2, h->stream, in, pv, j == L ? 1 : 0);
+        hipLaunchKernelGGL(fn, dim3(h->fused_ntiles), dim3(h->pair_block), lds2, h->stream, pv, bufs, j == L ? 1 : 0);
         HIP_TRY(hipGetLastError());
       }
       if (h->v.nhalo > 0) {   // the copy after the launch's second subcycle

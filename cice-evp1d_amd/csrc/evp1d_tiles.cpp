@@ -323,6 +323,42 @@ struct TileWork {
 
 }  // namespace
 
+namespace {
+constexpr int kCus = 256;   // compute units of an MI355X
+}
+
+// The first rung that gives at most `most` tiles.  A tile's time is its chain
+// of four phases, whatever runs beside it, until the CUs are full.  So with
+// at most one tile per CU the smallest tile is the fastest: in 15x11 every
+// phase is one pass of 256 threads (18x14 cells at level 1), in 22x16 one of
+// 512.  Measured on 1D lists, 31x19 / chosen, us per subcycle: 64x48 5.3 /
+// 4.0, 200x150 6.2 / 4.1, 300x220 6.9 / 5.9, 520x400 11.1 / 10.3 (31x15).
+// Beyond two tiles per CU the border's extra work counts: 31x19.
+TileIds pair_tiles(const GridCoords &c, int order, int *block) {
+  struct Rung { int w, h, block, most; };
+  static const Rung rungs[5] = {
+      {15, 11, 256, kCus}, {22, 16, 512, kCus}, {31, 19, 512, kCus}, {31, 15, 512, 2 * kCus}, {31, 19, 512, 0}};
+  TileIds t;
+  for (const Rung &r : rungs) {
+    if (r.most > 0 && (int64_t)c.gx.size() / (r.w * r.h) > r.most) continue;
+    t = tile_ids(c, r.w, r.h, order);
+    *block = r.block;
+    if (t.ntiles <= r.most) break;
+  }
+  return t;
+}
+
+// 31x19 where its busiest tile has more than 512 level-2 stress points
+// (contiguous ice: 32x20) takes workgroups of 1024 threads, one per CU, which
+// nothing overlaps: 31x15 then (at most 512, two per CU).  1280x1520 in
+// contiguous ice 75.4 / 61.2 us per subcycle, 733x517 17.9 / 15.4.
+bool pair_may_crowd(const TileIds &t) { return t.tile_w == 31 && t.tile_h == 19 && t.ntiles > kCus; }
+bool pair_uncrowd(const GridCoords &c, int na, const int32_t *const idx[6], const uint8_t *skip, TileIds &t) {
+  if (!pair_may_crowd(t) || max_level2(na, idx, skip, t) <= 512) return false;
+  t = tile_ids(c, 31, 15, t.order);
+  return true;
+}
+
 // T point q is read by the stepu points ee(q), ne(q) and se(q) (as their nw,
 // sw and sse neighbour): it is a halo entry of the other tiles among theirs.
 int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids) {
@@ -710,12 +746,12 @@ struct PairWork {
 };
 }  // namespace
 
-// ghost slot -> copy-list source slot (-1: zero), or -2 when not listed
-std::vector<int32_t> halo_map(const HaloList &halo, int na, int navel) {
-  std::vector<int32_t> m((size_t)std::max(navel - na, 0), -2);
+// slot -> copy-list source slot (-1: zero), or -2 when not a destination
+static std::vector<int32_t> halo_map(const HaloList &halo, int navel) {
+  std::vector<int32_t> m((size_t)navel, -2);
   for (int k = 0; k < halo.n; ++k) {
     const int32_t d = halo.dst[k];
-    if (d >= na && d < navel) m[(size_t)(d - na)] = halo.src[k] < 0 ? -1 : halo.src[k];
+    if (d >= 0 && d < navel) m[(size_t)d] = halo.src[k] < 0 ? -1 : halo.src[k];
   }
   return m;
 }
@@ -730,7 +766,7 @@ PairPlan plan_pairs(const TilePlan &p, int na, int navel, const int32_t *const i
   }
   const int t_end = p.cnt[0] + p.cnt[1], u_begin = p.cnt[0], u_end = t_end + p.cnt[2];
   const std::vector<int32_t> inv = inverse_perm(p, na);
-  const std::vector<int32_t> hmap = halo_map(halo, na, navel);
+  const std::vector<int32_t> hmap = halo_map(halo, navel);
   auto slot = [&](int32_t q) { return q < na ? inv[(size_t)q] : q; };
   const int nt = (int)p.tiles.size();
   std::vector<PairWork> work((size_t)nt);
@@ -760,8 +796,8 @@ PairPlan plan_pairs(const TilePlan &p, int na, int navel, const int32_t *const i
       for (int c = 0; c < 4; ++c) {
         uint16_t en = PairPlan::kNoEntry;
         int32_t s = src[c];
-        const bool ghost = s >= na && hmap[(size_t)(s - na)] != -2;
-        if (ghost) s = hmap[(size_t)(s - na)];
+        const bool ghost = hmap[(size_t)s] != -2;
+        if (ghost) s = hmap[(size_t)s];
         if (s >= u_begin && s < u_end) {
           const int v = vm.find_or_add(s, nUo + (int)wk.e.size(), added);
           if (added) wk.e.push_back(s);
@@ -895,7 +931,7 @@ std::string check_pairs(const PairPlan &q, const TilePlan &p, int na, int navel,
   if (q.tiles.size() != p.tiles.size()) return "pair plan and tiling differ in tiles";
   const int t_end = p.cnt[0] + p.cnt[1], u_begin = p.cnt[0], u_end = t_end + p.cnt[2];
   const std::vector<int32_t> inv = inverse_perm(p, na);
-  const std::vector<int32_t> hmap = halo_map(halo, na, navel);
+  const std::vector<int32_t> hmap = halo_map(halo, navel);
   auto slot = [&](int32_t r) { return r < na ? inv[(size_t)r] : r; };
   std::vector<std::string> err(q.tiles.size());
   std::vector<std::vector<int32_t>> smaps((size_t)plan_threads()), vmaps((size_t)plan_threads());
@@ -970,8 +1006,8 @@ std::string check_pairs(const PairPlan &q, const TilePlan &p, int na, int navel,
       const int32_t want[4] = {g, slot(idx[0][r0]), slot(idx[1][r0]), slot(idx[2][r0])};
       for (int c = 0; c < 4; ++c) {
         const int en = q.vloc[(size_t)4 * (pt.v0 + k) + c];
-        const bool ghost = want[c] >= na && hmap[(size_t)(want[c] - na)] != -2;
-        const int32_t s = ghost ? hmap[(size_t)(want[c] - na)] : want[c];
+        const bool ghost = hmap[(size_t)want[c]] != -2;
+        const int32_t s = ghost ? hmap[(size_t)want[c]] : want[c];
         const bool active = s >= u_begin && s < u_end;
         bool ok;
         if (en == PairPlan::kNoEntry)

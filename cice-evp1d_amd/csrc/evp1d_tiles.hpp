@@ -136,6 +136,14 @@ TileIds tile_ids(int na, int navel, const int32_t *const idx[6], int tile_w, int
 // (its level-2 entries in the pair form, one thread each) for these flags.
 int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids);
 
+// The pair form's tiles by domain size; *block: the workgroup size that one
+// subcycle per launch uses on the same tiles.
+TileIds pair_tiles(const GridCoords &c, int order, int *block);
+// Whether those tiles can be crowded by contiguous ice, and the smaller ones
+// that replace them where they are (false: t stays).
+bool pair_may_crowd(const TileIds &t);
+bool pair_uncrowd(const GridCoords &c, int na, const int32_t *const idx[6], const uint8_t *skip, TileIds &t);
+
 // idx: ee, ne, se, nw, sw, sse as 0-based caller positions (values in
 // [0, navel); positions >= na are ghost slots).  skip: bit0 skipT, bit1 skipU.
 // idx may be null (no tiling, class order only).
@@ -184,8 +192,8 @@ struct PairPlan {
   // its ee, ne, se neighbours, so one load gives every address the entry's
   // stress gathers
   Table<int32_t> tnbr;
-  // Ghost copy list (evp1d_set_halo): between the two subcycles of a launch
-  // a listed ghost slot holds the copy of its source.  A level-2 read of such
+  // Copy list (evp1d_set_halo, evp2d_set_halo): between the two subcycles of a
+  // launch a listed slot holds the copy of its source.  A level-2 read of such
   // a ghost names the source's level-1 velocity entry when the source is an
   // active U point; otherwise vloc holds kFixBase + j and fix[f0 + j] is the
   // source slot (a velocity no subcycle changes) or -1 (the copy is zero).
@@ -196,8 +204,9 @@ struct PairPlan {
   static constexpr uint16_t kFixBase = 0xc000;   // velocity table entries stay below it
 };
 
-// Ghost copy list in slot space: ghost slot dst[k] (>= na) takes the value
-// of slot src[k] (< na) or zero (src[k] < 0) after every subcycle.
+// Copy list in slot space: slot dst[k], a ghost or another slot that no stepu
+// writes, takes the value of slot src[k] or zero (src[k] < 0) after every
+// subcycle.
 struct HaloList {
   int n = 0;
   const int32_t *dst = nullptr, *src = nullptr;

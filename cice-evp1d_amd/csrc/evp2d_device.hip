@@ -34,10 +34,13 @@
 #include <cstdio>
 #include <cstring>
 #include <new>
+#include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/evp1d.h"
 #include "evp1d_cache.hpp"
+#include "evp1d_pair.hpp"
 #include "evp1d_point.hpp"
 #include "evp1d_tiles.hpp"
 #include "evp1d_xcd.hpp"
@@ -311,6 +314,51 @@ __global__ __launch_bounds__(kB2F) void k2_fused(View2 v, Fused2 f, int last) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// pair form: two subcycles per launch (evp1d_pair.hpp)
+// ---------------------------------------------------------------------------
+// The cells of the lists become a 1D point list in slot order (class, then
+// tile), with the neighbours at the cell offsets and the halo update as its
+// copy list, so the planner, the tiles and the kernel are the 1D engine's.
+// What changes during a run lives by slot: velocities and stresses, gathered
+// from the block arrays before the run and scattered after it.  As in the 1D
+// list the kernel is bound by the latency of its phases at 16 waves per CU,
+// with half the bytes of k2_fused: 1280x1520 in one block, 1000 subcycles,
+// 88 -> 65 us per subcycle; 800x600 in 2 x 2 blocks, 120 subcycles, 26.7 ->
+// 21.5 us, where the halo update is one launch per two subcycles, not four.
+
+// velocities of every slot, into both buffers
+__global__ void k2p_vel(double2 *a, double2 *b, const double2 *vel, const int32_t *cell, int n) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const double2 v = vel[cell[s]];
+  a[s] = v;
+  b[s] = v;
+}
+// constant fields of every point (kPairT<true> stress pairs, seven stepu pairs)
+__global__ void k2p_const(View2 v, const int32_t *cell, double2 *pc, long lp) {
+  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= lp) return;
+  const long c = cell[s];
+  pc[s] = make_double2(v.dxt[c], v.dyt[c]);
+  pc[lp + s] = make_double2(v.strength[c], v.dmin[c]);
+  pc[2 * lp + s] = make_double2(v.cxp[c], v.cyp[c]);
+  pc[3 * lp + s] = make_double2(v.cxm[c], v.cym[c]);
+  pc[4 * lp + s] = make_double2(v.dxhy[c], v.dyhx[c]);
+  pc[5 * lp + s] = make_double2(v.cw[c], v.aix[c]);
+  pc[6 * lp + s] = make_double2(v.uocn[c], v.vocn[c]);
+  pc[7 * lp + s] = make_double2(v.waterx[c], v.watery[c]);
+  pc[8 * lp + s] = make_double2(v.forcex[c], v.forcey[c]);
+  pc[9 * lp + s] = make_double2(v.umassdti[c], v.fm[c]);
+  pc[10 * lp + s] = make_double2(v.uarear[c], v.tbu[c]);
+  pc[11 * lp + s] = v.vinit[c];
+}
+// stepu slots' velocities back into the block array
+__global__ void k2p_vel_back(double2 *vel, const double2 *a, const int32_t *cell, int u_begin, int u_end) {
+  const int s = u_begin + blockIdx.x * blockDim.x + threadIdx.x;
+  if (s < u_end) vel[cell[s]] = a[s];
+}
+
 // halo update of uvel and vvel (vars.F90:113-142): the fill, then the copies
 __global__ void k2_fill(double2 *vel, const int32_t *cells, int n) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -368,7 +416,22 @@ struct evp2d_handle {
   double2 *sg_dev[2] = {nullptr, nullptr};             // packed stresses during a run
   long et = 0, eu = 0, no = 0;                          // T entries, U entries, owned T cells
   int ntiles = 0;
+  bool tiles_built = false;   // the one-subcycle form's tables
   double2 *vel_alt = nullptr;
+  // pair form: the planned 1D list of the cells and its tables
+  bool pair_built = false, pair_ok = false;
+  int list_runs = 0;          // fused runs since the lists or the halo tables changed
+  int na = 0, nslots = 0;     // points, and with the unchanging cells that they read
+  int t_end = 0, u_begin = 0, u_end = 0;
+  int ptiles = 0, pblock = 0, pcap = 0, pcapv = 0, pnhalo = 0;
+  std::vector<void *> pbufs;
+  const evp1d::PairTile *ptiles_dev = nullptr;
+  const int32_t *phlist = nullptr, *pxlist = nullptr, *pelist = nullptr, *pfix = nullptr, *pcell = nullptr;
+  const int32_t *phdst = nullptr, *phsrc = nullptr;
+  const uint2 *puloc = nullptr, *pvloc = nullptr;
+  const int4 *ptnbr = nullptr;
+  int *pcnz = nullptr;
+  double2 *pvel[2] = {nullptr, nullptr}, *psig[2] = {nullptr, nullptr}, *pconst = nullptr;
   // captured subcycle loop
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -400,6 +463,11 @@ void free_lists2(evp2d_handle *h) {
   h->tc_dev = h->uc_dev = h->sg_dev[0] = h->sg_dev[1] = nullptr;
   h->et = h->eu = h->no = 0;
   h->ntiles = 0;
+  h->tiles_built = false;
+  for (void *b : h->pbufs) (void)hipFree(b);
+  h->pbufs.clear();
+  h->pair_built = h->pair_ok = false;
+  h->list_runs = 0;
 }
 
 void release2(evp2d_handle *h) {
@@ -430,6 +498,7 @@ int alloc2(evp2d_handle *h, void **ptr, size_t bytes) {
 // on the first row, and of the south-west tile when both; LDS entry of cell
 // (i, j) in tile (tx, ty): (j-1 - ty*kTH) * (kTW+1) + (i-1 - tx*kTW).
 int build_tiles2(evp2d_handle *h) {
+  h->tiles_built = true;
   const int ntx = (h->nxb + kTW - 1) / kTW, nty = (h->nyb + kTH - 1) / kTH;
   const long nt_all = (long)h->nblocks * ntx * nty;
   std::vector<std::vector<int32_t>> own((size_t)nt_all), halo((size_t)nt_all), uc((size_t)nt_all);
@@ -537,6 +606,194 @@ int build_tiles2(evp2d_handle *h) {
   return EVP1D_OK;
 }
 
+// The pair form serves runs of at least kPairMinSub subcycles (it gathers and
+// scatters the state once per run) on lists that have been run before, or of
+// at least kPairFirstSub.  Its plan costs more host time than the
+// one-subcycle tables (at 1280x1520 about 40 ms more, against 26 us saved per
+// subcycle; at 800x600 10 ms against 5 us), so lists that are used for one
+// run, as when every model step has its own ice mask, are not planned.
+constexpr int kPairMinSub = 4, kPairFirstSub = 2000;
+bool wants_pair(const evp2d_handle *h, int nsub) {
+  return nsub >= kPairMinSub && (h->list_runs > 0 || nsub >= kPairFirstSub);
+}
+
+typedef void (*Pair2Fn)(PairView, PairBufs, int);
+// [workgroup size][with a copy list][cache hints]
+#define PAIR2_ROW(B)                                                  \
+  {{k_pair<B, true>, k_pair<B, true, false, false, true>},            \
+   {k_pair<B, true, false, true>, k_pair<B, true, false, true, true>}}
+const Pair2Fn kPair2Fns[kNumPairBlocks][2][2] = {PAIR2_ROW(256), PAIR2_ROW(512), PAIR2_ROW(1024)};
+#undef PAIR2_ROW
+
+// The pair form's list, plan and tables; pair_ok stays false where they do
+// not fit (then runs use one subcycle per launch).
+int build_pairs2(evp2d_handle *h) {
+  h->pair_built = true;
+  const int nxb = h->nxb;
+  enum : uint8_t { kT = 1, kU = 2, kFill = 4 };
+  std::vector<uint8_t> mark((size_t)h->n, 0);
+  for (const auto &l : h->tl)
+    for (int32_t c : l) mark[(size_t)c] |= kT;
+  for (const auto &l : h->ul)
+    for (int32_t c : l) mark[(size_t)c] |= kU;
+  // cells that the halo update writes, and where each takes its value (-1: zero)
+  std::vector<int32_t> hd, hs;
+  const bool halo = h->halo_on && h->nblocks > 1;
+  if (halo) {
+    for (int32_t c : h->fill_h) mark[(size_t)c] |= kFill;
+    for (int32_t c : h->dst_h) mark[(size_t)c] &= (uint8_t)~kFill;
+    for (size_t k = 0; k < h->fill_h.size(); ++k)
+      if (mark[(size_t)h->fill_h[k]] & kFill) {
+        hd.push_back(h->fill_h[k]);
+        hs.push_back(-1);
+      }
+    for (size_t k = 0; k < h->dst_h.size(); ++k) {
+      const int32_t c = h->src_h[k];
+      hd.push_back(h->dst_h[k]);
+      hs.push_back(c >= 0 && (mark[(size_t)c] & kFill) ? -1 : c);   // a filled cell is copied as zero
+    }
+    for (int32_t c : hd)
+      if (mark[(size_t)c] & kU) return EVP1D_OK;   // stepu writes a halo cell too: one subcycle per launch
+  }
+  // points: the cells of the lists in cell order; then one unchanging slot
+  // that nothing reads, and the other cells whose velocity a T point or a
+  // copy reads
+  std::vector<int32_t> pos((size_t)h->n, -1), cell;
+  for (long c = 0; c < h->n; ++c)
+    if (mark[(size_t)c] & (kT | kU)) {
+      pos[(size_t)c] = (int32_t)cell.size();
+      cell.push_back((int32_t)c);
+    }
+  const int na = (int)cell.size();
+  if (na == 0 || (long)h->nblocks * (nxb + 1) > 0x7fffffffL) return EVP1D_OK;
+  const int32_t dummy = na;
+  cell.push_back(0);
+  auto ghost = [&](long c) {
+    int32_t &p = pos[(size_t)c];
+    if (p < 0) {
+      p = (int32_t)cell.size();
+      cell.push_back((int32_t)c);
+    }
+    return p;
+  };
+  // ee, ne, se, nw, sw, sse of every point: (di, dj) of each
+  static const int di[6] = {-1, -1, 0, 1, 1, 0}, dj[6] = {0, -1, -1, 0, 1, 1};
+  std::vector<int32_t> nb[6];
+  const int32_t *idx[6];
+  for (int k = 0; k < 6; ++k) {
+    nb[k].resize((size_t)na);
+    idx[k] = nb[k].data();
+  }
+  std::vector<uint8_t> skip((size_t)na);
+  for (int p = 0; p < na; ++p) {
+    const long c = cell[(size_t)p], l = c % h->plane;
+    const int i = (int)(l % nxb), j = (int)(l / nxb);
+    const uint8_t m = mark[(size_t)c];
+    skip[(size_t)p] = (uint8_t)((m & kT ? 0 : 1) | (m & kU ? 0 : 2));
+    for (int k = 0; k < 6; ++k) {
+      const int ii = i + di[k], jj = j + dj[k];
+      int32_t q = dummy;
+      if (ii >= 0 && ii < nxb && jj >= 0 && jj < h->nyb) {
+        const long cc = c + dj[k] * (long)nxb + di[k];
+        q = pos[(size_t)cc];
+        if (q >= na || q < 0) q = k < 3 && (m & kT) ? ghost(cc) : dummy;   // str of other cells is zero
+      }
+      nb[k][(size_t)p] = q;
+    }
+  }
+  std::vector<int32_t> hdst, hsrc;   // by position; the cells that some point reads
+  for (size_t k = 0; k < hd.size(); ++k) {
+    const int32_t d = pos[(size_t)hd[k]];
+    if (d < 0) continue;
+    hdst.push_back(d);
+    hsrc.push_back(hs[k] < 0 ? -1 : ghost(hs[k]));
+  }
+  const int nslots = (int)cell.size();
+  // the cells' own coordinates, the blocks side by side
+  evp1d::GridCoords coords;
+  coords.ok = true;
+  coords.width = (int64_t)h->nblocks * (nxb + 1);
+  coords.height = h->nyb;
+  coords.gx.resize((size_t)na);
+  coords.gy.resize((size_t)na);
+  for (int p = 0; p < na; ++p) {
+    const long c = cell[(size_t)p], l = c % h->plane;
+    coords.gx[(size_t)p] = (int32_t)((c / h->plane) * (nxb + 1) + l % nxb);
+    coords.gy[(size_t)p] = (int32_t)(l / nxb);
+  }
+  int block1 = 0;
+  evp1d::TileIds ids = evp1d::pair_tiles(coords, 0, &block1);
+  if (ids.ntiles == 0) return EVP1D_OK;
+  evp1d::pair_uncrowd(coords, na, idx, skip.data(), ids);
+  const evp1d::TilePlan plan = evp1d::plan_tiles(na, nslots, idx, skip.data(), ids, kPairMaxLds / 64);
+  std::string bad = evp1d::check_plan(plan, na, nslots, idx, skip.data());
+  if (!bad.empty()) return fail2(EVP1D_EINDEX, "evp2d slot layout: %s", bad.c_str());
+  if (!plan.ok) return EVP1D_OK;
+  std::vector<int32_t> inv((size_t)na);
+  for (int s = 0; s < na; ++s) inv[(size_t)plan.perm[(size_t)s]] = s;
+  auto slot = [&](int32_t p) { return p >= 0 && p < na ? inv[(size_t)p] : p; };
+  for (int32_t &p : hdst) p = slot(p);
+  for (int32_t &p : hsrc) p = slot(p);
+  evp1d::HaloList hl;
+  hl.n = (int)hdst.size();
+  hl.dst = hdst.data();
+  hl.src = hsrc.data();
+  const evp1d::PairPlan q = evp1d::plan_pairs(plan, na, nslots, idx, skip.data(), kPairMaxLds / 64, kPairMaxLds / 16,
+                                              kPairBlocks[kNumPairBlocks - 1], hl);
+  if (!q.ok) return EVP1D_OK;
+  bad = evp1d::check_pairs(q, plan, na, nslots, idx, skip.data(), hl);
+  if (!bad.empty()) return fail2(EVP1D_EINDEX, "evp2d pair plan: %s", bad.c_str());
+  const int cap = std::max(q.cap_s, 1), capv = std::max(q.cap_v, 1);
+  if (pair_lds(cap, capv) > (size_t)kPairMaxLds) return EVP1D_OK;
+  std::vector<int32_t> scell((size_t)nslots);
+  for (int s = 0; s < nslots; ++s) scell[(size_t)s] = cell[(size_t)(s < na ? plan.perm[(size_t)s] : s)];
+  auto get = [&](auto **dst, const void *src, size_t bytes) -> int {
+    void *p = nullptr;
+    HIP2(hipMalloc(&p, std::max<size_t>(bytes, 256)));
+    h->pbufs.push_back(p);
+    if (src && bytes) HIP2(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, h->stream));
+    *dst = static_cast<std::remove_reference_t<decltype(*dst)>>(p);
+    return EVP1D_OK;
+  };
+  auto up = [&](auto **dst, const auto &v) { return get(dst, v.data(), v.size() * sizeof(v[0])); };
+  RC2(up(&h->ptiles_dev, q.tiles));
+  RC2(up(&h->phlist, plan.list));
+  RC2(up(&h->pxlist, q.xlist));
+  RC2(up(&h->pelist, q.elist));
+  RC2(up(&h->puloc, q.uloc));
+  RC2(up(&h->pvloc, q.vloc));
+  RC2(up(&h->ptnbr, q.tnbr));
+  RC2(up(&h->pfix, q.fix));
+  RC2(up(&h->pcell, scell));
+  RC2(up(&h->phdst, hdst));
+  RC2(up(&h->phsrc, hsrc));
+  const std::vector<int> zero(1, 0);
+  RC2(up(&h->pcnz, zero));   // str of every cell outside the T list is zero
+  h->t_end = plan.cnt[0] + plan.cnt[1];
+  h->u_begin = plan.cnt[0];
+  h->u_end = h->t_end + plan.cnt[2];
+  const size_t n2 = sizeof(double2);
+  RC2(get(&h->pconst, nullptr, n2 * (size_t)(kPairT<true> + kPairU) * na));
+  for (int b = 0; b < 2; ++b) {
+    RC2(get(&h->pvel[b], nullptr, n2 * nslots));
+    RC2(get(&h->psig[b], nullptr, n2 * 6 * std::max(h->t_end, 1)));
+  }
+  HIP2(hipStreamSynchronize(h->stream));   // the host tables go out of scope
+  int b = 0;
+  while (kPairBlocks[b] < q.max_t2) ++b;   // max_t2 <= the largest block (plan limit)
+  h->pblock = kPairBlocks[b];
+  h->pcap = cap;
+  h->pcapv = capv;
+  h->na = na;
+  h->nslots = nslots;
+  h->pnhalo = (int)hdst.size();
+  h->ptiles = (int)q.tiles.size();
+  for (const auto &kind : kPair2Fns[b])
+    for (Pair2Fn fn : kind)
+      HIP2(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
+  h->pair_ok = true;
+  return EVP1D_OK;
+}
 // upload the concatenated lists (and the halo tables) when they changed;
 // a host allocation failure while building them returns EVP1D_ENOMEM
 int ensure2_impl(evp2d_handle *h);
@@ -564,7 +821,6 @@ int ensure2_impl(evp2d_handle *h) {
   RC2(up(&h->fill_dev, h->fill_h));
   RC2(up(&h->dst_dev, h->dst_h));
   RC2(up(&h->src_dev, h->src_h));
-  RC2(build_tiles2(h));
   // str outside the lists must read as zero (the reference clears it)
   if (h->lists_dirty)
     for (double2 *s : h->str) HIP2(hipMemsetAsync(s, 0, (size_t)h->n * sizeof(double2), h->stream));
@@ -576,6 +832,18 @@ int ensure2_impl(evp2d_handle *h) {
   h->v.nu = (int)u.size();
   h->cells_dirty = false;
   h->graph_dirty = true;
+  return EVP1D_OK;
+}
+
+// the tables of the form that a run of nsub subcycles takes
+int ensure_form2(evp2d_handle *h, int nsub) {
+  if (wants_pair(h, nsub) && !h->pair_built)
+    RC2(evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); }));
+  const bool pair = wants_pair(h, nsub) && h->pair_ok;
+  if ((!pair || nsub % 2 == 1) && !h->tiles_built)
+    RC2(evp1d::no_throw("evp2d tiles", [h] { return build_tiles2(h); }));
+  if ((!pair || nsub % 2 == 1) && !h->vel_alt)
+    HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
   return EVP1D_OK;
 }
 
@@ -626,6 +894,13 @@ bool hints2(const evp2d_handle *h) {
   const double reread = 100.0 * h->et + 124.0 * h->eu + 32.0 * h->n;
   return hints_pay(reread, reread + 192.0 * h->no);
 }
+// The pair form's, as for the 1D list (there the stress constants are 56 B,
+// here 80).
+bool pair_hints2(const evp2d_handle *h) {
+  if (h->cache_hints >= 0) return h->cache_hints != 0;
+  const double reread = 152.0 * (h->u_end - h->u_begin) + 16.0 * h->nslots;
+  return hints_pay(reread, reread + 272.0 * h->t_end);
+}
 
 // nsub fused subcycles.  The velocities start in the handle's buffer (X),
 // are copied to the second one (Y), and the subcycles alternate so that the
@@ -664,6 +939,72 @@ int issue_fused2(evp2d_handle *h, int nsub) {
                        (const int32_t *)h->ocell_dev, (const double2 *)h->sg_dev[cur], h->no);
   HIP2(hipGetLastError());
   return EVP1D_OK;
+}
+
+// nsub subcycles of the fused mode: the pair form, after one subcycle of
+// k2_fused when nsub is odd, or k2_fused alone.  After every pair launch the
+// halo copies that some point reads are made by slot; after the run the halo
+// update of the block arrays sets the other halo cells too.
+int issue_run2(evp2d_handle *h, int nsub) {
+  if (!wants_pair(h, nsub) || !h->pair_ok) return issue_fused2(h, nsub);
+  if (nsub % 2 == 1) RC2(issue_fused2(h, 1));
+  const View2 &v = h->v;
+  PairView f{};
+  f.s = v.s;
+  f.tiles = h->ptiles_dev;
+  f.hlist = h->phlist;
+  f.xlist = h->pxlist;
+  f.elist = h->pelist;
+  f.uloc = h->puloc;
+  f.vloc = h->pvloc;
+  f.cnz = h->pcnz;
+  f.cap = h->pcap;
+  f.xcd = 1;
+  f.pc = h->pconst;
+  f.lp = h->na;
+  f.ls = std::max(h->t_end, 1);
+  f.tnbr = h->ptnbr;
+  f.fix = h->pfix;
+  f.u_begin = h->u_begin;
+  f.s15 = v.s15;
+  f.s27 = v.s27;
+  f.s36 = v.s36;
+  f.s48 = v.s48;
+  f.strintx = v.strintx;
+  f.strinty = v.strinty;
+  f.cb = v.taubx;
+  f.tauby = v.tauby;
+  f.cell = h->pcell;
+  hipLaunchKernelGGL(k2p_vel, dim3(blocks2(h->nslots)), dim3(kB2), 0, h->stream, h->pvel[0], h->pvel[1],
+                     (const double2 *)v.vel, h->pcell, h->nslots);
+  hipLaunchKernelGGL(k2p_const, dim3(blocks2(h->na)), dim3(kB2), 0, h->stream, v, h->pcell, h->pconst, (long)h->na);
+  if (h->t_end > 0)
+    hipLaunchKernelGGL(k2_pack_sig, dim3(blocks2(h->t_end)), dim3(kB2), 0, h->stream, (const double *)v.sig, h->n,
+                       h->pcell, h->psig[0], (long)h->t_end);
+  HIP2(hipGetLastError());
+  int b = 0;
+  while (kPairBlocks[b] != h->pblock) ++b;
+  const Pair2Fn fn = kPair2Fns[b][h->pnhalo > 0 ? 1 : 0][pair_hints2(h) ? 1 : 0];
+  const size_t lds = pair_lds(h->pcap, h->pcapv);
+  int cur = 0;
+  const int L = nsub / 2;
+  for (int j = 1; j <= L; ++j) {
+    const PairBufs bufs{h->pvel[cur], h->pvel[1 - cur], h->psig[cur], h->psig[1 - cur]};
+    hipLaunchKernelGGL(fn, dim3(h->ptiles), dim3(h->pblock), lds, h->stream, f, bufs, j == L ? 1 : 0);
+    cur = 1 - cur;
+    if (h->pnhalo > 0)
+      hipLaunchKernelGGL(k2_copy, dim3(blocks2(h->pnhalo)), dim3(kB2), 0, h->stream, h->pvel[cur], h->phdst, h->phsrc,
+                         h->pnhalo);
+    HIP2(hipGetLastError());
+  }
+  if (h->t_end > 0)
+    hipLaunchKernelGGL(k2_unpack_sig, dim3(blocks2(h->t_end)), dim3(kB2), 0, h->stream, v.sig, h->n, h->pcell,
+                       (const double2 *)h->psig[cur], (long)h->t_end);
+  if (h->u_end > h->u_begin)
+    hipLaunchKernelGGL(k2p_vel_back, dim3(blocks2(h->u_end - h->u_begin)), dim3(kB2), 0, h->stream, v.vel,
+                       (const double2 *)h->pvel[cur], h->pcell, h->u_begin, h->u_end);
+  HIP2(hipGetLastError());
+  return launch_halo2(h);
 }
 
 // field id -> where it lives
@@ -916,12 +1257,13 @@ int evp2d_run(evp2d_handle *h, int32_t nsub) {
   if (nsub < 0) return fail2(EVP1D_EINVAL, "evp2d_run: nsub=%d < 0", nsub);
   if (nsub == 0) return EVP1D_OK;
   RC2(ensure2(h));
+  const bool fused = h->mode == EVP2D_MODE_FUSED;
+  if (fused && !h->pair_built && wants_pair(h, nsub)) h->graph_dirty = true;   // captured before the lists were planned
   if (h->graph_dirty || h->graph_nsub != nsub || !h->exec) {
     drop_graph2(h);
-    const bool fused = h->mode == EVP2D_MODE_FUSED;
-    if (fused && !h->vel_alt) HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
+    if (fused) RC2(ensure_form2(h, nsub));
     HIP2(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = fused ? issue_fused2(h, nsub) : issue2(h, nsub);
+    const int rc = fused ? issue_run2(h, nsub) : issue2(h, nsub);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(h->stream, &g);
     if (rc) {
@@ -935,6 +1277,7 @@ int evp2d_run(evp2d_handle *h, int32_t nsub) {
     h->graph_dirty = false;
   }
   HIP2(hipGraphLaunch(h->exec, h->stream));
+  if (fused && h->list_runs < 1) ++h->list_runs;
   return EVP1D_OK;
 }
 
@@ -967,8 +1310,10 @@ int evp2d_set_cache_hints(evp2d_handle *h, int32_t hints) {
 int evp2d_get_cache_hints(evp2d_handle *h, int32_t *hints, int32_t *active) {
   if (!h) return fail2(EVP1D_EINVAL, "evp2d_get_cache_hints: NULL handle");
   RC2(ensure2(h));
+  if (h->mode == EVP2D_MODE_FUSED && active) RC2(ensure_form2(h, kPairMinSub));   // the form that runs use now
   if (hints) *hints = h->cache_hints;
-  if (active) *active = h->mode == EVP2D_MODE_FUSED && h->ntiles > 0 && hints2(h) ? 1 : 0;
+  if (active)
+    *active = h->mode == EVP2D_MODE_FUSED && (h->pair_ok ? pair_hints2(h) : h->ntiles > 0 && hints2(h)) ? 1 : 0;
   return EVP1D_OK;
 }
 
@@ -994,7 +1339,7 @@ int evp2d_run_individual(evp2d_handle *h, int32_t which, int32_t nsub) {
   RC2(ensure2(h));
   if (which == 2) {   // fused subcycles launched one by one (no graph)
     if (nsub <= 0) return EVP1D_OK;
-    if (!h->vel_alt) HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
+    RC2(ensure_form2(h, 1));
     return issue_fused2(h, nsub);
   }
   for (int k = 0; k < nsub; ++k) RC2(which == 0 ? launch_stress2(h) : launch_stepu2(h));

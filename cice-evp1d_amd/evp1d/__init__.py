@@ -663,7 +663,7 @@ class Engine2D:
         _check(self.L, self.L.evp2d_run(self.h, nsub))
 
     def set_mode(self, mode: str) -> None:
-        """"fused" (default): one tile kernel per subcycle; "plain": stress then stepu."""
+        """"fused" (default): one tile kernel per subcycle or per two; "plain": stress then stepu."""
         _check(self.L, self.L.evp2d_set_mode(self.h, {"plain": 0, "fused": 1}[mode]))
 
     def get_mode(self) -> str:

@@ -465,17 +465,22 @@ int evp2d_get_field(evp2d_handle *h, int32_t field, double *a, int64_t n);
  * max_blocks > 1 and tables are set (src/evp_v0.F90:93-136); a captured
  * hipGraph, asynchronous.                                                   */
 int evp2d_run(evp2d_handle *h, int32_t nsub);
-/* How evp2d_run runs a subcycle: EVP2D_MODE_FUSED (default) runs stress and
- * stepu of one 32 x 8 tile of cells per workgroup with str1..8 in LDS (the
- * T cells of the column east and the row north of the tile evaluated again),
- * velocities and stresses alternating between two buffers; EVP2D_MODE_PLAIN
- * runs the two kernels one after the other, as the reference does.  Results
- * are identical.                                                            */
+/* How evp2d_run runs the subcycles.  EVP2D_MODE_FUSED (default): two per
+ * launch with the 1D engine's pair form (evp1d_set_fused_depth), on the cells
+ * of the lists as a 1D list with the halo update as its copy list, when the
+ * same lists are run again (their plan takes host time) or for 2000
+ * subcycles and more; else, and where the pair tables do not fit or stepu
+ * writes a cell of the halo, one per launch: stress and stepu of one 32 x 8
+ * tile of cells per workgroup with str1..8 in LDS (the T cells of the column
+ * east and the row north of the tile evaluated again).  Velocities and
+ * stresses alternate between two buffers.  EVP2D_MODE_PLAIN runs the two
+ * kernels one after the other, as the reference does.  Results are
+ * identical.                                                                */
 enum evp2d_mode { EVP2D_MODE_PLAIN = 0, EVP2D_MODE_FUSED = 1 };
 int evp2d_set_mode(evp2d_handle *h, int32_t mode);
 int evp2d_get_mode(evp2d_handle *h, int32_t *mode);
-/* Cache hints of the fused form (no counterpart in the reference), as
- * evp1d_set_cache_hints: the tile kernel reads and writes its packed
+/* Cache hints of the fused forms (no counterpart in the reference), as
+ * evp1d_set_cache_hints: the tile kernels read and write their packed
  * stresses (and the last subcycle's str1..8) as non-temporal loads and
  * stores, so that the last-level cache keeps the packed constants, tables
  * and velocities between subcycles.  Same results bit for bit.  hints = -1
