@@ -12,10 +12,26 @@
 // are taken as products with its reciprocal), so no bit-exactness claim.
 #pragma once
 
-#include "evp1d_cache.hpp"
 #include "evp1d_point.hpp"
 
 namespace evp1d {
+
+// The compiler takes the value as a new one: products with it are computed
+// again rather than kept.
+template <class T>
+__host__ __device__ inline void fresh(T &v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(v));
+#endif
+}
+
+// Instructions are not moved across: keeps the compiler from interleaving
+// parts whose values would not fit the registers together.
+__host__ __device__ inline void sched_fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_sched_barrier(0);
+#endif
+}
 
 // ---------------------------------------------------------------------------
 // stepu (bench_v2b.F90:509-544)
@@ -89,89 +105,109 @@ __host__ __device__ inline void stepu_adjoint(const Scalars &s,
 __host__ __device__ inline void combos_adjoint(double dxT, double dyT, double dxhy, double dyhx,
                                                const double *b, double *sb) {
   const double b1 = b[0], b2 = b[1], b3 = b[2], b4 = b[3], b5 = b[4], b6 = b[5], b7 = b[6], b8 = b[7];
-  // str1..8 in terms of strp/strm/str12 and the csig terms
-  const double strp_a = -b1 + b2, strm_a = -b1 + b2;      // dF/dx north pair
-  const double strp_b = -b3 + b4, strm_b = -b3 + b4;      // dF/dx south pair
-  const double strp_c = -b5 + b6, strm_c = b5 - b6;       // dF/dy east pair
-  const double strp_d = -b7 + b8, strm_d = b7 - b8;       // dF/dy west pair
-  const double s12ew = -b1 + b3, s12we = -b2 + b4, s12ns = -b5 + b7, s12sn = -b6 + b8;
-  const double cpne = -dxhy * b1 - dyhx * b5, cmne = dxhy * b1 - dyhx * b5, c12ne = dyhx * b1 + dxhy * b5;
-  const double cpnw = -dxhy * b2 - dyhx * b7, cmnw = dxhy * b2 - dyhx * b7, c12nw = dyhx * b2 + dxhy * b7;
-  const double cpse = -dxhy * b3 - dyhx * b6, cmse = dxhy * b3 - dyhx * b6, c12se = dyhx * b3 + dxhy * b6;
-  const double cpsw = -dxhy * b4 - dyhx * b8, cmsw = dxhy * b4 - dyhx * b8, c12sw = dyhx * b4 + dxhy * b8;
-  // strp/strm = p25*d*(p333*A + p166*B)
+  // the three families one after the other: few values live at a time
   const double ay = p25 * dyT, ax = p25 * dxT;
-  const double pn = ay * (p333 * strp_a + p166 * strp_b), ps = ay * (p166 * strp_a + p333 * strp_b);
-  const double pe = ax * (p333 * strp_c + p166 * strp_d), pw = ax * (p166 * strp_c + p333 * strp_d);
-  const double mn = ay * (p333 * strm_a + p166 * strm_b), ms = ay * (p166 * strm_a + p333 * strm_b);
-  const double me = ax * (p333 * strm_c + p166 * strm_d), mw = ax * (p166 * strm_c + p333 * strm_d);
-  // str12 = p5*d*(p333*A + p166*B)
-  const double hx = p5 * dxT, hy = p5 * dyT;
-  const double e12 = hx * (p333 * s12ew + p166 * s12we), w12 = hx * (p166 * s12ew + p333 * s12we);
-  const double n12 = hy * (p333 * s12ns + p166 * s12sn), s12 = hy * (p166 * s12ns + p333 * s12sn);
   // csig p/m: csig_ne = p111*x1 + ssig2 + p027*x3, nw = p111*x2 + ssig1 + p027*x4,
   //           sw = p111*x3 + ssig2 + p027*x1, se = p111*x4 + ssig1 + p027*x2
   // ssig1 = (x1 + x3)*p055, ssig2 = (x2 + x4)*p055
-  const double qp1 = (cpnw + cpse) * p055, qp2 = (cpne + cpsw) * p055;
-  const double qm1 = (cmnw + cmse) * p055, qm2 = (cmne + cmsw) * p055;
+  // strp/strm = p25*d*(p333*A + p166*B); ssigpn = x1+x2, ps = x3+x4, pe = x1+x4, pw = x2+x3
+  {
+    const double a = -b1 + b2, b_ = -b3 + b4, c = -b5 + b6, d = -b7 + b8;   // strp: dF/dx north, south, dF/dy east, west
+    const double ne = -dxhy * b1 - dyhx * b5, nw = -dxhy * b2 - dyhx * b7;
+    const double se = -dxhy * b3 - dyhx * b6, sw = -dxhy * b4 - dyhx * b8;
+    const double n = ay * (p333 * a + p166 * b_), s = ay * (p166 * a + p333 * b_);
+    const double e = ax * (p333 * c + p166 * d), w = ax * (p166 * c + p333 * d);
+    const double q1 = (nw + se) * p055, q2 = (ne + sw) * p055;
+    sb[0] += n + e + p111 * ne + p027 * sw + q1;
+    sb[1] += n + w + p111 * nw + p027 * se + q2;
+    sb[2] += s + w + p111 * sw + p027 * ne + q1;
+    sb[3] += s + e + p111 * se + p027 * nw + q2;
+  }
+  sched_fence();
+  {
+    const double a = -b1 + b2, b_ = -b3 + b4, c = b5 - b6, d = b7 - b8;   // strm
+    const double ne = dxhy * b1 - dyhx * b5, nw = dxhy * b2 - dyhx * b7;
+    const double se = dxhy * b3 - dyhx * b6, sw = dxhy * b4 - dyhx * b8;
+    const double n = ay * (p333 * a + p166 * b_), s = ay * (p166 * a + p333 * b_);
+    const double e = ax * (p333 * c + p166 * d), w = ax * (p166 * c + p333 * d);
+    const double q1 = (nw + se) * p055, q2 = (ne + sw) * p055;
+    sb[4] += n + e + p111 * ne + p027 * sw + q1;
+    sb[5] += n + w + p111 * nw + p027 * se + q2;
+    sb[6] += s + w + p111 * sw + p027 * ne + q1;
+    sb[7] += s + e + p111 * se + p027 * nw + q2;
+  }
+  sched_fence();
   // csig12: ne = p222*x1 + ssig122 + p055*x3, nw = p222*x2 + ssig121 + p055*x4,
   //         sw = p222*x3 + ssig122 + p055*x1, se = p222*x4 + ssig121 + p055*x2
-  // ssig121 = (x1 + x3)*p111, ssig122 = (x2 + x4)*p111
-  const double q121 = (c12nw + c12se) * p111, q122 = (c12ne + c12sw) * p111;
-  // p family: ssigpn = x1+x2, ps = x3+x4, pe = x1+x4, pw = x2+x3
-  sb[0] += pn + pe + p111 * cpne + p027 * cpsw + qp1;
-  sb[1] += pn + pw + p111 * cpnw + p027 * cpse + qp2;
-  sb[2] += ps + pw + p111 * cpsw + p027 * cpne + qp1;
-  sb[3] += ps + pe + p111 * cpse + p027 * cpnw + qp2;
-  sb[4] += mn + me + p111 * cmne + p027 * cmsw + qm1;
-  sb[5] += mn + mw + p111 * cmnw + p027 * cmse + qm2;
-  sb[6] += ms + mw + p111 * cmsw + p027 * cmne + qm1;
-  sb[7] += ms + me + p111 * cmse + p027 * cmnw + qm2;
-  sb[8] += n12 + e12 + p222 * c12ne + p055 * c12sw + q121;
-  sb[9] += n12 + w12 + p222 * c12nw + p055 * c12se + q122;
-  sb[10] += s12 + w12 + p222 * c12sw + p055 * c12ne + q121;
-  sb[11] += s12 + e12 + p222 * c12se + p055 * c12nw + q122;
+  // ssig121 = (x1 + x3)*p111, ssig122 = (x2 + x4)*p111; str12 = p5*d*(p333*A + p166*B)
+  {
+    const double ew = -b1 + b3, we = -b2 + b4, ns = -b5 + b7, sn = -b6 + b8;
+    const double hx = p5 * dxT, hy = p5 * dyT;
+    const double ne = dyhx * b1 + dxhy * b5, nw = dyhx * b2 + dxhy * b7;
+    const double se = dyhx * b3 + dxhy * b6, sw = dyhx * b4 + dxhy * b8;
+    const double e = hx * (p333 * ew + p166 * we), w = hx * (p166 * ew + p333 * we);
+    const double n = hy * (p333 * ns + p166 * sn), s = hy * (p166 * ns + p333 * sn);
+    const double q1 = (nw + se) * p111, q2 = (ne + sw) * p111;
+    sb[8] += n + e + p222 * ne + p055 * sw + q1;
+    sb[9] += n + w + p222 * nw + p055 * se + q2;
+    sb[10] += s + w + p222 * sw + p055 * ne + q1;
+    sb[11] += s + e + p222 * se + p055 * nw + q2;
+  }
 }
 
-// Reverse of one subcycle's stress at one T point.  Inputs: the forward
-// inputs of stress_point, the adjoint of the updated stresses (sig_b_new[c *
-// ss], c = 0..11) and of str1..8 (str_b).  Writes the adjoint of the
-// stresses before the update to sig_b_out[c * ss] (which may be sig_b_new:
-// every element is read first), the velocity adjoint contributions at cc,
-// ee, se, ne to vel_b[8], and returns d/d strength.  The four corners are
-// reversed one after the other, each from its own strain rates, and feed the
-// velocity accumulators as they go: few values stay live (no per-corner
-// arrays), so the kernel keeps several waves per SIMD without spills.
-// NT: the adjoint stresses read and written with the cache hints
-// (evp1d_cache.hpp).
-template <bool NT = false>
-__host__ __device__ inline double stress_adjoint(const Scalars &s,
+// The scalars with the sums that the stress adjoint uses in every corner
+// (taken on the host: a uniform sum held in a register per lane costs the
+// kernels two VGPRs).
+struct AdjScalars {
+  Scalars s;
+  double keep;     // 1 - arlx1i*revp
+  double kp, km;   // 1 + Ktens, 1 - Ktens
+};
+inline AdjScalars adj_scalars(const Scalars &s) {
+  return AdjScalars{s, c1 - s.arlx1i * s.revp, c1 + s.Ktens, c1 - s.Ktens};
+}
+
+// Reverse of one subcycle's stress at one T point, the first part: adds the
+// str1..8 path (str_b, the adjoint of str1..8) to the adjoint of the updated
+// stresses (sb[12]).
+__host__ __device__ inline void stress_adjoint_sums(double dxT, double dyT, double hte, double htn, double htem1,
+                                                    double htnm1, const double *str_b, double *sb) {
+  combos_adjoint(dxT, dyT, p5 * (hte - htem1), p5 * (htn - htnm1), str_b, sb);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) fresh(sb[k]);
+  sched_fence();
+}
+
+// The second part.  Inputs: the forward inputs of stress_point and the sums
+// of the first (sb[12]).  Replaces sb by the adjoint of the stresses before
+// the update, writes the velocity adjoint contributions at cc, ee, se, ne to
+// vel_b[8], and returns d/d strength.  The four corners are reversed one
+// after the other, each from its own strain rates, and feed the velocity
+// accumulators as they go, so that few values stay live.  fresh and
+// sched_fence hold the compiler to that: left alone it sinks the corners' sums
+// into one another and keeps their common products, 184 VGPRs in all
+// (k_stress_adj, 2 waves per SIMD; 138 with them), and k_pair_adj, which may
+// have 128, spilled 122 of them.
+__host__ __device__ inline double stress_adjoint_corners(const AdjScalars &as,
     double uvel_cc, double vvel_cc, double uvel_ee, double vvel_ee,
     double uvel_se, double vvel_se, double uvel_ne, double vvel_ne,
     double dxT, double dyT, double strength,
     double hte, double htn, double htem1, double htnm1,
-    const double *sig_b_new, const double *str_b, double *sig_b_out, long ss, double *vel_b) {
+    double *sb, double *vel_b) {
+  const Scalars &s = as.s;
   const double cxp = c1p5 * htn - p5 * htnm1;
   const double cyp = c1p5 * hte - p5 * htem1;
   const double cxm = -(c1p5 * htnm1 - p5 * htn);
   const double cym = -(c1p5 * htem1 - p5 * hte);
   const double DminTarea = s.deltaminEVP * (dxT * dyT);
-  const double dxhy = p5 * (hte - htem1);
-  const double dyhx = p5 * (htn - htnm1);
-
-  // adjoint of the updated stresses including the str1..8 path
-  double sb[12];
-#pragma unroll
-  for (int k = 0; k < 12; ++k) sb[k] = in1<NT>(sig_b_new + k * ss);
-  combos_adjoint(dxT, dyT, dxhy, dyhx, str_b, sb);
-
-  const double keep = c1 - s.arlx1i * s.revp;
   const bool cap1 = s.capping == c1;
   double strength_b = 0.0;
   double ucc = 0, vcc = 0, uee = 0, vee = 0, use = 0, vse = 0, une = 0, vne = 0;
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     // strain rates and Delta of corner c: 0 ne, 1 nw, 2 sw, 3 se (stress index 1..4)
+    fresh(dxT);
+    fresh(dyT);
     double dv, tn, sh;
     if (c == 0) {
       dv = cyp * uvel_cc - dyT * uvel_ee + cxp * vvel_cc - dxT * vvel_se;
@@ -211,14 +247,14 @@ __host__ __device__ inline double stress_adjoint(const Scalars &s,
             (c1 - s.capping) * (-strength / (dsum * dsum));
       rD = D > 0.0 ? c1 / D : 0.0;
     }
-    const double zeta = (c1 + s.Ktens) * T;
+    const double zeta = as.kp * T;
     const double eta = s.epp2i * zeta;
     // sp = (sp0*keep + arlx1i*(zeta*div - rep))*denom1, rep = (1-K)*T*D
     // sm = (sm0*keep + arlx1i*eta*ten)*denom1, s12 = (s120*keep + arlx1i*p5*eta*shr)*denom1
     const double P = sb[c] * s.denom1, M = sb[4 + c] * s.denom1, Q = sb[8 + c] * s.denom1;
-    out1<NT>(sig_b_out + c * ss, P * keep);
-    out1<NT>(sig_b_out + (4 + c) * ss, M * keep);
-    out1<NT>(sig_b_out + (8 + c) * ss, Q * keep);
+    sb[c] = P * as.keep;
+    sb[4 + c] = M * as.keep;
+    sb[8 + c] = Q * as.keep;
     const double zeta_b0 = P * s.arlx1i * dv;
     const double rep_b = -P * s.arlx1i;
     const double eta_b = M * s.arlx1i * tn + Q * s.arlx1i * p5 * sh;
@@ -226,16 +262,15 @@ __host__ __device__ inline double stress_adjoint(const Scalars &s,
     double tn_b = M * s.arlx1i * eta;
     double sh_b = Q * s.arlx1i * p5 * eta;
     const double zeta_b = zeta_b0 + s.epp2i * eta_b;
-    const double T_b = (c1 + s.Ktens) * zeta_b + (c1 - s.Ktens) * D * rep_b;
-    double D_b = (c1 - s.Ktens) * T * rep_b;
+    const double T_b = as.kp * zeta_b + as.km * D * rep_b;
+    double D_b = as.km * T * rep_b;
     strength_b += T_b * T_s;
     D_b += T_b * T_D;
-    if (D > 0.0) {
-      const double w = D_b * rD;
-      dv_b += w * dv;
-      tn_b += w * s.e_factor * tn;
-      sh_b += w * s.e_factor * sh;
-    }
+    const double w = D > 0.0 ? D_b * rD : 0.0;   // the strain rates are 0 where Delta is
+    dv_b += w * dv;
+    tn_b += w * s.e_factor * tn;
+    sh_b += w * s.e_factor * sh;
+    sched_fence();
     // reverse of this corner's strain rates (linear in the 8 velocities)
     if (c == 0) {
       ucc += cyp * dv_b; uee -= dyT * dv_b; vcc += cxp * dv_b; vse -= dxT * dv_b;
@@ -254,12 +289,27 @@ __host__ __device__ inline double stress_adjoint(const Scalars &s,
       use -= cym * tn_b; une -= dyT * tn_b; vse += cxp * tn_b; vcc -= dxT * tn_b;
       vse -= cym * sh_b; vne -= dyT * sh_b; use -= cxp * sh_b; ucc += dxT * sh_b;
     }
+    fresh(ucc); fresh(vcc); fresh(uee); fresh(vee); fresh(use); fresh(vse); fresh(une); fresh(vne);
+    fresh(sb[c]); fresh(sb[4 + c]); fresh(sb[8 + c]); fresh(strength_b);
+    sched_fence();
   }
   vel_b[0] = ucc; vel_b[1] = vcc;
   vel_b[2] = uee; vel_b[3] = vee;
   vel_b[4] = use; vel_b[5] = vse;
   vel_b[6] = une; vel_b[7] = vne;
   return strength_b;
+}
+
+// both parts
+__host__ __device__ inline double stress_adjoint(const AdjScalars &as,
+    double uvel_cc, double vvel_cc, double uvel_ee, double vvel_ee,
+    double uvel_se, double vvel_se, double uvel_ne, double vvel_ne,
+    double dxT, double dyT, double strength,
+    double hte, double htn, double htem1, double htnm1,
+    double *sb, const double *str_b, double *vel_b) {
+  stress_adjoint_sums(dxT, dyT, hte, htn, htem1, htnm1, str_b, sb);
+  return stress_adjoint_corners(as, uvel_cc, vvel_cc, uvel_ee, vvel_ee, uvel_se, vvel_se, uvel_ne, vvel_ne, dxT, dyT,
+                                strength, hte, htn, htem1, htnm1, sb, vel_b);
 }
 
 }  // namespace evp1d

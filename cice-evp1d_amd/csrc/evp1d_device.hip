@@ -45,6 +45,7 @@
 #include "evp1d_point.hpp"
 #include "evp1d_cache.hpp"
 #include "evp1d_pair.hpp"
+#include "evp1d_pair_adj.hpp"
 #include "evp1d_xcd.hpp"
 
 #ifndef EVP1D_FMA
@@ -548,8 +549,9 @@ __global__ __launch_bounds__(kBlock) void k_persistent(DevView d, int nsub) {
 // adjoint kernels (reverse mode of one subcycle, see evp1d_adjoint.hpp)
 // ---------------------------------------------------------------------------
 struct AdjView {
+  evp1d::AdjScalars as;
   double2 *ub;            // [navel] adjoint of (uvel, vvel)
-  double *sigb;           // [12][ldsig] adjoint of the stresses
+  double2 *sigb;          // [6][ldsig] adjoint of the stresses, in pairs
   double2 *g;             // [navel] uarear * adjoint of (cc1, cc2); zero off the stepu range
   double2 *vc;            // [4][na] stress-adjoint velocity contributions: cc, ee, se, ne
   double *gstr, *gcw, *gfx, *gfy;   // [na] gradient accumulators
@@ -671,10 +673,17 @@ __global__ __launch_bounds__(256) void k_stress_adj(DevView d, AdjView a) {
   const double str_b[8] = {g0.x, ge.x, gs.x, gn.x, g0.y, gs.y, ge.y, gn.y};
   const long lp = a.lp;
   const double2 m0 = a.pc[iw], m1 = a.pc[lp + iw], m2 = a.pc[2 * lp + iw];
-  double vb[8];
-  const double gs_b = evp1d::stress_adjoint<NT>(d.s, cc.x, cc.y, ve.x, ve.y, vs.x, vs.y, vn.x, vn.y, m0.x, m0.y,
-                                            d.strength[iw], m1.x, m1.y, m2.x, m2.y, a.sigb + iw, str_b,
-                                            a.sigb + iw, d.ldsig, vb);
+  double sb[12], vb[8];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    const double2 s = in2<NT>(a.sigb + (c * d.ldsig + iw));
+    sb[2 * c] = s.x;
+    sb[2 * c + 1] = s.y;
+  }
+  const double gs_b = evp1d::stress_adjoint(a.as, cc.x, cc.y, ve.x, ve.y, vs.x, vs.y, vn.x, vn.y, m0.x, m0.y,
+                                            d.strength[iw], m1.x, m1.y, m2.x, m2.y, sb, str_b, vb);
+#pragma unroll
+  for (int c = 0; c < 6; ++c) out2<NT>(a.sigb + (c * d.ldsig + iw), make_double2(sb[2 * c], sb[2 * c + 1]));
   const long na = d.na;
   out2<NT>(a.vc + iw, make_double2(vb[0], vb[1]));
   out2<NT>(a.vc + (na + iw), make_double2(vb[2], vb[3]));
@@ -1419,6 +1428,18 @@ static const PairPersistFn kPairPersistFns[kNumPairBlocks][2] = {
     {k_pair_persistent<1024, false>, k_pair_persistent<1024, true>}};
 // the pair form runs when selected and planned
 static bool pair_form(const evp1d_handle *h) { return h->fused_depth == 2 && h->pair_ok; }
+typedef void (*PairAdjFn)(PairView, PairAdjBufs, int);
+static const PairAdjFn kPairAdjFns[kNumPairBlocks][2] = {{k_pair_adj<256, false>, k_pair_adj<256, true>},
+                                                         {k_pair_adj<512, false>, k_pair_adj<512, true>},
+                                                         {k_pair_adj<1024, false>, k_pair_adj<1024, true>}};
+// the reverse sweep's pair form: where the forward's runs and its larger
+// tables fit.  It is the faster one at every size: with the forward sweep, 60
+// subcycles, 1.28 -> 0.89 ms at 64x48, 1.82 -> 1.52 at 400x300, 5.9 -> 5.0 at
+// 900x700, 21.7 -> 19.0 at 1700x1400 (1000 subcycles of 1280x1520: 199 ->
+// 161 ms).
+static bool pair_adj_form(const evp1d_handle *h) {
+  return pair_form(h) && pair_adj_lds(h->pair_cap, h->pair_capv) <= (size_t)kPairMaxLds;
+}
 
 // Whether the pair form's launches use the cache hints (NT).  By default:
 // when all the bytes a launch touches exceed the last-level cache (256 MiB
@@ -1456,6 +1477,9 @@ static int ensure_fused_buffers(evp1d_handle *h) {
       for (const auto &kind : size)
         for (PairFn fn : kind)
           HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
+    for (const auto &size : kPairAdjFns)
+      for (PairAdjFn fn : size)
+        HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
   }
   if (!h->vel_alt) HIP_TRY(hipMalloc((void **)&h->vel_alt, (size_t)h->navel * sizeof(double2)));
   if ((!h->fused_inplace || pair_form(h)) && !h->sig_alt)
@@ -2536,6 +2560,7 @@ struct AdjointRun {
   std::vector<StateBuf> slots;
   std::vector<char> used;
   StateBuf final_state;
+  double2 *sigb2 = nullptr, *ub2 = nullptr, *g2 = nullptr;   // k_pair_adj's second buffers of sigb, ub and g
   double2 *str_save = nullptr;   // [4][navel]
   double *ut = nullptr, *vt = nullptr, *terms = nullptr;
   Schedule sched;
@@ -2849,12 +2874,47 @@ return EVP1D_OK;
     const bool hints = pair_hints(h);
     const auto stepu_adj = hints ? k_stepu_adj<true, true> : k_stepu_adj<true, false>;
     const auto stress_adj = hints ? k_stress_adj<true, true> : k_stress_adj<true, false>;
+    const bool pairs = pair_adj_form(h) && h->fused_ntiles > 0;
     for (int k = N; k >= 1; --k) {
       const DevView dk = view(k);
       if (nu > 0) hipLaunchKernelGGL(stepu_adj, dim3(blocks(nu)), dim3(256), 0, h->stream, dk, a);
-      if (nt > 0) hipLaunchKernelGGL(stress_adj, dim3(blocks(nt)), dim3(256), 0, h->stream, dk, a);
+      HIP_TRY(hipGetLastError());
+      // the stress adjoint of k .. the stepu adjoint of k - 2, two subcycles
+      // on, per launch
+      for (; pairs && k >= 3; k -= 2) RC_TRY(pair_adj(U, W, k, hints));
+      if (nt > 0) hipLaunchKernelGGL(stress_adj, dim3(blocks(nt)), dim3(256), 0, h->stream, view(k), a);
       HIP_TRY(hipGetLastError());
     }
+    return EVP1D_OK;
+  }
+  // one k_pair_adj launch after the stepu adjoint of subcycle k of the
+  // segment stored at U
+  int pair_adj(const double2 *U, const DevView &W, int k, bool hints) {
+    const long nu = W.u_end - W.u_begin;
+    PairView pv{};
+    pv.s = W.s;
+    pv.tiles = h->ptiles_dev;
+    pv.hlist = h->hlist_dev;
+    pv.xlist = h->pxlist_dev;
+    pv.elist = h->pelist_dev;
+    pv.uloc = h->puloc_dev;
+    pv.vloc = h->pvloc_dev;
+    pv.cap = h->pair_cap;
+    pv.xcd = h->tile_xcd;
+    pv.pc = a.pc;
+    pv.lp = a.lp;
+    pv.strength = W.strength;
+    pv.ls = h->ldsig;
+    pv.tnbr = h->ptnbr_dev;
+    pv.u_begin = W.u_begin;
+    const PairAdjBufs b{a.sigb, a.ub,     a.g,    sigb2, ub2,   g2,    U + (k - 1) * nu, U + (k - 2) * nu,
+                        U + (k - 3) * nu, W.vel, (int)nu, a.gstr, a.gcw, a.gfx, a.gfy, a.as};
+    hipLaunchKernelGGL(kPairAdjFns[pair_block_index(h->pair_block)][hints ? 1 : 0], dim3(h->fused_ntiles),
+                       dim3(h->pair_block), pair_adj_lds(h->pair_cap, h->pair_capv), h->stream, pv, b, h->pair_capv);
+    HIP_TRY(hipGetLastError());
+    std::swap(a.sigb, sigb2);
+    std::swap(a.ub, ub2);
+    std::swap(a.g, g2);
     return EVP1D_OK;
   }
   // reverse steps a+1 .. a+n; x_a is stored in slot sa; s further free slots
@@ -2921,10 +2981,14 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
   // from one allocation that the handle keeps (large allocations are slow),
   // cleared on every call
   {
-    const size_t parts[12] = {nV, R.sig_bytes(), nV, 4 * (size_t)h->na * sizeof(double2), nA, nA, nA, nA,
-                              nA, nA, nA, sizeof(int)};
-    size_t total = 0;
-    for (size_t b : parts) total += (b + 255) / 256 * 256;
+    const bool pairs = pair_adj_form(h);
+    const size_t parts[15] = {nV, R.sig_bytes(), nV, 4 * (size_t)h->na * sizeof(double2), nA, nA, nA, nA,
+                              nA, nA, nA, sizeof(int), pairs ? nV : 0, pairs ? nV : 0, pairs ? R.sig_bytes() : 0};
+    size_t total = 0, clear = 0;
+    for (int k = 0; k < 15; ++k) {
+      total += (parts[k] + 255) / 256 * 256;
+      if (k == 12) clear = total;   // ub2 and sigb2 are written before they are read
+    }
     if (h->adj_ws_bytes < total) {
       HIP_TRY(hipStreamSynchronize(h->stream));
       if (h->adj_ws) HIP_TRY(hipFree(h->adj_ws));
@@ -2937,7 +3001,7 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
       }
       h->adj_ws_bytes = total;
     }
-    HIP_TRY(hipMemsetAsync(h->adj_ws, 0, total, h->stream));
+    HIP_TRY(hipMemsetAsync(h->adj_ws, 0, clear, h->stream));
     char *base = static_cast<char *>(h->adj_ws);
     size_t off = 0;
     int part = 0;
@@ -2947,7 +3011,7 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
       return p;
     };
     R.a.ub = static_cast<double2 *>(carve());
-    R.a.sigb = static_cast<double *>(carve());
+    R.a.sigb = static_cast<double2 *>(carve());
     R.a.g = static_cast<double2 *>(carve());
     R.a.vc = static_cast<double2 *>(carve());
     R.a.gstr = static_cast<double *>(carve());
@@ -2958,8 +3022,12 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
     R.vt = static_cast<double *>(carve());
     R.terms = static_cast<double *>(carve());
     cnz = static_cast<int *>(carve());
+    R.g2 = static_cast<double2 *>(carve());
+    R.ub2 = static_cast<double2 *>(carve());
+    R.sigb2 = static_cast<double2 *>(carve());
   }
   R.a.cnz = cnz;
+  R.a.as = evp1d::adj_scalars(h->v.s);
   if (h->navel > h->v.t_end) {
     hipLaunchKernelGGL(k_const_flag, dim3((unsigned)((h->navel - h->v.t_end + 255) / 256)), dim3(256), 0, h->stream,
                        h->v, cnz);
