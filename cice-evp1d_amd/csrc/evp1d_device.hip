@@ -44,6 +44,7 @@
 #include "evp1d_tiles.hpp"
 #include "evp1d_point.hpp"
 #include "evp1d_cache.hpp"
+#include "evp1d_hostmem.hpp"
 #include "evp1d_pair.hpp"
 #include "evp1d_pair_adj.hpp"
 #include "evp1d_xcd.hpp"
@@ -1462,24 +1463,28 @@ static int fused_block_index(int b) {
   return -1;
 }
 
-static int ensure_fused_buffers(evp1d_handle *h) {
-  if (!h->cnz_dev) {
-    HIP_TRY(hipMalloc((void **)&h->cnz_dev, 256));
-    // tables above 64 KiB of LDS
-    for (auto &row : kFusedFns)
-      for (FusedFn fn : row)
-        HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    kFusedMaxEntries * 4 * (int)sizeof(double2)));
-    for (FusedFn fn : kFusedSplitFns)
-      HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  kFusedMaxEntries * 4 * (int)sizeof(double2)));
-    for (const auto &size : kPairFns)
-      for (const auto &kind : size)
-        for (PairFn fn : kind)
-          HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
-    for (const auto &size : kPairAdjFns)
-      for (PairAdjFn fn : size)
-        HIP_TRY(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
+// Lets fn use `bytes` of LDS where that is more than every kernel may: asked
+// for the kernels about to run, not for every variant of a new handle.
+static int allow_lds(const void *fn, size_t bytes) {
+  if (bytes > 64 * 1024)
+    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  return EVP1D_OK;
+}
+
+// traj: for a gradient's sweeps (the trajectory-storing forward forms and the
+// reverse)
+static int ensure_fused_buffers(evp1d_handle *h, bool traj = false) {
+  if (!h->cnz_dev) HIP_TRY(hipMalloc((void **)&h->cnz_dev, 256));
+  const size_t lds = (size_t)4 * h->fused_cap * sizeof(double2);
+  const int fb = fused_block_index(h->tile_block);
+  RC_TRY(allow_lds((const void *)kFusedFns[fb][h->tile_xcd ? 1 : 0], lds));
+  if (traj) RC_TRY(allow_lds((const void *)kFusedSplitFns[fb], lds));
+  if (pair_form(h)) {
+    const int b = pair_block_index(h->pair_block), hints = pair_hints(h) ? 1 : 0;
+    const size_t lds2 = pair_lds(h->pair_cap, h->pair_capv), lds3 = pair_adj_lds(h->pair_cap, h->pair_capv);
+    RC_TRY(allow_lds((const void *)kPairFns[b][h->v.nhalo > 0 ? kPairFix : kPairPlain][hints], lds2));
+    if (traj) RC_TRY(allow_lds((const void *)kPairFns[b][kPairTraj][hints], lds2));
+    if (traj && pair_adj_form(h)) RC_TRY(allow_lds((const void *)kPairAdjFns[b][hints], lds3));
   }
   if (!h->vel_alt) HIP_TRY(hipMalloc((void **)&h->vel_alt, (size_t)h->navel * sizeof(double2)));
   if ((!h->fused_inplace || pair_form(h)) && !h->sig_alt)
@@ -1975,16 +1980,18 @@ static int get_field_impl(evp1d_handle *h, int k, int32_t field, double *dst, in
   if (n == 0) return EVP1D_OK;
   if (!dst) return fail(EVP1D_EINVAL, "evp1d_get_field: dst is NULL");
   // the caller->slot map always matches the data, so no relayout is needed
-  
   const Span sp{m.a_off, m.m_na, m.g_off, n};
+  double *const direct = page_locked(dst, (size_t)n * sizeof(double));
+  double *const to = direct ? direct : h->scratch;
   if (r.kind == FK_PLAIN)
-    hipLaunchKernelGGL(k_gather_plain, dim3(blocks_for(n)), dim3(kBlock), 0, h->stream, h->scratch,
+    hipLaunchKernelGGL(k_gather_plain, dim3(blocks_for(n)), dim3(kBlock), 0, h->stream, to,
                        (const double *)r.plain, (const int32_t *)h->inv_dev, h->na, sp);
   else
-    hipLaunchKernelGGL(k_gather_comp, dim3(blocks_for(n)), dim3(kBlock), 0, h->stream, h->scratch,
+    hipLaunchKernelGGL(k_gather_comp, dim3(blocks_for(n)), dim3(kBlock), 0, h->stream, to,
                        (const double2 *)r.pair, (const int32_t *)h->inv_dev, h->na, sp, r.comp);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(dst, h->scratch, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  if (!direct)
+    HIP_TRY(hipMemcpyAsync(dst, h->scratch, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
   return EVP1D_OK;
 }
@@ -2815,14 +2822,14 @@ return EVP1D_OK;
     };
     if (pair_form(h)) {
       // two subcycles per launch, both stored (k_pair<.., TRAJ>)
-      RC_TRY(ensure_fused_buffers(h));
+      RC_TRY(ensure_fused_buffers(h, true));
       RC_TRY(issue_fused(h, N, U, false, sig_at, !lazy || final));
       sig_at = nullptr;
     } else if (h->fused_ok) {
       // fused forward sweep; two-buffer stresses ping-pong between the
       // handle's buffers and end in its own (subcycle k writes it when N - k
       // is even)
-      RC_TRY(ensure_fused_buffers(h));
+      RC_TRY(ensure_fused_buffers(h, true));
       if (!h->fused_inplace)
         HIP_TRY(hipMemcpyAsync(h->sig_alt, W.sig, (size_t)12 * h->ldsig * sizeof(double), hipMemcpyDeviceToDevice,
                                h->stream));

@@ -40,6 +40,7 @@
 
 #include "../../include/evp1d.h"
 #include "evp1d_cache.hpp"
+#include "evp1d_hostmem.hpp"
 #include "evp1d_pair.hpp"
 #include "evp1d_point.hpp"
 #include "evp1d_tiles.hpp"
@@ -1244,9 +1245,11 @@ int evp2d_get_field(evp2d_handle *h, int32_t field, double *a, int64_t n) {
   } else {
     const double2 *s = l.kind == 1 ? h->v.vel : (l.kind == 2 ? h->v.vinit : h->str[l.idx / 2]);
     const int comp = l.kind == 4 ? l.idx % 2 : l.idx;
-    hipLaunchKernelGGL(k2_get_comp, dim3(blocks2(n)), dim3(kB2), 0, h->stream, h->staging, s, (long)n, comp);
+    double *const direct = page_locked(a, bytes);
+    hipLaunchKernelGGL(k2_get_comp, dim3(blocks2(n)), dim3(kB2), 0, h->stream, direct ? direct : h->staging, s,
+                       (long)n, comp);
     HIP2(hipGetLastError());
-    HIP2(hipMemcpyAsync(a, h->staging, bytes, hipMemcpyDeviceToHost, h->stream));
+    if (!direct) HIP2(hipMemcpyAsync(a, h->staging, bytes, hipMemcpyDeviceToHost, h->stream));
   }
   HIP2(hipStreamSynchronize(h->stream));
   return EVP1D_OK;

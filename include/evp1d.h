@@ -127,7 +127,8 @@ int evp1d_get_params(const evp1d_handle *h, evp1d_params *p);
 int evp1d_get_sizes(const evp1d_handle *h, int32_t *na, int32_t *navel);
 
 /* Host -> device copies.  n must equal the field's length.  Index lists are
- * validated (1 <= idx <= navel) before upload.                              */
+ * validated (1 <= idx <= navel) before upload.  Read-back into page-locked
+ * memory (evp1d_host_alloc) is written by the device directly, without a copy. */
 int evp1d_set_field(evp1d_handle *h, int32_t field, const double *src, int32_t n);
 int evp1d_get_field(evp1d_handle *h, int32_t field, double *dst, int32_t n);
 int evp1d_set_index(evp1d_handle *h, int32_t which, const int32_t *idx, int32_t n);
