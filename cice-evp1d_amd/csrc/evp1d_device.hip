@@ -717,10 +717,10 @@ __global__ __launch_bounds__(256) void k_stress_tl(DevView d, TanView t) {
 #pragma unroll
   for (int c = 0; c < 12; ++c) sig[c] = DD(d.sig[c * d.ldsig + iw], t.dsig[c * d.ldsig + iw]);
   evp1d::StressOutT<Dual> o;
-  evp1d::stress_point<Dual>(d.s, DD(cc.x, tc.x), DD(cc.y, tc.y), DD(ve.x, te.x), DD(ve.y, te.y),
+  evp1d::stress_point(d.s, DD(cc.x, tc.x), DD(cc.y, tc.y), DD(ve.x, te.x), DD(ve.y, te.y),
                             DD(vs.x, ts.x), DD(vs.y, ts.y), DD(vn.x, tn.x), DD(vn.y, tn.y),
-                            D0(d.dxT[iw]), D0(d.dyT[iw]), DD(d.strength[iw], t.dstrength[iw]),
-                            D0(d.hte[iw]), D0(d.htn[iw]), D0(d.htem1[iw]), D0(d.htnm1[iw]), sig, o);
+                            d.dxT[iw], d.dyT[iw], DD(d.strength[iw], t.dstrength[iw]),
+                            d.hte[iw], d.htn[iw], d.htem1[iw], d.htnm1[iw], sig, o);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     d.sig[c * d.ldsig + iw] = o.sp[c].v;       t.dsig[c * d.ldsig + iw] = o.sp[c].d;
@@ -744,11 +744,11 @@ __global__ __launch_bounds__(256) void k_stepu_tl(DevView d, TanView t, int writ
   const double2 c = d.s36[js], tcs = t.ds36[js];
   const double2 e = d.s48[jsw], te = t.ds48[jsw];
   evp1d::StepuOutT<Dual> o;
-  evp1d::stepu_point<Dual>(d.s, DD(v.x, tv.x), DD(v.y, tv.y), DD(d.cw[iw], t.dcw[iw]), D0(d.aiu[iw]),
-                           D0(d.uocn[iw]), D0(d.vocn[iw]), D0(d.waterx[iw]), D0(d.watery[iw]),
-                           DD(d.forcex[iw], t.dfx[iw]), DD(d.forcey[iw], t.dfy[iw]), D0(d.umassdti[iw]),
-                           D0(d.fm[iw]), D0(d.uarear[iw]), D0(d.uvel_init[iw]), D0(d.vvel_init[iw]),
-                           D0(d.tbu[iw]), DD(a.x, ta.x), DD(b.x, tb.x), DD(c.x, tcs.x), DD(e.x, te.x),
+  evp1d::stepu_point(d.s, DD(v.x, tv.x), DD(v.y, tv.y), DD(d.cw[iw], t.dcw[iw]), d.aiu[iw],
+                           d.uocn[iw], d.vocn[iw], d.waterx[iw], d.watery[iw],
+                           DD(d.forcex[iw], t.dfx[iw]), DD(d.forcey[iw], t.dfy[iw]), d.umassdti[iw],
+                           d.fm[iw], d.uarear[iw], d.uvel_init[iw], d.vvel_init[iw],
+                           d.tbu[iw], DD(a.x, ta.x), DD(b.x, tb.x), DD(c.x, tcs.x), DD(e.x, te.x),
                            DD(a.y, ta.y), DD(c.y, tcs.y), DD(b.y, tb.y), DD(e.y, te.y), o);
   d.vel[iw] = make_double2(o.uvel.v, o.vvel.v);
   t.dvel[iw] = make_double2(o.uvel.d, o.vvel.d);
@@ -759,13 +759,151 @@ __global__ __launch_bounds__(256) void k_stepu_tl(DevView d, TanView t, int writ
   }
 }
 
-// loss and its directional derivative terms at the current state
-__global__ void k_loss_tl(DevView d, TanView t, const double *ut, const double *vt, double *terms) {
+// One tangent-linear subcycle of a tile per workgroup, on k_fused's tiles and
+// tables: values and derivatives side by side.  During the run the stresses
+// live as (value, derivative) pairs and the velocities as (u, v), (du, dv),
+// two buffers each: halo entries are evaluated again from the input buffers.
+// LDS: [8][cap], str1..8 of the tile's entries as such pairs.  Bound by the
+// latency of its two phases (at 188 VGPRs two waves per SIMD, one workgroup
+// per CU): one subcycle takes 15 us at 400x300 (212 tiles, where k_stress_tl
+// and k_stepu_tl took 12.5 + 8.3 us and a launch gap more) and 196 us at
+// 1280x1520.  The tiles stay the forward's: at 400x300 15x11, 22x16 and 31x15
+// need more than one round of workgroups and take 18, 20 and 20 us.
+struct TanFused {
+  const double2 *sg_in;   // [12][ls]
+  double2 *sg_out;
+  const double2 *v_in;    // [navel][2]
+  double2 *v_out;
+  long ls;
+  const double2 *pc;      // [kPairConst][lp]: the constant fields in pairs (k_pack_const)
+  long lp;
+  const double *dstrength, *dcw, *dfx, *dfy;   // [na] direction
+  int cap;
+  int xcd;
+};
+
+template <int B>
+__global__ __launch_bounds__(B) void k_fused_tl(DevView d, FusedView f, TanFused t, int last) {
+  using evp1d::Dual;
+  extern __shared__ double2 lds[];
+  const int cap = t.cap;
+  const evp1d::TileDesc td = f.tiles[tile_of(blockIdx.x, gridDim.x, t.xcd != 0)];
+  const int nA = td.a1 - td.a0, nB = td.b1 - td.b0, nO = nA + nB, nS = nO + td.nh, nE = nS + td.nk;
+  const bool cz = *f.cnz == 0;
+  const double2 *pc = t.pc;
+  const long lp = t.lp;
+  for (int k = threadIdx.x; k < nE; k += B) {
+    if (k < nS) {
+      const int g = k < nA ? td.a0 + k : k < nO ? td.b0 + (k - nA) : f.hlist[td.h0 + (k - nO)];
+      const int ie = d.ee[g], in = d.ne[g], is = d.se[g];
+      Dual sig[12];
+#pragma unroll
+      for (int c = 0; c < 12; ++c) {
+        const double2 v = t.sg_in[c * t.ls + g];
+        sig[c] = DD(v.x, v.y);
+      }
+      const double2 m0 = pc[g], m1 = pc[lp + g], m2 = pc[2 * lp + g];
+      const double2 cc = t.v_in[2 * (long)g], tc = t.v_in[2 * (long)g + 1];
+      const double2 ve = t.v_in[2 * (long)ie], te = t.v_in[2 * (long)ie + 1];
+      const double2 vn = t.v_in[2 * (long)in], tn = t.v_in[2 * (long)in + 1];
+      const double2 vs = t.v_in[2 * (long)is], ts = t.v_in[2 * (long)is + 1];
+      evp1d::StressOutT<Dual> o;
+      evp1d::stress_point(d.s, DD(cc.x, tc.x), DD(cc.y, tc.y), DD(ve.x, te.x), DD(ve.y, te.y), DD(vs.x, ts.x),
+                          DD(vs.y, ts.y), DD(vn.x, tn.x), DD(vn.y, tn.y), m0.x, m0.y,
+                          DD(d.strength[g], t.dstrength[g]), m1.x, m1.y, m2.x, m2.y, sig, o);
+      if (k < nO) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          t.sg_out[c * t.ls + g] = make_double2(o.sp[c].v, o.sp[c].d);
+          t.sg_out[(4 + c) * t.ls + g] = make_double2(o.sm[c].v, o.sm[c].d);
+          t.sg_out[(8 + c) * t.ls + g] = make_double2(o.s12[c].v, o.s12[c].d);
+        }
+        if (last) {   // str1..8 are observable after the run
+          d.s15[g] = make_double2(o.str[0].v, o.str[4].v);
+          d.s27[g] = make_double2(o.str[1].v, o.str[6].v);
+          d.s36[g] = make_double2(o.str[2].v, o.str[5].v);
+          d.s48[g] = make_double2(o.str[3].v, o.str[7].v);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 8; ++c) lds[c * cap + k] = make_double2(o.str[c].v, o.str[c].d);
+    } else {
+      double2 p[4] = {};   // s15, s27, s36, s48
+      if (!cz) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) p[c] = f.cstr[c * f.nk + (td.k0 + (k - nS))];
+      }
+      lds[k] = make_double2(p[0].x, 0.0);
+      lds[cap + k] = make_double2(p[1].x, 0.0);
+      lds[2 * cap + k] = make_double2(p[2].x, 0.0);
+      lds[3 * cap + k] = make_double2(p[3].x, 0.0);
+      lds[4 * cap + k] = make_double2(p[0].y, 0.0);
+      lds[5 * cap + k] = make_double2(p[2].y, 0.0);
+      lds[6 * cap + k] = make_double2(p[1].y, 0.0);
+      lds[7 * cap + k] = make_double2(p[3].y, 0.0);
+    }
+  }
+  __syncthreads();
+  const int nU = nB + (td.c1 - td.c0);
+  for (int k = threadIdx.x; k < nU; k += B) {
+    const int q = k < nB ? td.b0 + k : td.c0 + (k - nB);
+    const uint2 w = f.uloc[q - d.u_begin];
+    auto str = [&](int c, unsigned e) {
+      const double2 v = lds[c * cap + e];
+      return DD(v.x, v.y);
+    };
+    const unsigned own = w.x & 0xffffu, nw = w.x >> 16, sse = w.y & 0xffffu, sw = w.y >> 16;
+    const double2 v = t.v_in[2 * (long)q], tv = t.v_in[2 * (long)q + 1];
+    double2 c[kPairU];
+#pragma unroll
+    for (int i = 0; i < kPairU; ++i) c[i] = pc[(kPairT<false> + i) * lp + q];
+    evp1d::StepuOutT<Dual> o;
+    evp1d::stepu_point(d.s, DD(v.x, tv.x), DD(v.y, tv.y), DD(c[0].x, t.dcw[q]), c[0].y, c[1].x, c[1].y, c[2].x,
+                       c[2].y, DD(c[3].x, t.dfx[q]), DD(c[3].y, t.dfy[q]), c[4].x, c[4].y, c[5].x, c[6].x, c[6].y,
+                       c[5].y, str(0, own), str(1, nw), str(2, sse), str(3, sw), str(4, own), str(5, sse), str(6, nw),
+                       str(7, sw), o);
+    t.v_out[2 * (long)q] = make_double2(o.uvel.v, o.vvel.v);
+    t.v_out[2 * (long)q + 1] = make_double2(o.uvel.d, o.vvel.d);
+    if (last) {
+      d.strintx[q] = o.strintx.v;
+      d.strinty[q] = o.strinty.v;
+      d.cb[q] = o.Cb.v;
+    }
+  }
+}
+
+// the handle's state into k_fused_tl's buffers (both velocity buffers: the
+// slots that no stepu writes stay), and its values back
+__global__ void k_pack_tl(DevView d, double2 *sg, long ls, double2 *v0, double2 *v1) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < d.t_end) {
+#pragma unroll
+    for (int c = 0; c < 12; ++c) sg[c * ls + i] = make_double2(d.sig[c * d.ldsig + i], 0.0);
+  }
+  if (i < d.navel) {
+    const double2 v = d.vel[i], zero = make_double2(0.0, 0.0);
+    v0[2 * i] = v1[2 * i] = v;
+    v0[2 * i + 1] = v1[2 * i + 1] = zero;
+  }
+}
+__global__ void k_unpack_tl(DevView d, const double2 *sg, long ls, const double2 *v) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < d.t_end) {
+#pragma unroll
+    for (int c = 0; c < 12; ++c) d.sig[c * d.ldsig + i] = sg[c * ls + i].x;
+  }
+  if (i >= d.u_begin && i < d.u_end) d.vel[i] = v[2 * i];
+}
+
+// loss and its directional derivative terms at the current state; dvel:
+// slot q's derivative at q * stride
+__global__ void k_loss_tl(DevView d, const double2 *dvel, int stride, const double *ut, const double *vt,
+                          double *terms) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= d.na) return;
   double l = 0.0, dl = 0.0;
   if (q >= d.u_begin && q < d.u_end) {
-    const double2 v = d.vel[q], tv = t.dvel[q];
+    const double2 v = d.vel[q], tv = dvel[(long)stride * q];
     const double ex = v.x - ut[q], ey = v.y - vt[q];
     l = 0.5 * (ex * ex + ey * ey);
     dl = ex * tv.x + ey * tv.y;
@@ -1538,6 +1676,14 @@ static void fused_step(evp1d_handle *h, FusedView &f, int k) {
   f.hsig_in = h->hsig_dev + ((k - 1) % 2) * n;
   f.hsig_out = h->hsig_dev + (k % 2) * n;
 }
+
+typedef void (*TanFn)(DevView, FusedView, TanFused, int);
+static const int kTanBlocks[2] = {256, 512};
+static const TanFn kTanFns[2] = {k_fused_tl<256>, k_fused_tl<512>};
+static size_t tan_lds(const evp1d_handle *h) { return (size_t)8 * std::max(h->fused_cap, 1) * sizeof(double2); }
+static int tan_block(const evp1d_handle *h) { return h->fused_cap <= kTanBlocks[0] ? 0 : 1; }
+// tangent subcycles run fused where there are tiles and their tables fit
+static bool tan_fused(const evp1d_handle *h) { return h->fused_ok && tan_lds(h) <= (size_t)kPairMaxLds; }
 
 // nsub fused subcycles.  The state starts in the handle's buffers (X).
 // Velocities, and stresses of a two-buffer run, are copied to the second set
@@ -2970,6 +3116,34 @@ static int download_caller_order(evp1d_handle *h, double *dst, const double *src
   return EVP1D_OK;
 }
 
+// The buffers of one gradient or tangent call, at[k] of parts[k] bytes each:
+// carved from one allocation that the handle keeps (large allocations are
+// slow; evp1d_release_gradient_storage gives it back).
+static int gradient_workspace(evp1d_handle *h, const std::vector<size_t> &parts, std::vector<void *> &at,
+                              const char *name) {
+  size_t total = 0;
+  for (size_t b : parts) total += (b + 255) / 256 * 256;
+  if (h->adj_ws_bytes < total) {
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    if (h->adj_ws) HIP_TRY(hipFree(h->adj_ws));
+    h->adj_ws = nullptr;
+    h->adj_ws_bytes = 0;
+    const hipError_t e = hipMalloc(&h->adj_ws, total);
+    if (e != hipSuccess) {
+      h->adj_ws = nullptr;
+      return fail(EVP1D_ENOMEM, "%s: hipMalloc(%zu): %s", name, total, hipGetErrorString(e));
+    }
+    h->adj_ws_bytes = total;
+  }
+  char *p = static_cast<char *>(h->adj_ws);
+  at.clear();
+  for (size_t b : parts) {
+    at.push_back(p);
+    p += (b + 255) / 256 * 256;
+  }
+  return EVP1D_OK;
+}
+
 int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double *u_target, const double *v_target,
                       double *loss, double *g_strength, double *g_cdn_ocn, double *g_forcex, double *g_forcey) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_adjoint_run: NULL handle");
@@ -2984,54 +3158,32 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
   R.nsub = nsub;
   const size_t nA = (size_t)h->na * sizeof(double), nV = (size_t)h->navel * sizeof(double2);
   int *cnz = nullptr;
-  // adjoint state, gradient accumulators, targets and loss terms: carved
-  // from one allocation that the handle keeps (large allocations are slow),
-  // cleared on every call
+  // adjoint state, gradient accumulators, targets and loss terms
   {
     const bool pairs = pair_adj_form(h);
-    const size_t parts[15] = {nV, R.sig_bytes(), nV, 4 * (size_t)h->na * sizeof(double2), nA, nA, nA, nA,
-                              nA, nA, nA, sizeof(int), pairs ? nV : 0, pairs ? nV : 0, pairs ? R.sig_bytes() : 0};
-    size_t total = 0, clear = 0;
-    for (int k = 0; k < 15; ++k) {
-      total += (parts[k] + 255) / 256 * 256;
-      if (k == 12) clear = total;   // ub2 and sigb2 are written before they are read
-    }
-    if (h->adj_ws_bytes < total) {
-      HIP_TRY(hipStreamSynchronize(h->stream));
-      if (h->adj_ws) HIP_TRY(hipFree(h->adj_ws));
-      h->adj_ws = nullptr;
-      h->adj_ws_bytes = 0;
-      const hipError_t e = hipMalloc(&h->adj_ws, total);
-      if (e != hipSuccess) {
-        h->adj_ws = nullptr;
-        return fail(EVP1D_ENOMEM, "evp1d_adjoint_run: hipMalloc(%zu): %s", total, hipGetErrorString(e));
-      }
-      h->adj_ws_bytes = total;
-    }
-    HIP_TRY(hipMemsetAsync(h->adj_ws, 0, clear, h->stream));
-    char *base = static_cast<char *>(h->adj_ws);
-    size_t off = 0;
-    int part = 0;
-    auto carve = [&]() {
-      void *p = base + off;
-      off += (parts[part++] + 255) / 256 * 256;
-      return p;
-    };
-    R.a.ub = static_cast<double2 *>(carve());
-    R.a.sigb = static_cast<double2 *>(carve());
-    R.a.g = static_cast<double2 *>(carve());
-    R.a.vc = static_cast<double2 *>(carve());
-    R.a.gstr = static_cast<double *>(carve());
-    R.a.gcw = static_cast<double *>(carve());
-    R.a.gfx = static_cast<double *>(carve());
-    R.a.gfy = static_cast<double *>(carve());
-    R.ut = static_cast<double *>(carve());
-    R.vt = static_cast<double *>(carve());
-    R.terms = static_cast<double *>(carve());
-    cnz = static_cast<int *>(carve());
-    R.g2 = static_cast<double2 *>(carve());
-    R.ub2 = static_cast<double2 *>(carve());
-    R.sigb2 = static_cast<double2 *>(carve());
+    const std::vector<size_t> parts = {nV, R.sig_bytes(), nV, 4 * (size_t)h->na * sizeof(double2), nA, nA, nA, nA,
+                                       nA, nA, nA, sizeof(int), pairs ? nV : 0, pairs ? nV : 0,
+                                       pairs ? R.sig_bytes() : 0};
+    std::vector<void *> at;
+    RC_TRY(gradient_workspace(h, parts, at, "evp1d_adjoint_run"));
+    // all but ub2 and sigb2, which are written before they are read
+    HIP_TRY(hipMemsetAsync(h->adj_ws, 0, (size_t)(static_cast<char *>(at[13]) - static_cast<char *>(h->adj_ws)),
+                           h->stream));
+    R.a.ub = static_cast<double2 *>(at[0]);
+    R.a.sigb = static_cast<double2 *>(at[1]);
+    R.a.g = static_cast<double2 *>(at[2]);
+    R.a.vc = static_cast<double2 *>(at[3]);
+    R.a.gstr = static_cast<double *>(at[4]);
+    R.a.gcw = static_cast<double *>(at[5]);
+    R.a.gfx = static_cast<double *>(at[6]);
+    R.a.gfy = static_cast<double *>(at[7]);
+    R.ut = static_cast<double *>(at[8]);
+    R.vt = static_cast<double *>(at[9]);
+    R.terms = static_cast<double *>(at[10]);
+    cnz = static_cast<int *>(at[11]);
+    R.g2 = static_cast<double2 *>(at[12]);
+    R.ub2 = static_cast<double2 *>(at[13]);
+    R.sigb2 = static_cast<double2 *>(at[14]);
   }
   R.a.cnz = cnz;
   R.a.as = evp1d::adj_scalars(h->v.s);
@@ -3144,56 +3296,76 @@ int evp1d_tangent_run(evp1d_handle *h, int32_t nsub, const double *d_strength, c
   if (h->v.nhalo > 0) return fail(EVP1D_ESTATE, "evp1d_tangent_run: a ghost copy list is set");
   RC_TRY(ensure(h));
   const size_t nA = (size_t)h->na * sizeof(double), nV = (size_t)h->navel * sizeof(double2);
-  std::vector<void *> mem;
-  struct Free {
-    std::vector<void *> &m;
-    hipStream_t s;
-    ~Free() {
-      (void)hipStreamSynchronize(s);
-      for (void *p : m) (void)hipFree(p);
-    }
-  } guard{mem, h->stream};
-  auto A = [&](void **p, size_t bytes) -> int {
-    const hipError_t e = hipMalloc(p, bytes ? bytes : 256);
-    if (e != hipSuccess) return fail(EVP1D_ENOMEM, "evp1d_tangent_run: hipMalloc(%zu)", bytes);
-    mem.push_back(*p);
-    HIP_TRY(hipMemsetAsync(*p, 0, bytes ? bytes : 256, h->stream));
-    return EVP1D_OK;
-  };
+  const bool fused = tan_fused(h) && nsub > 0 && h->fused_ntiles > 0;
+  const size_t nS = (size_t)12 * h->ldsig * sizeof(double);
+  // direction, targets, loss terms, then the tangent state: the unfused
+  // form's derivatives, or the fused form's two buffers of both
+  std::vector<size_t> parts = {nA, nA, nA, nA, nA, nA, 2 * nA};
+  for (size_t b : fused ? std::vector<size_t>{2 * nS, 2 * nS, 2 * nV, 2 * nV} : std::vector<size_t>{nS, nV, nV, nV, nV, nV})
+    parts.push_back(b);
+  std::vector<void *> at;
+  RC_TRY(gradient_workspace(h, parts, at, "evp1d_tangent_run"));
   TanView t{};
-  double *dir[4] = {nullptr, nullptr, nullptr, nullptr}, *ut = nullptr, *vt = nullptr, *terms = nullptr;
-  RC_TRY(A((void **)&t.dsig, (size_t)12 * h->ldsig * sizeof(double)));
-  RC_TRY(A((void **)&t.dvel, nV));
-  RC_TRY(A((void **)&t.ds15, nV));
-  RC_TRY(A((void **)&t.ds27, nV));
-  RC_TRY(A((void **)&t.ds36, nV));
-  RC_TRY(A((void **)&t.ds48, nV));
+  double *dir[4], *ut = (double *)at[4], *vt = (double *)at[5], *terms = (double *)at[6];
   const double *src[4] = {d_strength, d_cdn_ocn, d_forcex, d_forcey};
   for (int k = 0; k < 4; ++k) {
-    RC_TRY(A((void **)&dir[k], nA));
+    dir[k] = (double *)at[k];
     if (src[k]) RC_TRY(upload_caller_order(h, dir[k], src[k]));
+    else HIP_TRY(hipMemsetAsync(dir[k], 0, nA, h->stream));
   }
   t.dstrength = dir[0];
   t.dcw = dir[1];
   t.dfx = dir[2];
   t.dfy = dir[3];
-  RC_TRY(A((void **)&ut, nA));
-  RC_TRY(A((void **)&vt, nA));
-  RC_TRY(A((void **)&terms, 2 * nA));
   RC_TRY(upload_caller_order(h, ut, u_target));
   RC_TRY(upload_caller_order(h, vt, v_target));
   const DevView &d = h->v;
-  for (int k = 0; k < nsub; ++k) {
-    if (d.t_end > 0) hipLaunchKernelGGL(k_stress_tl, dim3((d.t_end + 255) / 256), dim3(256), 0, h->stream, d, t);
-    if (d.u_end > d.u_begin)
-      hipLaunchKernelGGL(k_stepu_tl, dim3((d.u_end - d.u_begin + 255) / 256), dim3(256), 0, h->stream, d, t,
-                         k == nsub - 1 ? 1 : 0);
+  const double2 *dvel = nullptr;
+  if (fused) {
+    RC_TRY(ensure_fused_buffers(h));
+    double2 *sg[2] = {(double2 *)at[7], (double2 *)at[8]}, *v[2] = {(double2 *)at[9], (double2 *)at[10]};
+    if (!h->pconst) HIP_TRY(hipMalloc((void **)&h->pconst, (size_t)kPairConst * std::max(h->na, 1) * sizeof(double2)));
+    hipLaunchKernelGGL(k_pack_const, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, d, h->pconst, (long)h->na);
     HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_pack_tl, dim3(blocks_for(h->navel)), dim3(kBlock), 0, h->stream, d, sg[0], h->ldsig, v[0], v[1]);
+    HIP_TRY(hipGetLastError());
+    FusedView f;
+    RC_TRY(fused_prologue(h, d, f, false));
+    const int b = tan_block(h);
+    const TanFn fn = kTanFns[b];
+    const size_t lds = tan_lds(h);
+    RC_TRY(allow_lds((const void *)fn, lds));
+    for (int k = 0; k < nsub; ++k) {
+      const TanFused tf{sg[k % 2], sg[1 - k % 2], v[k % 2], v[1 - k % 2], h->ldsig, h->pconst, h->na,
+                        t.dstrength, t.dcw, t.dfx, t.dfy, std::max(h->fused_cap, 1), h->tile_xcd};
+      hipLaunchKernelGGL(fn, dim3(h->fused_ntiles), dim3(kTanBlocks[b]), lds, h->stream, d, f, tf, k == nsub - 1 ? 1 : 0);
+      HIP_TRY(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_unpack_tl, dim3(blocks_for(h->navel)), dim3(kBlock), 0, h->stream, d,
+                       (const double2 *)sg[nsub % 2], h->ldsig, (const double2 *)v[nsub % 2]);
+    HIP_TRY(hipGetLastError());
+    dvel = v[nsub % 2] + 1;
+  } else {
+    t.dsig = (double *)at[7];
+    t.dvel = (double2 *)at[8];
+    t.ds15 = (double2 *)at[9];
+    t.ds27 = (double2 *)at[10];
+    t.ds36 = (double2 *)at[11];
+    t.ds48 = (double2 *)at[12];
+    HIP_TRY(hipMemsetAsync(at[7], 0, (size_t)(static_cast<char *>(at[12]) - static_cast<char *>(at[7])) + nV, h->stream));
+    for (int k = 0; k < nsub; ++k) {
+      if (d.t_end > 0) hipLaunchKernelGGL(k_stress_tl, dim3((d.t_end + 255) / 256), dim3(256), 0, h->stream, d, t);
+      if (d.u_end > d.u_begin)
+        hipLaunchKernelGGL(k_stepu_tl, dim3((d.u_end - d.u_begin + 255) / 256), dim3(256), 0, h->stream, d, t,
+                           k == nsub - 1 ? 1 : 0);
+      HIP_TRY(hipGetLastError());
+    }
+    dvel = t.dvel;
   }
   double l = 0.0, dl = 0.0;
   if (h->na > 0) {
-    hipLaunchKernelGGL(k_loss_tl, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, d, t, (const double *)ut,
-                       (const double *)vt, terms);
+    hipLaunchKernelGGL(k_loss_tl, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, d, dvel, fused ? 2 : 1,
+                       (const double *)ut, (const double *)vt, terms);
     HIP_TRY(hipGetLastError());
     std::vector<double> buf(2 * (size_t)h->na);
     HIP_TRY(hipMemcpyAsync(buf.data(), terms, 2 * nA, hipMemcpyDeviceToHost, h->stream));

@@ -63,6 +63,7 @@ __host__ __device__ inline Dual operator/(double a, Dual b) {
   return {q, -q * b.d / b.v};
 }
 __host__ __device__ inline bool operator>(Dual a, Dual b) { return a.v > b.v; }
+__host__ __device__ inline bool operator>(Dual a, double b) { return a.v > b; }
 __host__ __device__ inline Dual sqrt(Dual a) {
   const double r = ::sqrt(a.v);
   return {r, r > 0.0 ? a.d / (2.0 * r) : 0.0};
@@ -90,15 +91,15 @@ using StressOut = StressOutT<double>;
 // strength's sign, so +0 * q is the zero with strength's sign.  A NaN Delta
 // (or any other case) takes the division.  The tangent-linear type always
 // takes the division.
-template <class R>
-__host__ __device__ inline bool capping_fast(const Scalars &, R, R) {
+template <class R, class M>
+__host__ __device__ inline bool capping_fast(const Scalars &, R, M) {
   return false;
 }
 __host__ __device__ inline bool capping_fast(const Scalars &s, double strength, double DminArea) {
   return s.capping == c1 && DminArea > 0.0 && fabs(strength) <= fmin(__DBL_MAX__, DminArea * 0x1p1000);
 }
-template <class R>
-__host__ __device__ inline R capping_term(const Scalars &s, bool, R strength, R DminArea, R Delta) {
+template <class R, class M>
+__host__ __device__ inline R capping_term(const Scalars &s, bool, R strength, M DminArea, R Delta) {
   return (c1 - s.capping) * (strength / (Delta + DminArea));
 }
 __host__ __device__ inline double capping_term(const Scalars &s, bool fast, double strength, double DminArea,
@@ -108,11 +109,11 @@ __host__ __device__ inline double capping_term(const Scalars &s, bool fast, doub
 }
 
 // visc_replpress (bench_v2b.F90:415-437); fast: capping_fast(s, strength, DminArea)
-template <class R>
-__host__ __device__ inline void visc_replpress(const Scalars &s, R strength, R DminArea,
+template <class R, class M>
+__host__ __device__ inline void visc_replpress(const Scalars &s, R strength, M DminArea,
                                                R Delta, R &zetax2, R &etax2,
                                                R &rep_prs, bool fast = false) {
-  const R dmax = (Delta > DminArea) ? Delta : DminArea;   // max(Delta, DminArea)
+  const R dmax = (Delta > DminArea) ? Delta : R{DminArea};   // max(Delta, DminArea)
   const R tmpcalc = s.capping * (strength / dmax) + capping_term(s, fast, strength, DminArea, Delta);
   zetax2 = (c1 + s.Ktens) * tmpcalc;
   rep_prs = (c1 - s.Ktens) * tmpcalc * Delta;
@@ -125,13 +126,14 @@ __host__ __device__ inline void visc_replpress(const Scalars &s, R strength, R D
 // kernel computes them first, stress_point below).  sig_in: the 12 stresses
 // at the start of the subcycle in the order stressp_1..4, stressm_1..4,
 // stress12_1..4.  Velocities: cc = (i,j), ee = (i-1,j), se = (i,j-1),
-// ne = (i-1,j-1).
-template <class R>
+// ne = (i-1,j-1).  M: the type of the values that are no function of the
+// state or of a derivative's direction, double or (with derivative 0) R.
+template <class R, class M>
 __host__ __device__ inline void stress_core(const Scalars &s,
     R uvel_cc, R vvel_cc, R uvel_ee, R vvel_ee,
     R uvel_se, R vvel_se, R uvel_ne, R vvel_ne,
-    R dxT, R dyT, R strength,
-    R cxp, R cyp, R cxm, R cym, R DminTarea, R dxhy, R dyhx,
+    M dxT, M dyT, R strength,
+    M cxp, M cyp, M cxm, M cym, M DminTarea, M dxhy, M dyhx,
     const R *sig_in, StressOutT<R> &o) {
 
   // strain rates (bench_v2b.F90:363-390)
@@ -250,21 +252,21 @@ __host__ __device__ inline void stress_core(const Scalars &s,
 
 // Stress at one point of the 1D list (bench_v2b.F90:125-311): the metric
 // terms from HTE, HTN and their i-1 / j-1 neighbours (139-147), then the core.
-template <class R>
+template <class R, class M>
 __host__ __device__ inline void stress_point(const Scalars &s,
     R uvel_cc, R vvel_cc, R uvel_ee, R vvel_ee,
     R uvel_se, R vvel_se, R uvel_ne, R vvel_ne,
-    R dxT, R dyT, R strength,
-    R hte, R htn, R htem1, R htnm1,
+    M dxT, M dyT, R strength,
+    M hte, M htn, M htem1, M htnm1,
     const R *sig_in, StressOutT<R> &o) {
-  const R cxp = c1p5 * htn - p5 * htnm1;
-  const R cyp = c1p5 * hte - p5 * htem1;
-  const R cxm = -(c1p5 * htnm1 - p5 * htn);
-  const R cym = -(c1p5 * htem1 - p5 * hte);
-  const R tmparea = dxT * dyT;
-  const R DminTarea = s.deltaminEVP * tmparea;
-  const R dxhy = p5 * (hte - htem1);
-  const R dyhx = p5 * (htn - htnm1);
+  const M cxp = c1p5 * htn - p5 * htnm1;
+  const M cyp = c1p5 * hte - p5 * htem1;
+  const M cxm = -(c1p5 * htnm1 - p5 * htn);
+  const M cym = -(c1p5 * htem1 - p5 * hte);
+  const M tmparea = dxT * dyT;
+  const M DminTarea = s.deltaminEVP * tmparea;
+  const M dxhy = p5 * (hte - htem1);
+  const M dyhx = p5 * (htn - htnm1);
   stress_core(s, uvel_cc, vvel_cc, uvel_ee, vvel_ee, uvel_se, vvel_se, uvel_ne, vvel_ne, dxT, dyT, strength,
               cxp, cyp, cxm, cym, DminTarea, dxhy, dyhx, sig_in, o);
 }
@@ -277,11 +279,11 @@ using StepuOut = StepuOutT<double>;
 
 // stepu for one U point (bench_v2b.F90:509-544).  str1/str5 are the point's
 // own values; str2/str7 come from nw, str3/str6 from sse, str4/str8 from sw.
-template <class R>
+template <class R, class M>
 __host__ __device__ inline void stepu_point(const Scalars &s,
-    R uold, R vold, R Cw, R aiX, R uocn, R vocn,
-    R waterx, R watery, R forcex, R forcey, R umassdti,
-    R fm, R uarear, R uvel_init, R vvel_init, R Tbu,
+    R uold, R vold, R Cw, M aiX, M uocn, M vocn,
+    M waterx, M watery, R forcex, R forcey, M umassdti,
+    M fm, M uarear, M uvel_init, M vvel_init, M Tbu,
     R str1, R str2_nw, R str3_sse, R str4_sw,
     R str5, R str6_sse, R str7_nw, R str8_sw, StepuOutT<R> &o) {
   const R du = uocn - uold;

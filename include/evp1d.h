@@ -370,9 +370,9 @@ int evp1d_loss_noalloc(evp1d_handle *h, const double *u_target, const double *v_
  * the same bit for bit for every seg and nsnap.                            */
 int evp1d_set_adjoint_segment(evp1d_handle *h, int32_t seg);
 int evp1d_get_adjoint_segment(evp1d_handle *h, int32_t *seg);
-/* Device memory that gradient calls keep with the handle (no counterpart in
- * the reference): the stored trajectory, the stored states of checkpointed
- * calls and the adjoint work arrays.  evp1d_get_gradient_storage reports the
+/* Device memory that gradient and tangent calls keep with the handle (no
+ * counterpart in the reference): the stored trajectory, the stored states of
+ * checkpointed calls and the work arrays of both.  evp1d_get_gradient_storage reports the
  * bytes held; evp1d_release_gradient_storage gives them back (the next
  * gradient call allocates again), for callers that need the memory for other
  * work without destroying the handle.                                       */
