@@ -503,6 +503,16 @@ __global__ void k_fill_const(DevView d, const int32_t *klist, double2 *cstr, lon
 
 constexpr int kFusedMaxEntries = 2560;   // 160 KiB of LDS per workgroup (gfx950)
 constexpr int kFusedMinSub = 4;          // evp1d_run in AUTO mode: fused from this many subcycles
+// evp1d_run in AUTO mode plans tiles for a new set of skip flags at its first
+// run of this many subcycles, or at the second run; a shorter first run (a
+// model step whose ice mask is new) goes over the points in class order, one
+// kernel for stress and one for stepu.  Planning takes 32 ms longer than the
+// class order at 1280x1520 and the tiles then save 57 us a subcycle (62
+// against 119): even at 560 subcycles, and at 550 for 2560x3040 (150 ms, 270
+// us), 500 for 64x48 (1.3 ms, 2.5 us), 1200 for 400x300 and 700x500 (5.5 and
+// 10 ms, 4.6 and 7.8 us).  A step of 240 subcycles at 1280x1520 with new
+// flags, fields in and out of 2D arrays: 65 -> 45 ms.
+constexpr int kPlanSub = 500;
 // launch configurations the autotuner chooses from
 constexpr int kNumBlocks = 5;
 constexpr int kBlocks[kNumBlocks] = {64, 128, 256, 512, 1024};
@@ -1031,6 +1041,8 @@ struct evp1d_handle {
   std::vector<int32_t> perm, inv;  // slot -> caller position, and inverse
   std::vector<int32_t> halo_dst_host, halo_src_host;   // caller order, -1 = fill
   bool layout_dirty = false;       // skip flags changed since the last relayout
+  bool layout_tiled = false;       // the slot order was made with tiles (or none fit), not by class alone
+  long layout_runs = 0;            // evp1d_run calls since the slot order was first made for these flags
   bool idx_dirty = false;          // slot-space lists need re-upload
   int mode = EVP1D_MODE_AUTO;
   LaunchCfg cfg_stress, cfg_stepu;
@@ -1369,27 +1381,28 @@ static int install_pairs(evp1d_handle *h, const evp1d::TilePlan &plan, const int
 
 // Rebuild the slot order (class, then fused tile, then caller position) from
 // the skip flags and the neighbour lists, and move every resident array into
-// it.  Without a complete set of lists the order is class, caller position.
-static int relayout_impl(evp1d_handle *h);
-static int relayout(evp1d_handle *h) {
-  return evp1d::no_throw("slot layout", [h] { return relayout_impl(h); });
+// it.  Without a complete set of lists, or without tiles asked for, the order
+// is class, caller position.
+static int relayout_impl(evp1d_handle *h, bool tiles);
+static int relayout(evp1d_handle *h, bool tiles) {
+  return evp1d::no_throw("slot layout", [h, tiles] { return relayout_impl(h, tiles); });
 }
-static int relayout_impl(evp1d_handle *h) {
+static int relayout_impl(evp1d_handle *h, bool tiles) {
   const int na = h->na;
   const int32_t *idx[6];
-  bool all = na > 0;
+  bool all = na > 0 && tiles;
   for (int k = 0; k < 6; ++k) {
     all = all && h->idx_set[k] && h->idx_host[k].size() == (size_t)na;
     idx[k] = all ? h->idx_host[k].data() : nullptr;
   }
   // the tile of each point depends on the lists and the tile size only: it
   // is kept while only skip flags change (a new model step's ice masks)
-  if (!h->coords_ok) {
+  if (tiles && !h->coords_ok) {
     h->coords = evp1d::grid_coords(na, h->navel, all ? idx : nullptr);
     h->coords_ok = true;
     h->tile_cache_ok = false;
   }
-  if (h->tiling_auto && !h->tile_cache_ok) {
+  if (tiles && h->tiling_auto && !h->tile_cache_ok) {
     if (h->fused_depth == 2) {
       h->tile_cache = evp1d::pair_tiles(h->coords, h->tile_order, &h->tile_block);
     } else {
@@ -1411,8 +1424,8 @@ static int relayout_impl(evp1d_handle *h) {
   if (h->tiling_auto && h->fused_depth == 2 && all &&
       evp1d::pair_uncrowd(h->coords, na, idx, h->skip_host.data(), h->tile_cache))
     h->tile_h = h->tile_cache.tile_h;
-  if (!h->tile_cache_ok || h->tile_cache.tile_w != h->tile_w || h->tile_cache.tile_h != h->tile_h ||
-      h->tile_cache.order != h->tile_order) {
+  if (tiles && (!h->tile_cache_ok || h->tile_cache.tile_w != h->tile_w || h->tile_cache.tile_h != h->tile_h ||
+                h->tile_cache.order != h->tile_order)) {
     h->tile_cache = evp1d::tile_ids(h->coords, h->tile_w, h->tile_h, h->tile_order);
     h->tile_cache_ok = true;
   }
@@ -1450,11 +1463,13 @@ static int relayout_impl(evp1d_handle *h) {
     h->perm_dev_dirty = true;
   }
   RC_TRY(install_tiling(h, plan));
+  if (!tiles) h->fused_why = "no tiles are planned for a first short run";
   RC_TRY(install_pairs(h, plan, all ? idx : nullptr));
   h->v.t_end = plan.cnt[0] + plan.cnt[1];
   h->v.u_begin = plan.cnt[0];
   h->v.u_end = plan.cnt[0] + plan.cnt[1] + plan.cnt[2];
   h->layout_dirty = false;
+  h->layout_tiled = tiles;
   h->idx_dirty = true;
   h->graph_dirty = true;
   return EVP1D_OK;
@@ -1462,9 +1477,11 @@ static int relayout_impl(evp1d_handle *h) {
 
 static inline int32_t slot_of(const evp1d_handle *h, int32_t q) { return q < h->na ? h->inv[(size_t)q] : q; }
 
-// bring the device copy of layout, lists and halo up to date
-static int ensure(evp1d_handle *h) {
-  if (h->layout_dirty) RC_TRY(relayout(h));
+// bring the device copy of layout, lists and halo up to date; tiles: and the
+// fused forms' tiles (else an order that is up to date stays, tiled or not)
+static int ensure(evp1d_handle *h, bool tiles = true) {
+  if (h->layout_dirty) h->layout_runs = 0;
+  if (h->layout_dirty || (tiles && !h->layout_tiled)) RC_TRY(relayout(h, tiles));
   if (!h->idx_dirty) return EVP1D_OK;
   const int na = h->na;
   if (na > 0 && h->perm_dev_dirty) {
@@ -2179,14 +2196,14 @@ static int set_skip_impl(evp1d_handle *h, int k, int32_t which, const int32_t *f
   if (n != m.m_na) return fail(EVP1D_EINVAL, "evp1d_set_skip: length %d != na %d", n, m.m_na);
   if (n > 0 && !flags) return fail(EVP1D_EINVAL, "evp1d_set_skip: flags is NULL");
   const uint8_t bit = (uint8_t)(1u << which);
-  bool changed = false;
+  uint8_t diff = 0;
+  uint8_t *__restrict__ const skip = h->skip_host.data() + m.a_off;
   for (int i = 0; i < n; ++i) {
-    uint8_t &b = h->skip_host[(size_t)m.a_off + i];
-    const uint8_t nb = (uint8_t)(flags[i] ? (b | bit) : (b & ~bit));
-    changed |= nb != b;
-    b = nb;
+    const uint8_t nb = (uint8_t)((skip[i] & ~bit) | (flags[i] ? bit : 0));
+    diff |= (uint8_t)(nb ^ skip[i]);
+    skip[i] = nb;
   }
-  if (changed) h->layout_dirty = true;
+  if (diff) h->layout_dirty = true;
   return EVP1D_OK;
 }
 
@@ -2254,20 +2271,20 @@ int evp1d_set_halo(evp1d_handle *h, int32_t n, const int32_t *dst, const int32_t
 int evp1d_stress(evp1d_handle *h) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_stress: NULL handle");
   if (!ready(h)) return fail(EVP1D_ESTATE, "evp1d_stress: neighbour lists not set");
-  RC_TRY(ensure(h));
+  RC_TRY(ensure(h, false));
   return launch_stress(h);
 }
 
 int evp1d_stepu(evp1d_handle *h) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_stepu: NULL handle");
   if (!ready(h)) return fail(EVP1D_ESTATE, "evp1d_stepu: neighbour lists not set");
-  RC_TRY(ensure(h));
+  RC_TRY(ensure(h, false));
   return launch_stepu(h, true);
 }
 
 int evp1d_halo(evp1d_handle *h) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_halo: NULL handle");
-  RC_TRY(ensure(h));
+  RC_TRY(ensure(h, false));
   return launch_halo(h);
 }
 
@@ -2288,8 +2305,10 @@ int evp1d_run(evp1d_handle *h, int32_t nsub) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_run: NULL handle");
   if (nsub < 0) return fail(EVP1D_EINVAL, "evp1d_run: nsub=%d < 0", nsub);
   if (!ready(h)) return fail(EVP1D_ESTATE, "evp1d_run: neighbour lists not set");
-  RC_TRY(ensure(h));
+  const bool first = h->layout_dirty || h->layout_runs == 0;
+  RC_TRY(ensure(h, h->mode != EVP1D_MODE_AUTO || !first || nsub >= kPlanSub));
   if (nsub == 0 || h->na == 0) return EVP1D_OK;
+  ++h->layout_runs;
   switch (h->mode) {
     case EVP1D_MODE_LAUNCH: return issue_subcycles(h, nsub);
     case EVP1D_MODE_PERSISTENT: return run_persistent(h, nsub);
@@ -2299,6 +2318,8 @@ int evp1d_run(evp1d_handle *h, int32_t nsub) {
     case EVP1D_MODE_GRAPH: return run_graph(h, nsub, false);
     case EVP1D_MODE_AUTO:
     default:
+      // these flags' first, short run: a captured graph would serve it only
+      if (!h->layout_tiled) return issue_subcycles(h, nsub);
       // the fused form copies the state once per run (two buffers), which
       // only pays off over several subcycles
       return run_graph(h, nsub, h->fused_ok && nsub >= kFusedMinSub);
@@ -2309,7 +2330,7 @@ int evp1d_run_individual(evp1d_handle *h, int32_t which, int32_t nsub) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_run_individual: NULL handle");
   if (!ready(h)) return fail(EVP1D_ESTATE, "evp1d_run_individual: neighbour lists not set");
   if (which < 0 || which > 2) return fail(EVP1D_EINVAL, "evp1d_run_individual: which=%d", which);
-  RC_TRY(ensure(h));
+  RC_TRY(ensure(h, which == 2));
   if (which == 2) {
     if (!h->fused_ok)
       return fail(EVP1D_ESTATE, "evp1d_run_individual: fused form unavailable (%s)", h->fused_why.c_str());
@@ -3383,7 +3404,7 @@ int evp1d_tangent_run(evp1d_handle *h, int32_t nsub, const double *d_strength, c
 int evp1d_loss(evp1d_handle *h, const double *u_target, const double *v_target, double *loss) {
   if (!h || !loss) return fail(EVP1D_EINVAL, "evp1d_loss: NULL argument");
   if (h->na > 0 && (!u_target || !v_target)) return fail(EVP1D_EINVAL, "evp1d_loss: NULL target");
-  RC_TRY(ensure(h));
+  RC_TRY(ensure(h, false));
   *loss = 0.0;
   if (h->na == 0) return EVP1D_OK;
   double *buf = nullptr;

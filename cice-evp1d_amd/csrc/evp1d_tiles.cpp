@@ -4,6 +4,7 @@
 #include "evp1d_tiles.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
@@ -25,13 +26,6 @@ constexpr int kDx[6] = {-1, -1, 0, 1, 1, 0};
 constexpr int kDy[6] = {0, -1, -1, 0, 1, 1};
 
 // class order with caller order inside each class (the untiled layout)
-void class_order(int na, const uint8_t *skip, TilePlan &p) {
-  std::fill(p.cnt, p.cnt + 4, 0);
-  for (int q = 0; q < na; ++q) ++p.cnt[point_class(skip[q])];
-  int start[4] = {0, p.cnt[0], p.cnt[0] + p.cnt[1], p.cnt[0] + p.cnt[1] + p.cnt[2]};
-  p.perm.assign((size_t)na, 0);
-  for (int q = 0; q < na; ++q) p.perm[(size_t)start[point_class(skip[q])]++] = q;
-}
 
 // Grid coordinates of every point from the neighbour lists, one frame per
 // connected component, components placed side by side.  Returns false when
@@ -274,6 +268,34 @@ void par_items(int n, F f) {
   run_workers(T, [&](int w) {
     for (int i = next.fetch_add(8); i < n; i = next.fetch_add(8))
       for (int j = i; j < std::min(n, i + 8); ++j) f(j, w);
+  });
+}
+
+// the order by class, then caller position: per-chunk counts, then each chunk
+// places its points
+void class_order(int na, const uint8_t *skip, TilePlan &p) {
+  const int T = std::max(1, std::min(plan_threads(), na / (1 << 15)));
+  auto lo = [&](int w) { return (int64_t)na * w / T; };
+  std::vector<std::array<int32_t, 4>> pos((size_t)T);
+  run_workers(T, [&](int w) {
+    std::array<int32_t, 4> n{};
+    for (int64_t q = lo(w); q < lo(w + 1); ++q) ++n[(size_t)point_class(skip[q])];
+    pos[(size_t)w] = n;
+  });
+  int32_t at = 0;
+  for (int c = 0; c < 4; ++c) {
+    const int32_t first = at;
+    for (int w = 0; w < T; ++w) {
+      const int32_t n = pos[(size_t)w][(size_t)c];
+      pos[(size_t)w][(size_t)c] = at;
+      at += n;
+    }
+    p.cnt[c] = at - first;
+  }
+  p.perm.assign((size_t)na, 0);
+  run_workers(T, [&](int w) {
+    std::array<int32_t, 4> n = pos[(size_t)w];
+    for (int64_t q = lo(w); q < lo(w + 1); ++q) p.perm[(size_t)n[(size_t)point_class(skip[q])]++] = (int32_t)q;
   });
 }
 

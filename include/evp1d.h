@@ -108,7 +108,9 @@ enum evp1d_mode {
                                  (evp1d_set_fused_depth 2, planned) the pair form's tiles with one grid
                                  barrier per two subcycles, else stress and stepu over all points with a
                                  grid barrier between phases (hipLaunchCooperativeKernel) */
-  EVP1D_MODE_AUTO = 3,        /* library default: FUSED when the lists tile and nsub >= 4, else GRAPH */
+  EVP1D_MODE_AUTO = 3,        /* library default: FUSED when the lists tile and nsub >= 4, else GRAPH;
+                                 LAUNCH for the first run with new skip flags if it is shorter than
+                                 500 subcycles (tiles are planned at the second run, or for a long one) */
   EVP1D_MODE_FUSED = 4        /* one launch per subcycle: stress and stepu per tile of points, str1..8
                                  kept on chip (hipGraph); needs lists that describe a grid */
 };
