@@ -350,16 +350,24 @@ constexpr int kCus = 256;   // compute units of an MI355X
 }
 
 // The first rung that gives at most `most` tiles.  A tile's time is its chain
-// of four phases, whatever runs beside it, until the CUs are full.  So with
-// at most one tile per CU the smallest tile is the fastest: in 15x11 every
-// phase is one pass of 256 threads (18x14 cells at level 1), in 22x16 one of
-// 512.  Measured on 1D lists, 31x19 / chosen, us per subcycle: 64x48 5.3 /
-// 4.0, 200x150 6.2 / 4.1, 300x220 6.9 / 5.9, 520x400 11.1 / 10.3 (31x15).
-// Beyond two tiles per CU the border's extra work counts: 31x19.
+// of four phases, whatever runs beside it, until the CUs are full, and a last
+// round of workgroups that is nearly empty takes as long as a full one.  So
+// the smallest tile is the fastest that is done in one round of one workgroup
+// per CU (in 15x11 every phase is one pass of 256 threads, 18x14 cells at
+// level 1; in 22x16 one of 512), then in one round of two per CU, then (31x13)
+// in two such rounds.  Beyond, the border's extra work counts: 31x19.
+// Measured on 1D lists, 31x19 / chosen, us per subcycle: 64x48 5.3 / 4.0,
+// 200x150 6.2 / 4.1, 352x256 7.0 / 6.0 (26x16), 400x300 7.3 / 6.8 (31x17),
+// 450x350 10.1 / 8.4 and 497x304 9.8 / 8.4 (22x16), 550x420 10.8 / 10.5
+// (31x17), 640x480 13.9 / 13.5, 700x500 15.2 / 14.4 and 733x517 15.6 / 15.2
+// (31x13); 800x600 18.6, 31x13 18.7; 900x700 22.2, 31x13 23.1.
 TileIds pair_tiles(const GridCoords &c, int order, int *block) {
   struct Rung { int w, h, block, most; };
-  static const Rung rungs[5] = {
-      {15, 11, 256, kCus}, {22, 16, 512, kCus}, {31, 19, 512, kCus}, {31, 15, 512, 2 * kCus}, {31, 19, 512, 0}};
+  static const Rung rungs[13] = {
+      {15, 11, 256, kCus},     {22, 16, 512, kCus},     {26, 16, 512, kCus},     {31, 15, 512, kCus},
+      {31, 17, 512, kCus},     {31, 19, 512, kCus},     {22, 16, 512, 2 * kCus}, {26, 16, 512, 2 * kCus},
+      {31, 15, 512, 2 * kCus}, {31, 17, 512, 2 * kCus}, {31, 19, 512, 2 * kCus}, {31, 13, 512, 4 * kCus},
+      {31, 19, 512, 0}};
   TileIds t;
   for (const Rung &r : rungs) {
     if (r.most > 0 && (int64_t)c.gx.size() / (r.w * r.h) > r.most) continue;
@@ -370,11 +378,12 @@ TileIds pair_tiles(const GridCoords &c, int order, int *block) {
   return t;
 }
 
-// 31x19 where its busiest tile has more than 512 level-2 stress points
-// (contiguous ice: 32x20) takes workgroups of 1024 threads, one per CU, which
-// nothing overlaps: 31x15 then (at most 512, two per CU).  1280x1520 in
-// contiguous ice 75.4 / 61.2 us per subcycle, 733x517 17.9 / 15.4.
-bool pair_may_crowd(const TileIds &t) { return t.tile_w == 31 && t.tile_h == 19 && t.ntiles > kCus; }
+// 31x17 and 31x19 where their busiest tile has more than 512 level-2 stress
+// points (contiguous ice: 32x18, 32x20) take workgroups of 1024 threads, one
+// per CU, which nothing overlaps: 31x15 then (at most 512, two per CU).
+// 1280x1520 in contiguous ice 75.4 / 61.2 us per subcycle, 800x600 20.9 /
+// 17.7, 550x420 12.9 (31x17) / 11.1.  With one tile per CU nothing is lost.
+bool pair_may_crowd(const TileIds &t) { return t.tile_w == 31 && t.tile_h >= 17 && t.ntiles > kCus; }
 bool pair_uncrowd(const GridCoords &c, int na, const int32_t *const idx[6], const uint8_t *skip, TileIds &t) {
   if (!pair_may_crowd(t) || max_level2(na, idx, skip, t) <= 512) return false;
   t = tile_ids(c, 31, 15, t.order);

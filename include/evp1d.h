@@ -235,10 +235,12 @@ int evp1d_get_tuning(const evp1d_handle *h, int32_t *stress_block, int32_t *stre
  * the tile ((tile_w+1)(tile_h+1) <= 2560), the workgroup size (64 to 512)
  * and the XCD-aware tile order (xcd = 0/1); a new tile re-lays the points out
  * at the next run.  Until it is called the library chooses by domain size.
- * Pair form (fused depth 2, the default): 15x11 cells if that gives at most
- * 256 tiles (one per CU), else 22x16 if at most 256, else 31x19 if at most
- * 256, else 31x15 if at most 512 or if some 31x19 tile has more than 512
- * level-2 stress points (contiguous ice), else 31x19.  One subcycle per
+ * Pair form (fused depth 2, the default): the first of 15x11, 22x16, 26x16,
+ * 31x15, 31x17 and 31x19 cells that gives at most 256 tiles (one per CU), else
+ * the first of 22x16, 26x16, 31x15, 31x17 and 31x19 with at most 512, else
+ * 31x13 if at most 1024, else 31x19; 31x15 in place of 31x17 and 31x19 where
+ * they give more than 256 tiles and one of them has more than 512 level-2
+ * stress points (contiguous ice).  One subcycle per
  * launch: 64x16 on 512 threads if that gives at least 1024 tiles, else 32x8
  * on 256 if at least 512, else 16x8 on 128 (XCD-aware order).
  * evp1d_get_tiling reports the tiling and the number of tiles (0 when the
