@@ -19,6 +19,7 @@ pytestmark = pytest.mark.gpu
     (40, 30, 0.7, 4, 0, 0),
     (70, 50, 0.4, 9, 3, -1),         # units of 3
     (70, 50, 1.0, 16, 4, 1),         # units of 4, the sweep's stresses packed from the stored states
+    (70, 50, 0.7, 10, 4, -1),        # units of 3 made 4: 4, 4, 2
     (352, 257, 1.0, 5, 0, -1),       # 1024 threads
     (497, 304, 0.7, 6, 0, 1),        # 31x15
     (620, 480, 0.7, 5, 0, 0),        # 31x19, 512 threads
