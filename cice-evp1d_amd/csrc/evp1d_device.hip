@@ -1089,7 +1089,7 @@ struct evp1d_handle {
   evp1d::PairTile *ptiles_dev = nullptr;
   int32_t *pxlist_dev = nullptr, *pelist_dev = nullptr, *pklist_dev = nullptr;
   uint2 *puloc_dev = nullptr, *pvloc_dev = nullptr;
-  int4 *ptnbr_dev = nullptr;
+  int4 *ptnbr_dev = nullptr, *ptsrc_dev = nullptr;
   int32_t *pfix_dev = nullptr;
   double2 *pcstr_dev = nullptr;
   double2 *pconst = nullptr;       // constant fields in pairs, [kPairConst][na], packed per run
@@ -1144,14 +1144,14 @@ static void drop_graph(evp1d_handle *h) {
 }
 
 static void free_pairs(evp1d_handle *h) {
-  void *bufs[9] = {h->ptiles_dev, h->pxlist_dev, h->pelist_dev, h->pklist_dev, h->puloc_dev,
-                   h->pvloc_dev,  h->pcstr_dev,  h->ptnbr_dev,  h->pfix_dev};
+  void *bufs[10] = {h->ptiles_dev, h->pxlist_dev, h->pelist_dev, h->pklist_dev, h->puloc_dev,
+                   h->pvloc_dev,  h->pcstr_dev,  h->ptnbr_dev,  h->pfix_dev, h->ptsrc_dev};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   h->ptiles_dev = nullptr;
   h->pxlist_dev = h->pelist_dev = h->pklist_dev = nullptr;
   h->puloc_dev = h->pvloc_dev = nullptr;
-  h->ptnbr_dev = nullptr;
+  h->ptnbr_dev = h->ptsrc_dev = nullptr;
   h->pfix_dev = nullptr;
   h->pcstr_dev = nullptr;
   h->pair_ok = false;
@@ -1367,6 +1367,7 @@ static int install_pairs(evp1d_handle *h, const evp1d::TilePlan &plan, const int
   RC_TRY(upload_table(h, &h->puloc_dev, reinterpret_cast<const uint2 *>(q.uloc.data()), q.uloc.size() / 4));
   RC_TRY(upload_table(h, &h->pvloc_dev, reinterpret_cast<const uint2 *>(q.vloc.data()), q.vloc.size() / 4));
   RC_TRY(upload_table(h, &h->ptnbr_dev, reinterpret_cast<const int4 *>(q.tnbr.data()), q.tnbr.size() / 4));
+  RC_TRY(upload_table(h, &h->ptsrc_dev, reinterpret_cast<const int4 *>(q.tsrc.data()), q.tsrc.size() / 4));
   RC_TRY(upload_table(h, &h->pfix_dev, q.fix.data(), q.fix.size()));
   h->pk_total = (long)q.klist.size();
   HIP_TRY(hipMalloc((void **)&h->pcstr_dev, std::max<size_t>((size_t)4 * h->pk_total, 1) * sizeof(double2)));
@@ -1830,6 +1831,11 @@ static int issue_fused(evp1d_handle *h, int nsub, double2 *traj = nullptr, bool 
       }
       const PairBufs bufs{in.vel, out.vel, P[pin], P[1 - pin]};
       pin = 1 - pin;
+      // from the third launch on a ghost's source is read in its place; the
+      // ghosts that copy no active point are the copies after the first two
+      // (one into each buffer), and the last one leaves them all as the run does
+      const bool copy = h->v.nhalo > 0 && (j <= 2 || j == L);
+      pv.tnbr = h->v.nhalo > 0 && j > 2 ? h->ptsrc_dev : h->ptnbr_dev;
       const PairKind kind = traj ? kPairTraj : h->v.nhalo > 0 ? kPairFix : kPairPlain;
       const PairFn fn = kPairFns[pair_block_index(h->pair_block)][kind][pair_hints(h) ? 1 : 0];
       if (traj) {
@@ -1841,7 +1847,7 @@ static int issue_fused(evp1d_handle *h, int nsub, double2 *traj = nullptr, bool 
         hipLaunchKernelGGL(fn, dim3(h->fused_ntiles), dim3(h->pair_block), lds2, h->stream, pv, bufs, j == L ? 1 : 0);
         HIP_TRY(hipGetLastError());
       }
-      if (h->v.nhalo > 0) {   // the copy after the launch's second subcycle
+      if (copy) {   // the copy after the launch's second subcycle
         hipLaunchKernelGGL(k_halo, dim3(blocks_for(h->v.nhalo)), dim3(kBlock), 0, h->stream, out);
         HIP_TRY(hipGetLastError());
       }

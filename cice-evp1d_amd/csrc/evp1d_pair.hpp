@@ -55,7 +55,7 @@ struct PairView {
   long lp;
   const double *strength;   // V0 = false: by slot
   long ls;                  // stresses: [6][ls] pairs (p1 p2, p3 p4, m1 m2, m3 m4, 12_1 12_2, 12_3 12_4)
-  const int4 *tnbr;         // per level-1 stress entry (PairTile::n0 + k): slot, ee, ne, se
+  const int4 *tnbr;         // per level-1 stress entry (PairTile::n0 + k): slot, ee, ne, se (PairPlan::tnbr, tsrc)
   const int32_t *fix;       // fixed copy-list sources of level-2 ghost reads (PairPlan::fix)
   // gradient trajectory (k_pair<.., TRAJ>): the velocities of the stepu
   // slots after the launch's first subcycle (tr_mid) and after its second
@@ -156,8 +156,9 @@ __device__ __forceinline__ void pair_tile(const PairView &f, PairBufs bf, int la
   // level 1, stress (or constants) of entry k
   auto level1 = [&](int k) {
     if (k < nT) {
-      const int4 n = f.tnbr[pt.n0 + k];   // slot and ee, ne, se of the entry
-      const int g = k < nO ? tslot(k) : n.x;
+      // slot (FIX: the slot of its velocity) and ee, ne, se of the entry
+      const int4 n = f.tnbr[pt.n0 + k];
+      const int g = k < nO || FIX ? tslot(k) : n.x;
       double sig[12];
 #pragma unroll
       for (int c = 0; c < 6; ++c) {
@@ -170,7 +171,7 @@ __device__ __forceinline__ void pair_tile(const PairView &f, PairBufs bf, int la
       for (int c = 0; c < kPairT<V0>; ++c) m[c] = in2<NT>(pc + (c * lp + g));
       const double st = V0 ? 0.0 : in1<NT>(f.strength + g);
       evp1d::StressOut o;
-      const double2 cc = bf.vel[g], ve = bf.vel[n.y], vn = bf.vel[n.z], vs = bf.vel[n.w];
+      const double2 cc = bf.vel[FIX ? n.x : g], ve = bf.vel[n.y], vn = bf.vel[n.z], vs = bf.vel[n.w];
       stress(cc, ve, vn, vs, m, st, sig, o);
       if (k == me) {
 #pragma unroll
@@ -241,7 +242,7 @@ __device__ __forceinline__ void pair_tile(const PairView &f, PairBufs bf, int la
   double2 c2[4];
   if (me < nS) {
     const int4 n = f.tnbr[pt.n0 + me];
-    g2 = me < nO ? tslot(me) : n.x;
+    g2 = me < nO || FIX ? tslot(me) : n.x;
     w2 = f.vloc[pt.v0 + me];
     c2[0] = bf.vel[g2];
     if (!FIX) {   // no copy list: every entry is a table entry or kNoEntry

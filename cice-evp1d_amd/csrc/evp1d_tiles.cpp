@@ -938,6 +938,7 @@ PairPlan plan_pairs(const TilePlan &p, int na, int navel, const int32_t *const i
   r.uloc.resize(4 * nu);
   r.vloc.resize(4 * nv);
   r.tnbr.resize(4 * nn);
+  r.tsrc.resize(halo.n > 0 ? 4 * nn : 0);
   r.fix.resize(nf);
   par_items(nt, [&](int t, int) {
     const PairWork &wk = work[(size_t)t];
@@ -948,6 +949,11 @@ PairPlan plan_pairs(const TilePlan &p, int na, int navel, const int32_t *const i
     std::copy(wk.uloc.begin(), wk.uloc.end(), r.uloc.begin() + (size_t)4 * pt.u0);
     std::copy(wk.vloc.begin(), wk.vloc.end(), r.vloc.begin() + (size_t)4 * pt.v0);
     std::copy(wk.tn.begin(), wk.tn.end(), r.tnbr.begin() + (size_t)4 * pt.n0);
+    if (halo.n > 0)
+      for (size_t j = 0; j < wk.tn.size(); ++j) {
+        const int32_t s = hmap[(size_t)wk.tn[j]];
+        r.tsrc[(size_t)4 * pt.n0 + j] = s >= u_begin && s < u_end ? s : wk.tn[j];
+      }
     std::copy(wk.fx.begin(), wk.fx.end(), r.fix.begin() + pt.f0);
   });
   r.ok = true;
@@ -983,6 +989,7 @@ std::string check_pairs(const PairPlan &q, const TilePlan &p, int na, int navel,
     if (pt.u0 < 0 || (size_t)4 * ((size_t)pt.u0 + nU) > q.uloc.size()) { e = "uloc range"; return; }
     if (pt.v0 < 0 || (size_t)4 * ((size_t)pt.v0 + nS) > q.vloc.size()) { e = "vloc range"; return; }
     if (pt.n0 < 0 || (size_t)4 * ((size_t)pt.n0 + nT) > q.tnbr.size()) { e = "tnbr range"; return; }
+    if (q.tsrc.size() != (halo.n > 0 ? q.tnbr.size() : 0)) { e = "tsrc range"; return; }
     if (nS > q.max_t2 || nE > q.cap_s || nU > q.cap_v) { e = "tile exceeds the plan's limits"; return; }
     std::vector<int32_t> &sm = smaps[(size_t)w], &vm = vmaps[(size_t)w];
     sm.assign((size_t)nE, -1);
@@ -1027,6 +1034,13 @@ std::string check_pairs(const PairPlan &q, const TilePlan &p, int na, int navel,
       if (tn[0] != g || tn[1] != slot(idx[0][r0]) || tn[2] != slot(idx[1][r0]) || tn[3] != slot(idx[2][r0])) {
         e = "stress entry " + std::to_string(k) + " of tile " + std::to_string(t) + ": bad neighbour slots";
         return;
+      }
+      for (int c = 0; c < 4 && halo.n > 0; ++c) {
+        const int32_t s = hmap[(size_t)tn[c]], want = s >= u_begin && s < u_end ? s : tn[c];
+        if (q.tsrc[(size_t)4 * (pt.n0 + k) + c] != want) {
+          e = "stress entry " + std::to_string(k) + " of tile " + std::to_string(t) + ": bad source slots";
+          return;
+        }
       }
     }
     // every level-2 stress read names the level-1 velocity of an active U

@@ -192,6 +192,10 @@ struct PairPlan {
   // its ee, ne, se neighbours, so one load gives every address the entry's
   // stress gathers
   Table<int32_t> tnbr;
+  // With a copy list, the same (first the slot whose velocity is the entry's
+  // own) with ghosts replaced by their source where that is an active U
+  // point: what a launch reads in place of copies made before it.
+  Table<int32_t> tsrc;
   // Copy list (evp1d_set_halo, evp2d_set_halo): between the two subcycles of a
   // launch a listed slot holds the copy of its source.  A level-2 read of such
   // a ghost names the source's level-1 velocity entry when the source is an

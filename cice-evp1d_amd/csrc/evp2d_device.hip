@@ -326,7 +326,9 @@ __global__ __launch_bounds__(kB2F) void k2_fused(View2 v, Fused2 f, int last) {
 // list the kernel is bound by the latency of its phases at 16 waves per CU,
 // with half the bytes of k2_fused: 1280x1520 in one block, 1000 subcycles,
 // 88 -> 65 us per subcycle; 800x600 in 2 x 2 blocks, 120 subcycles, 26.7 ->
-// 21.5 us, where the halo update is one launch per two subcycles, not four.
+// 20.6 us, where the halo update was four launches per two subcycles, and is
+// none after the second launch of a run: the tables name a halo cell's source
+// in its place (0.9 us a subcycle less than one copy per launch).
 
 // velocities of every slot, into both buffers
 __global__ void k2p_vel(double2 *a, double2 *b, const double2 *vel, const int32_t *cell, int n) {
@@ -430,7 +432,7 @@ struct evp2d_handle {
   const int32_t *phlist = nullptr, *pxlist = nullptr, *pelist = nullptr, *pfix = nullptr, *pcell = nullptr;
   const int32_t *phdst = nullptr, *phsrc = nullptr;
   const uint2 *puloc = nullptr, *pvloc = nullptr;
-  const int4 *ptnbr = nullptr;
+  const int4 *ptnbr = nullptr, *ptsrc = nullptr;
   int *pcnz = nullptr;
   double2 *pvel[2] = {nullptr, nullptr}, *psig[2] = {nullptr, nullptr}, *pconst = nullptr;
   // captured subcycle loop
@@ -764,6 +766,7 @@ int build_pairs2(evp2d_handle *h) {
   RC2(up(&h->puloc, q.uloc));
   RC2(up(&h->pvloc, q.vloc));
   RC2(up(&h->ptnbr, q.tnbr));
+  RC2(up(&h->ptsrc, q.tsrc));
   RC2(up(&h->pfix, q.fix));
   RC2(up(&h->pcell, scell));
   RC2(up(&h->phdst, hdst));
@@ -964,7 +967,6 @@ int issue_run2(evp2d_handle *h, int nsub) {
   f.pc = h->pconst;
   f.lp = h->na;
   f.ls = std::max(h->t_end, 1);
-  f.tnbr = h->ptnbr;
   f.fix = h->pfix;
   f.u_begin = h->u_begin;
   f.s15 = v.s15;
@@ -990,10 +992,14 @@ int issue_run2(evp2d_handle *h, int nsub) {
   int cur = 0;
   const int L = nsub / 2;
   for (int j = 1; j <= L; ++j) {
+    // from the third launch on a halo cell's source is read in its place: the
+    // copies after the first two (one into each buffer) are for the cells that
+    // copy no active point
+    f.tnbr = h->pnhalo > 0 && j > 2 ? h->ptsrc : h->ptnbr;
     const PairBufs bufs{h->pvel[cur], h->pvel[1 - cur], h->psig[cur], h->psig[1 - cur]};
     hipLaunchKernelGGL(fn, dim3(h->ptiles), dim3(h->pblock), lds, h->stream, f, bufs, j == L ? 1 : 0);
     cur = 1 - cur;
-    if (h->pnhalo > 0)
+    if (h->pnhalo > 0 && j <= 2 && j < L)
       hipLaunchKernelGGL(k2_copy, dim3(blocks2(h->pnhalo)), dim3(kB2), 0, h->stream, h->pvel[cur], h->phdst, h->phsrc,
                          h->pnhalo);
     HIP2(hipGetLastError());

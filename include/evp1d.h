@@ -369,9 +369,10 @@ int evp1d_loss_noalloc(evp1d_handle *h, const double *u_target, const double *v_
  * subcycles' velocities (seg x 16 B per stepu point beside the nsnap stored
  * states).  seg = 1: units of one subcycle, reversed from str1..8 recomputed
  * from the stored state.  seg = 0 (default): ceil(nsub / nsnap), made even in
- * the pair form when nsub is even, which stores every unit start and recomputes each unit once, when that trajectory fits
- * in free device memory beside the stored states, else 1.  The gradient is
- * the same bit for bit for every seg and nsnap.                            */
+ * the pair form when nsub is even, which stores every unit start and
+ * recomputes each unit once, when that trajectory fits in free device memory
+ * beside the stored states, else 1.  The gradient is the same bit for bit for
+ * every seg and nsnap.                                                      */
 int evp1d_set_adjoint_segment(evp1d_handle *h, int32_t seg);
 int evp1d_get_adjoint_segment(evp1d_handle *h, int32_t *seg);
 /* Device memory that gradient and tangent calls keep with the handle (no
