@@ -512,7 +512,11 @@ constexpr int kFusedMinSub = 4;          // evp1d_run in AUTO mode: fused from t
 // us), 500 for 64x48 (1.3 ms, 2.5 us), 1200 for 400x300 and 700x500 (5.5 and
 // 10 ms, 4.6 and 7.8 us).  A step of 240 subcycles at 1280x1520 with new
 // flags, fields in and out of 2D arrays: 65 -> 45 ms.
-constexpr int kPlanSub = 500;
+// The contracted build plans at the first run: there each form contracts in
+// its own way, and a state that goes on from a run in another form drifts from
+// the one it would have had (1e-13 after a run of 241 subcycles, up to 1e-7
+// after two).
+constexpr int kPlanSub = EVP1D_FMA ? 0 : 500;
 // launch configurations the autotuner chooses from
 constexpr int kNumBlocks = 5;
 constexpr int kBlocks[kNumBlocks] = {64, 128, 256, 512, 1024};
@@ -1700,8 +1704,11 @@ static const int kTanBlocks[2] = {256, 512};
 static const TanFn kTanFns[2] = {k_fused_tl<256>, k_fused_tl<512>};
 static size_t tan_lds(const evp1d_handle *h) { return (size_t)8 * std::max(h->fused_cap, 1) * sizeof(double2); }
 static int tan_block(const evp1d_handle *h) { return h->fused_cap <= kTanBlocks[0] ? 0 : 1; }
-// tangent subcycles run fused where there are tiles and their tables fit
-static bool tan_fused(const evp1d_handle *h) { return h->fused_ok && tan_lds(h) <= (size_t)kPairMaxLds; }
+// tangent subcycles run fused where there are tiles and their tables fit, but
+// not in the contracted build (kPlanSub)
+static bool tan_fused(const evp1d_handle *h) {
+  return !EVP1D_FMA && h->fused_ok && tan_lds(h) <= (size_t)kPairMaxLds;
+}
 
 // nsub fused subcycles.  The state starts in the handle's buffers (X).
 // Velocities, and stresses of a two-buffer run, are copied to the second set
@@ -3284,8 +3291,9 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
     int seg = h->adj_segment > 0 ? std::min<int>(h->adj_segment, nsub) : (nsub + S0 - 1) / S0;
     // whole pairs of subcycles: units then run from the stored stresses as
     // they are (lazy), without copies and without a first subcycle by itself
-    // (240 subcycles of 700x500 with 16 stored states 14.2 -> 13.4 ms)
-    if (h->adj_segment == 0 && seg > 1 && nsub % 2 == 0 && pair_form(h)) seg += seg % 2;
+    // (240 subcycles of 700x500 with 16 stored states 14.2 -> 13.4 ms; not in
+    // the contracted build, where another unit is another rounding)
+    if (!EVP1D_FMA && h->adj_segment == 0 && seg > 1 && nsub % 2 == 0 && pair_form(h)) seg += seg % 2;
     if (h->adj_segment == 0 && seg > 1) {
       size_t free_b = 0, total_b = 0;
       HIP_TRY(hipMemGetInfo(&free_b, &total_b));

@@ -46,6 +46,10 @@
 #include "evp1d_tiles.hpp"
 #include "evp1d_xcd.hpp"
 
+#ifndef EVP1D_FMA
+#define EVP1D_FMA 0
+#endif
+
 extern "C" int evp1d__set_error(int code, const char *msg);
 
 namespace {
@@ -614,10 +618,12 @@ int build_tiles2(evp2d_handle *h) {
 // at least kPairFirstSub.  Its plan costs more host time than the
 // one-subcycle tables (at 1280x1520 about 40 ms more, against 26 us saved per
 // subcycle; at 800x600 10 ms against 5 us), so lists that are used for one
-// run, as when every model step has its own ice mask, are not planned.
+// run, as when every model step has its own ice mask, are not planned.  The
+// contracted build keeps one subcycle per launch: its forms contract each in
+// its own way, and the first runs are never the pair form's.
 constexpr int kPairMinSub = 4, kPairFirstSub = 2000;
 bool wants_pair(const evp2d_handle *h, int nsub) {
-  return nsub >= kPairMinSub && (h->list_runs > 0 || nsub >= kPairFirstSub);
+  return !EVP1D_FMA && nsub >= kPairMinSub && (h->list_runs > 0 || nsub >= kPairFirstSub);
 }
 
 typedef void (*Pair2Fn)(PairView, PairBufs, int);

@@ -110,7 +110,8 @@ enum evp1d_mode {
                                  grid barrier between phases (hipLaunchCooperativeKernel) */
   EVP1D_MODE_AUTO = 3,        /* library default: FUSED when the lists tile and nsub >= 4, else GRAPH;
                                  LAUNCH for the first run with new skip flags if it is shorter than
-                                 500 subcycles (tiles are planned at the second run, or for a long one) */
+                                 500 subcycles (tiles are planned at the second run, or for a long one;
+                                 libevp1d_fma.so, whose forms round differently, plans at the first) */
   EVP1D_MODE_FUSED = 4        /* one launch per subcycle: stress and stepu per tile of points, str1..8
                                  kept on chip (hipGraph); needs lists that describe a grid */
 };
@@ -475,8 +476,9 @@ int evp2d_run(evp2d_handle *h, int32_t nsub);
  * launch with the 1D engine's pair form (evp1d_set_fused_depth), on the cells
  * of the lists as a 1D list with the halo update as its copy list, when the
  * same lists are run again (their plan takes host time) or for 2000
- * subcycles and more; else, and where the pair tables do not fit or stepu
- * writes a cell of the halo, one per launch: stress and stepu of one 32 x 8
+ * subcycles and more; else, in libevp1d_fma.so (whose forms round
+ * differently), and where the pair tables do not fit or stepu writes a cell
+ * of the halo, one per launch: stress and stepu of one 32 x 8
  * tile of cells per workgroup with str1..8 in LDS (the T cells of the column
  * east and the row north of the tile evaluated again).  Velocities and
  * stresses alternate between two buffers.  EVP2D_MODE_PLAIN runs the two

@@ -33,3 +33,18 @@ def test_chain_of_runs_and_flags(gpu, nx, ny, chain):
             lib.run(p, want, nsub)
             assert_state_bitexact(fetch_state(eng, st), want)
         assert eng.get_fused_depth()["active"] == bool((want.skipT == 0).any())
+
+
+def test_contracted_build_keeps_one_form(gpu):
+    """libevp1d_fma.so rounds by form: its first run takes the form that the
+    later ones take."""
+    st = synthetic_state(60, 45, seed=12, ice_prob=0.7)
+    got = []
+    for planned in (False, True):
+        with make_engine(st, 120, fma=True) as eng:
+            if planned:
+                assert eng.get_fused_depth()["active"]   # plans the tiles
+            eng.run(6)
+            eng.run(7)
+            got.append(fetch_state(eng, st))
+    assert_state_bitexact(got[0], got[1])
