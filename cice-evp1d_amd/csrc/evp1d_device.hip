@@ -2747,6 +2747,7 @@ struct AdjointRun {
   std::vector<StateBuf> slots;
   std::vector<char> used;
   StateBuf final_state;
+  bool pairs = false;            // k_pair_adj, with its second buffers
   double2 *sigb2 = nullptr, *ub2 = nullptr, *g2 = nullptr;   // k_pair_adj's second buffers of sigb, ub and g
   double2 *str_save = nullptr;   // [4][navel]
   double *ut = nullptr, *vt = nullptr, *terms = nullptr;
@@ -3061,7 +3062,6 @@ return EVP1D_OK;
     const bool hints = pair_hints(h);
     const auto stepu_adj = hints ? k_stepu_adj<true, true> : k_stepu_adj<true, false>;
     const auto stress_adj = hints ? k_stress_adj<true, true> : k_stress_adj<true, false>;
-    const bool pairs = pair_adj_form(h) && h->fused_ntiles > 0;
     for (int k = N; k >= 1; --k) {
       const DevView dk = view(k);
       if (nu > 0) hipLaunchKernelGGL(stepu_adj, dim3(blocks(nu)), dim3(256), 0, h->stream, dk, a);
@@ -3164,6 +3164,7 @@ static int gradient_workspace(evp1d_handle *h, const std::vector<size_t> &parts,
     h->adj_ws_bytes = 0;
     const hipError_t e = hipMalloc(&h->adj_ws, total);
     if (e != hipSuccess) {
+      (void)hipGetLastError();
       h->adj_ws = nullptr;
       return fail(EVP1D_ENOMEM, "%s: hipMalloc(%zu): %s", name, total, hipGetErrorString(e));
     }
@@ -3194,12 +3195,18 @@ int evp1d_adjoint_run(evp1d_handle *h, int32_t nsub, int32_t nsnap, const double
   int *cnz = nullptr;
   // adjoint state, gradient accumulators, targets and loss terms
   {
-    const bool pairs = pair_adj_form(h);
-    const std::vector<size_t> parts = {nV, R.sig_bytes(), nV, 4 * (size_t)h->na * sizeof(double2), nA, nA, nA, nA,
-                                       nA, nA, nA, sizeof(int), pairs ? nV : 0, pairs ? nV : 0,
-                                       pairs ? R.sig_bytes() : 0};
+    R.pairs = pair_adj_form(h) && h->fused_ntiles > 0;
+    std::vector<size_t> parts = {nV, R.sig_bytes(), nV, 4 * (size_t)h->na * sizeof(double2), nA, nA, nA, nA,
+                                 nA, nA, nA, sizeof(int), R.pairs ? nV : 0, R.pairs ? nV : 0,
+                                 R.pairs ? R.sig_bytes() : 0};
     std::vector<void *> at;
-    RC_TRY(gradient_workspace(h, parts, at, "evp1d_adjoint_run"));
+    int rc = gradient_workspace(h, parts, at, "evp1d_adjoint_run");
+    if (rc == EVP1D_ENOMEM && R.pairs) {   // the two kernels need less
+      R.pairs = false;
+      parts[12] = parts[13] = parts[14] = 0;
+      rc = gradient_workspace(h, parts, at, "evp1d_adjoint_run");
+    }
+    RC_TRY(rc);
     // all but ub2 and sigb2, which are written before they are read
     HIP_TRY(hipMemsetAsync(h->adj_ws, 0, (size_t)(static_cast<char *>(at[13]) - static_cast<char *>(h->adj_ws)),
                            h->stream));
@@ -3335,15 +3342,24 @@ int evp1d_tangent_run(evp1d_handle *h, int32_t nsub, const double *d_strength, c
   if (h->v.nhalo > 0) return fail(EVP1D_ESTATE, "evp1d_tangent_run: a ghost copy list is set");
   RC_TRY(ensure(h));
   const size_t nA = (size_t)h->na * sizeof(double), nV = (size_t)h->navel * sizeof(double2);
-  const bool fused = tan_fused(h) && nsub > 0 && h->fused_ntiles > 0;
+  bool fused = tan_fused(h) && nsub > 0 && h->fused_ntiles > 0;
   const size_t nS = (size_t)12 * h->ldsig * sizeof(double);
   // direction, targets, loss terms, then the tangent state: the unfused
   // form's derivatives, or the fused form's two buffers of both
-  std::vector<size_t> parts = {nA, nA, nA, nA, nA, nA, 2 * nA};
-  for (size_t b : fused ? std::vector<size_t>{2 * nS, 2 * nS, 2 * nV, 2 * nV} : std::vector<size_t>{nS, nV, nV, nV, nV, nV})
-    parts.push_back(b);
   std::vector<void *> at;
-  RC_TRY(gradient_workspace(h, parts, at, "evp1d_tangent_run"));
+  auto workspace = [&]() {
+    std::vector<size_t> parts = {nA, nA, nA, nA, nA, nA, 2 * nA};
+    for (size_t b : fused ? std::vector<size_t>{2 * nS, 2 * nS, 2 * nV, 2 * nV}
+                          : std::vector<size_t>{nS, nV, nV, nV, nV, nV})
+      parts.push_back(b);
+    return gradient_workspace(h, parts, at, "evp1d_tangent_run");
+  };
+  int wrc = workspace();
+  if (wrc == EVP1D_ENOMEM && fused) {   // the unfused form needs less
+    fused = false;
+    wrc = workspace();
+  }
+  RC_TRY(wrc);
   TanView t{};
   double *dir[4], *ut = (double *)at[4], *vt = (double *)at[5], *terms = (double *)at[6];
   const double *src[4] = {d_strength, d_cdn_ocn, d_forcex, d_forcey};

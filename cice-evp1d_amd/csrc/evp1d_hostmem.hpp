@@ -9,13 +9,14 @@
 
 // The address at which kernels write `bytes` at dst when dst is page-locked
 // host memory (evp1d_host_alloc, hipHostMalloc) of the current device that
-// holds them; null for any other memory, which takes a copy.  A gather that writes there needs no copy
-// behind it and no second wait for the queue: launch and wait take 11 us in
-// place of 14 for 100 values, 16 in place of 21 for 20 000, 40 in place of 47
-// for 200 000; from a million on both run at the host link's 50 GB/s (the
-// query takes 0.2 us).
+// holds them; null for any other memory, which takes a copy.  A gather that
+// writes there needs no copy behind it and no second wait for the queue: launch
+// and wait take 11 us in place of 14 for 100 values, 16 in place of 21 for
+// 20 000, 40 in place of 47 for 200 000, 155 in place of 163 for a million (the
+// query takes 0.2 us).  From two million values on the copy is 1 to 2 % faster
+// (53 GB/s): null for those.
 inline double *page_locked(double *dst, size_t bytes) {
-  if (reinterpret_cast<uintptr_t>(dst) % alignof(double)) return nullptr;
+  if (bytes > ((size_t)16 << 20) || reinterpret_cast<uintptr_t>(dst) % alignof(double)) return nullptr;
   hipPointerAttribute_t a{};
   hipDeviceptr_t base = nullptr;
   size_t size = 0;

@@ -758,7 +758,10 @@ int build_pairs2(evp2d_handle *h) {
   for (int s = 0; s < nslots; ++s) scell[(size_t)s] = cell[(size_t)(s < na ? plan.perm[(size_t)s] : s)];
   auto get = [&](auto **dst, const void *src, size_t bytes) -> int {
     void *p = nullptr;
-    HIP2(hipMalloc(&p, std::max<size_t>(bytes, 256)));
+    if (hipMalloc(&p, std::max<size_t>(bytes, 256)) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail2(EVP1D_ENOMEM, "evp2d pair plan: hipMalloc(%zu)", bytes);
+    }
     h->pbufs.push_back(p);
     if (src && bytes) HIP2(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, h->stream));
     *dst = static_cast<std::remove_reference_t<decltype(*dst)>>(p);
@@ -847,8 +850,16 @@ int ensure2_impl(evp2d_handle *h) {
 
 // the tables of the form that a run of nsub subcycles takes
 int ensure_form2(evp2d_handle *h, int nsub) {
-  if (wants_pair(h, nsub) && !h->pair_built)
-    RC2(evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); }));
+  if (wants_pair(h, nsub) && !h->pair_built) {
+    const int rc = evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); });
+    if (rc == EVP1D_ENOMEM) {   // one subcycle per launch needs less
+      HIP2(hipStreamSynchronize(h->stream));
+      for (void *b : h->pbufs) (void)hipFree(b);
+      h->pbufs.clear();
+    } else {
+      RC2(rc);
+    }
+  }
   const bool pair = wants_pair(h, nsub) && h->pair_ok;
   if ((!pair || nsub % 2 == 1) && !h->tiles_built)
     RC2(evp1d::no_throw("evp2d tiles", [h] { return build_tiles2(h); }));
