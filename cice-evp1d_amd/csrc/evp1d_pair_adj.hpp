@@ -25,7 +25,7 @@
 // What bounds it: bytes first, then the latency of the phases.  At 1280x1520
 // (31x19, 512 threads) a launch moves 890 MB at 4.7 TB/s (190 us for two
 // subcycles; streaming reaches 5.5 TB/s), where k_stepu_adj and k_stress_adj
-// move 1520 MB in 260 us: the adjoint stresses, ub, g and the accumulators go
+// move 1612 MB in 260 us: the adjoint stresses, ub, g and the accumulators go
 // through memory once per two subcycles, the velocity contributions never.
 // The launch bounds of k_pair (128 VGPRs, two 512-thread workgroups per CU)
 // hold because stress_adjoint is fenced (122 spilled registers without, 223
