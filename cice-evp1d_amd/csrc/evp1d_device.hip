@@ -909,36 +909,64 @@ __global__ void k_unpack_tl(DevView d, const double2 *sg, long ls, const double2
   if (i >= d.u_begin && i < d.u_end) d.vel[i] = v[2 * i];
 }
 
-// loss and its directional derivative terms at the current state; dvel:
-// slot q's derivative at q * stride
-__global__ void k_loss_tl(DevView d, const double2 *dvel, int stride, const double *ut, const double *vt,
-                          double *terms) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= d.na) return;
+// The sum of x over a workgroup of kBlock threads, in a fixed tree order; the
+// total is thread 0's.
+__device__ __forceinline__ double block_sum(double x) {
+  __shared__ double red[kBlock / 64];
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) x += __shfl_down(x, w, 64);
+  __syncthreads();   // a second call's writes wait for the first one's reads
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) x += red[w];
+  return x;
+}
+
+// Loss and its directional derivative at the current state, one sum per
+// workgroup: parts[b] and parts[gridDim.x + b].  dvel: slot q's derivative at
+// q * stride.  The host adds the parts in long double (sum_parts).  With every
+// slot's value copied to the host and added there one after the other, 11 MB at
+// 1280x1520, the rounding grew with the number of points: relative to the sum
+// in 64 bits of the same run 1.2e-14 at 400x300, now 6e-16.  Calls of 120
+// subcycles at 400x300 2.68 -> 2.53 ms, the gradient over 1000 at 1280x1520
+// 160.8 -> 159.6.
+__global__ __launch_bounds__(kBlock) void k_loss_tl(DevView d, const double2 *dvel, int stride, const double *ut,
+                                                    const double *vt, double *parts) {
+  const int q = blockIdx.x * kBlock + threadIdx.x;
   double l = 0.0, dl = 0.0;
-  if (q >= d.u_begin && q < d.u_end) {
+  if (q < d.na && q >= d.u_begin && q < d.u_end) {
     const double2 v = d.vel[q], tv = dvel[(long)stride * q];
     const double ex = v.x - ut[q], ey = v.y - vt[q];
     l = 0.5 * (ex * ex + ey * ey);
     dl = ex * tv.x + ey * tv.y;
   }
-  terms[q] = l;
-  terms[d.na + q] = dl;
+  l = block_sum(l);
+  dl = block_sum(dl);
+  if (threadIdx.x == 0) {
+    parts[blockIdx.x] = l;
+    parts[gridDim.x + blockIdx.x] = dl;
+  }
 }
 
-// loss terms and adjoint seed at the final state (active U slots)
-__global__ void k_seed(DevView d, AdjView a, const double *ut, const double *vt, double *terms) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= d.na) return;
+// loss (a sum per workgroup, as k_loss_tl) and adjoint seed at the final state
+// (active U slots)
+__global__ __launch_bounds__(kBlock) void k_seed(DevView d, AdjView a, const double *ut, const double *vt,
+                                                 double *parts) {
+  const int q = blockIdx.x * kBlock + threadIdx.x;
   double t = 0.0;
-  double2 s = make_double2(0.0, 0.0);
-  if (q >= d.u_begin && q < d.u_end) {
-    const double2 v = d.vel[q];
-    s = make_double2(v.x - ut[q], v.y - vt[q]);
-    t = 0.5 * (s.x * s.x + s.y * s.y);
+  if (q < d.na) {
+    double2 s = make_double2(0.0, 0.0);
+    if (q >= d.u_begin && q < d.u_end) {
+      const double2 v = d.vel[q];
+      s = make_double2(v.x - ut[q], v.y - vt[q]);
+      t = 0.5 * (s.x * s.x + s.y * s.y);
+    }
+    if (a.ub) a.ub[q] = s;
   }
-  if (a.ub) a.ub[q] = s;
-  terms[q] = t;
+  t = block_sum(t);
+  if (threadIdx.x == 0) parts[blockIdx.x] = t;
 }
 
 // data movement between caller order and slot order.  Element t of a host
@@ -2740,6 +2768,23 @@ static size_t trajectory_bytes(const evp1d_handle *h, int nsub) {
   return ((size_t)nsub * nu * sizeof(double2) + 255) / 256 * 256;
 }
 
+// The sums whose parts k_seed (m = 1) or k_loss_tl (m = 2) left at `parts`, one
+// per workgroup over the na points.  In long double the additions lose nothing
+// that the parts hold, so the result hardly depends on the order of the slots.
+static int sum_parts(evp1d_handle *h, const double *parts, int m, double *sums) {
+  const size_t nb = h->na > 0 ? (size_t)blocks_for(h->na) : 0;
+  std::vector<double> t(m * nb);
+  if (nb > 0)
+    HIP_TRY(hipMemcpyAsync(t.data(), parts, t.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  for (int k = 0; k < m; ++k) {
+    long double s = 0.0L;
+    for (size_t b = 0; b < nb; ++b) s += t[k * nb + b];
+    sums[k] = (double)s;
+  }
+  return EVP1D_OK;
+}
+
 struct AdjointRun {
   evp1d_handle *h;
   int nsub;
@@ -2911,16 +2956,11 @@ struct AdjointRun {
     for (int k = 0; k < 4; ++k)
       HIP_TRY(hipMemcpyAsync(str_save + (size_t)k * h->navel, pairs[k], nV, hipMemcpyDeviceToDevice, h->stream));
     if (h->na > 0) {
-      hipLaunchKernelGGL(k_seed, dim3(blocks(h->na)), dim3(256), 0, h->stream, fv, a, (const double *)ut,
+      hipLaunchKernelGGL(k_seed, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, fv, a, (const double *)ut,
                          (const double *)vt, terms);
       HIP_TRY(hipGetLastError());
     }
-    std::vector<double> t((size_t)h->na);
-    if (h->na > 0)
-      HIP_TRY(hipMemcpyAsync(t.data(), terms, (size_t)h->na * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    loss = 0.0;
-    for (double x : t) loss += x;
+    RC_TRY(sum_parts(h, terms, 1, &loss));
     return EVP1D_OK;
   }
   // reverse unit k with the working arrays holding its start state: one
@@ -3047,16 +3087,11 @@ return EVP1D_OK;
     if (final) {
       if (diag_save) RC_TRY(save_final());   // a segmented checkpointed run
       if (h->na > 0) {
-        hipLaunchKernelGGL(k_seed, dim3(blocks(h->na)), dim3(256), 0, h->stream, W, a, (const double *)ut,
+        hipLaunchKernelGGL(k_seed, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, W, a, (const double *)ut,
                            (const double *)vt, terms);
         HIP_TRY(hipGetLastError());
       }
-      std::vector<double> t((size_t)h->na);
-      if (h->na > 0)
-        HIP_TRY(hipMemcpyAsync(t.data(), terms, (size_t)h->na * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-      HIP_TRY(hipStreamSynchronize(h->stream));
-      loss = 0.0;
-      for (double x : t) loss += x;
+      RC_TRY(sum_parts(h, terms, 1, &loss));
     }
     // the reverse kernels take the handle's cache hints (pair_hints)
     const bool hints = pair_hints(h);
@@ -3417,21 +3452,15 @@ int evp1d_tangent_run(evp1d_handle *h, int32_t nsub, const double *d_strength, c
     }
     dvel = t.dvel;
   }
-  double l = 0.0, dl = 0.0;
+  double sums[2] = {0.0, 0.0};
   if (h->na > 0) {
     hipLaunchKernelGGL(k_loss_tl, dim3(blocks_for(h->na)), dim3(kBlock), 0, h->stream, d, dvel, fused ? 2 : 1,
                        (const double *)ut, (const double *)vt, terms);
     HIP_TRY(hipGetLastError());
-    std::vector<double> buf(2 * (size_t)h->na);
-    HIP_TRY(hipMemcpyAsync(buf.data(), terms, 2 * nA, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    for (int q = 0; q < h->na; ++q) {
-      l += buf[(size_t)q];
-      dl += buf[(size_t)h->na + q];
-    }
+    RC_TRY(sum_parts(h, terms, 2, sums));
   }
-  if (loss) *loss = l;
-  if (dloss) *dloss = dl;
+  if (loss) *loss = sums[0];
+  if (dloss) *dloss = sums[1];
   return EVP1D_OK;
 }
 
@@ -3451,14 +3480,10 @@ int evp1d_loss(evp1d_handle *h, const double *u_target, const double *v_target, 
                        (const double *)buf, (const double *)(buf + h->na), buf + 2 * h->na);
     if (hipGetLastError() != hipSuccess) rc = fail(EVP1D_EHIP, "evp1d_loss: launch failed");
   }
-  std::vector<double> t((size_t)h->na);
-  if (!rc && hipMemcpyAsync(t.data(), buf + 2 * h->na, (size_t)h->na * sizeof(double), hipMemcpyDeviceToHost,
-                            h->stream) != hipSuccess)
-    rc = fail(EVP1D_EHIP, "evp1d_loss: copy failed");
+  if (!rc) rc = sum_parts(h, buf + 2 * (size_t)h->na, 1, loss);
   if (hipStreamSynchronize(h->stream) != hipSuccess && !rc) rc = fail(EVP1D_EHIP, "evp1d_loss: sync failed");
   (void)hipFree(buf);
   if (rc) return rc;
-  for (double x : t) *loss += x;
   return EVP1D_OK;
 }
 
