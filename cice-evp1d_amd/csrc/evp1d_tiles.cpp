@@ -394,7 +394,10 @@ bool pair_uncrowd(const GridCoords &c, int na, const int32_t *const idx[6], cons
 // sw and sse neighbour): it is a halo entry of the other tiles among theirs.
 int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids) {
   std::vector<int32_t> n((size_t)std::max(ids.ntiles, 1), 0);
+  // counted per chunk and added once: one shared count for all was bound by its
+  // atomic additions (19 ms of the first run of a 1280x1520 grid on 8 threads)
   par_chunks(na, 1 << 15, [&](int64_t lo, int64_t hi, int) {
+    std::vector<int32_t> mine(n.size(), 0);
     for (int64_t q = lo; q < hi; ++q) {
       if (point_class(skip[q]) > 1) continue;
       int32_t seen[4] = {ids.tid[(size_t)q], -1, -1, -1};
@@ -407,8 +410,10 @@ int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const T
         const int32_t t = ids.tid[(size_t)r];
         if (std::find(seen, seen + m, t) == seen + m) seen[m++] = t;
       }
-      for (int i = 0; i < m; ++i) __atomic_fetch_add(&n[(size_t)seen[i]], 1, __ATOMIC_RELAXED);
+      for (int i = 0; i < m; ++i) ++mine[(size_t)seen[i]];
     }
+    for (size_t t = 0; t < n.size(); ++t)
+      if (mine[t]) __atomic_fetch_add(&n[t], mine[t], __ATOMIC_RELAXED);
   });
   return *std::max_element(n.begin(), n.end());
 }
