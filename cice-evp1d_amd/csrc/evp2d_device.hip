@@ -63,10 +63,15 @@ int fail2(int code, const char *fmt, ...) {
   return evp1d__set_error(code, buf);
 }
 
-#define HIP2(expr)                                                                      \
-  do {                                                                                  \
-    const hipError_t e_ = (expr);                                                       \
-    if (e_ != hipSuccess) return fail2(EVP1D_EHIP, "%s: %s", #expr, hipGetErrorString(e_)); \
+// (the runtime's last error is taken back: it belongs to this call, not to the
+// next one's launches)
+#define HIP2(expr)                                                               \
+  do {                                                                           \
+    const hipError_t e_ = (expr);                                                \
+    if (e_ != hipSuccess) {                                                      \
+      (void)hipGetLastError();                                                   \
+      return fail2(EVP1D_EHIP, "%s: %s", #expr, hipGetErrorString(e_));          \
+    }                                                                            \
   } while (0)
 #define RC2(expr)           \
   do {                      \
@@ -456,13 +461,12 @@ void drop_graph2(evp2d_handle *h) {
   h->graph_nsub = -1;
 }
 
-void free_lists2(evp2d_handle *h) {
-  void *bufs[16] = {h->tcell_dev, h->ucell_dev, h->fill_dev, h->dst_dev, h->src_dev,   h->tiles_dev,
-                    h->ftcell_dev, h->fucell_dev, h->ftlds_dev, h->fulds_dev, h->hidx_dev, h->ocell_dev,
-                    h->tc_dev,    h->uc_dev,     h->sg_dev[0], h->sg_dev[1]};
+// the one-subcycle form's tables
+void free_tiles2(evp2d_handle *h) {
+  void *bufs[11] = {h->tiles_dev, h->ftcell_dev, h->fucell_dev, h->ftlds_dev, h->fulds_dev, h->hidx_dev,
+                    h->ocell_dev, h->tc_dev,     h->uc_dev,     h->sg_dev[0], h->sg_dev[1]};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
-  h->tcell_dev = h->ucell_dev = h->fill_dev = h->dst_dev = h->src_dev = nullptr;
   h->tiles_dev = nullptr;
   h->ftcell_dev = h->fucell_dev = nullptr;
   h->ftlds_dev = h->fulds_dev = nullptr;
@@ -471,11 +475,32 @@ void free_lists2(evp2d_handle *h) {
   h->et = h->eu = h->no = 0;
   h->ntiles = 0;
   h->tiles_built = false;
+}
+
+// the pair form's tables
+void free_pairs2(evp2d_handle *h) {
   for (void *b : h->pbufs) (void)hipFree(b);
   h->pbufs.clear();
-  h->pair_built = h->pair_ok = false;
+  h->pair_ok = false;
+}
+
+void free_lists2(evp2d_handle *h) {
+  void *bufs[5] = {h->tcell_dev, h->ucell_dev, h->fill_dev, h->dst_dev, h->src_dev};
+  for (void *b : bufs)
+    if (b) (void)hipFree(b);
+  h->tcell_dev = h->ucell_dev = h->fill_dev = h->dst_dev = h->src_dev = nullptr;
+  free_tiles2(h);
+  free_pairs2(h);
+  h->pair_built = false;
   h->list_runs = 0;
 }
+
+// Waits for the stream's copies when it goes out of scope: declared after the
+// host memory that they read, whichever way that is left.
+struct CopiesDone {
+  hipStream_t stream;
+  ~CopiesDone() { (void)hipStreamSynchronize(stream); }
+};
 
 void release2(evp2d_handle *h) {
   if (!h) return;
@@ -504,8 +529,8 @@ int alloc2(evp2d_handle *h, void **ptr, size_t bytes) {
 // of it when it is on its tile's first column, of the tile south of it when
 // on the first row, and of the south-west tile when both; LDS entry of cell
 // (i, j) in tile (tx, ty): (j-1 - ty*kTH) * (kTW+1) + (i-1 - tx*kTW).
+// Left half done, as where memory lacks, they are freed (free_tiles2).
 int build_tiles2(evp2d_handle *h) {
-  h->tiles_built = true;
   const int ntx = (h->nxb + kTW - 1) / kTW, nty = (h->nyb + kTH - 1) / kTH;
   const long nt_all = (long)h->nblocks * ntx * nty;
   std::vector<std::vector<int32_t>> own((size_t)nt_all), halo((size_t)nt_all), uc((size_t)nt_all);
@@ -570,6 +595,7 @@ int build_tiles2(evp2d_handle *h) {
     ulds.insert(ulds.end(), uc_e[k].begin(), uc_e[k].end());
     tiles.push_back(d);
   }
+  const CopiesDone copies{h->stream};
   // every entry inside its tile's table, every stepu read too (the kernel
   // trusts these): the U entry e reads e+1, e+kTW+1 and e+kTW+2
   for (uint16_t e : tlds)
@@ -608,8 +634,8 @@ int build_tiles2(evp2d_handle *h) {
   HIP2(hipMalloc((void **)&h->uc_dev, std::max<size_t>((size_t)7 * h->eu, 1) * sizeof(double2)));
   for (int b = 0; b < 2; ++b)
     HIP2(hipMalloc((void **)&h->sg_dev[b], std::max<size_t>((size_t)6 * h->no, 1) * sizeof(double2)));
-  HIP2(hipStreamSynchronize(h->stream));   // the host vectors go out of scope
   h->ntiles = (int)tiles.size();
+  h->tiles_built = true;
   return EVP1D_OK;
 }
 
@@ -756,6 +782,8 @@ int build_pairs2(evp2d_handle *h) {
   if (pair_lds(cap, capv) > (size_t)kPairMaxLds) return EVP1D_OK;
   std::vector<int32_t> scell((size_t)nslots);
   for (int s = 0; s < nslots; ++s) scell[(size_t)s] = cell[(size_t)(s < na ? plan.perm[(size_t)s] : s)];
+  const std::vector<int> zero(1, 0);
+  const CopiesDone copies{h->stream};
   auto get = [&](auto **dst, const void *src, size_t bytes) -> int {
     void *p = nullptr;
     if (hipMalloc(&p, std::max<size_t>(bytes, 256)) != hipSuccess) {
@@ -780,7 +808,6 @@ int build_pairs2(evp2d_handle *h) {
   RC2(up(&h->pcell, scell));
   RC2(up(&h->phdst, hdst));
   RC2(up(&h->phsrc, hsrc));
-  const std::vector<int> zero(1, 0);
   RC2(up(&h->pcnz, zero));   // str of every cell outside the T list is zero
   h->t_end = plan.cnt[0] + plan.cnt[1];
   h->u_begin = plan.cnt[0];
@@ -791,7 +818,6 @@ int build_pairs2(evp2d_handle *h) {
     RC2(get(&h->pvel[b], nullptr, n2 * nslots));
     RC2(get(&h->psig[b], nullptr, n2 * 6 * std::max(h->t_end, 1)));
   }
-  HIP2(hipStreamSynchronize(h->stream));   // the host tables go out of scope
   int b = 0;
   while (kPairBlocks[b] < q.max_t2) ++b;   // max_t2 <= the largest block (plan limit)
   h->pblock = kPairBlocks[b];
@@ -852,17 +878,15 @@ int ensure2_impl(evp2d_handle *h) {
 int ensure_form2(evp2d_handle *h, int nsub) {
   if (wants_pair(h, nsub) && !h->pair_built) {
     const int rc = evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); });
-    if (rc == EVP1D_ENOMEM) {   // one subcycle per launch needs less
-      HIP2(hipStreamSynchronize(h->stream));
-      for (void *b : h->pbufs) (void)hipFree(b);
-      h->pbufs.clear();
-    } else {
-      RC2(rc);
-    }
+    if (rc) free_pairs2(h);
+    if (rc != EVP1D_ENOMEM) RC2(rc);   // one subcycle per launch needs less
   }
   const bool pair = wants_pair(h, nsub) && h->pair_ok;
-  if ((!pair || nsub % 2 == 1) && !h->tiles_built)
-    RC2(evp1d::no_throw("evp2d tiles", [h] { return build_tiles2(h); }));
+  if ((!pair || nsub % 2 == 1) && !h->tiles_built) {
+    const int rc = evp1d::no_throw("evp2d tiles", [h] { return build_tiles2(h); });
+    if (rc) free_tiles2(h);
+    RC2(rc);
+  }
   if ((!pair || nsub % 2 == 1) && !h->vel_alt)
     HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
   return EVP1D_OK;
