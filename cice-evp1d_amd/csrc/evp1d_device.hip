@@ -75,12 +75,16 @@ static int fail(int code, const char *fmt, ...) {
   return code;
 }
 
+// (the runtime's last error is taken back: it belongs to this call, not to the
+// next one's launches)
 #define HIP_TRY(expr)                                                          \
   do {                                                                         \
     hipError_t e_ = (expr);                                                    \
-    if (e_ != hipSuccess)                                                      \
+    if (e_ != hipSuccess) {                                                    \
+      (void)hipGetLastError();                                                 \
       return fail(EVP1D_EHIP, "%s failed: %s (%s:%d)", #expr,                  \
                   hipGetErrorString(e_), __FILE__, __LINE__);                  \
+    }                                                                          \
   } while (0)
 
 #define RC_TRY(expr)              \
@@ -1160,8 +1164,10 @@ static Scalars scalars_from(const evp1d_params &p) {
 static int dev_alloc(evp1d_handle *h, void **ptr, size_t bytes) {
   if (bytes == 0) bytes = 256;
   hipError_t e = hipMalloc(ptr, bytes);
-  if (e != hipSuccess)
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
     return fail(EVP1D_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+  }
   h->allocs.push_back(*ptr);
   HIP_TRY(hipMemsetAsync(*ptr, 0, bytes, h->stream));
   return EVP1D_OK;
@@ -1468,6 +1474,7 @@ static int relayout_impl(evp1d_handle *h, bool tiles) {
   if (!bad.empty()) return fail(EVP1D_EINDEX, "slot layout: %s", bad.c_str());
   const std::vector<int32_t> &nperm = plan.perm;
   if (na > 0 && nperm != h->perm) {
+    h->layout_dirty = h->idx_dirty = true;   // until the lists and tables follow, also where their plan fails
     std::vector<int32_t> map((size_t)na), ninv((size_t)na);
     for (int s = 0; s < na; ++s) {
       map[(size_t)s] = h->inv[(size_t)nperm[(size_t)s]];
@@ -2476,7 +2483,10 @@ struct SavedState {
       if (bytes == 0) return EVP1D_OK;
       void *b = nullptr;
       const hipError_t e = hipMalloc(&b, bytes);
-      if (e != hipSuccess) return fail(EVP1D_ENOMEM, "%s: hipMalloc(%zu): %s", who, bytes, hipGetErrorString(e));
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(EVP1D_ENOMEM, "%s: hipMalloc(%zu): %s", who, bytes, hipGetErrorString(e));
+      }
       bufs.push_back(Buf{p, b, bytes});
       HIP_TRY(hipMemcpyAsync(b, p, bytes, hipMemcpyDeviceToDevice, h->stream));
       return EVP1D_OK;
@@ -2833,6 +2843,7 @@ struct AdjointRun {
       h->ckpt_bytes = 0;
       const hipError_t e = hipMalloc(&h->ckpt, total);
       if (e != hipSuccess) {
+        (void)hipGetLastError();
         h->ckpt = nullptr;
         return fail(EVP1D_ENOMEM, "evp1d_adjoint_run: hipMalloc(%zu) for %d stored states: %s", total, nslots,
                     hipGetErrorString(e));
@@ -3022,6 +3033,7 @@ return EVP1D_OK;
                     need / 1e9, free_b / 1e9);
       const hipError_t e = hipMalloc(&h->traj, need);
       if (e != hipSuccess) {
+        (void)hipGetLastError();
         h->traj = nullptr;
         return fail(EVP1D_ENOMEM, "evp1d_adjoint_run: hipMalloc(%zu): %s", need, hipGetErrorString(e));
       }
@@ -3703,6 +3715,7 @@ int evp1d_host_alloc(int64_t bytes, void **ptr) {
   *ptr = nullptr;
   const hipError_t e = hipHostMalloc(ptr, (size_t)std::max<int64_t>(bytes, 1), hipHostMallocDefault);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     *ptr = nullptr;
     return fail(EVP1D_ENOMEM, "evp1d_host_alloc(%lld): %s", (long long)bytes, hipGetErrorString(e));
   }

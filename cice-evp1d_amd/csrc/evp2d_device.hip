@@ -517,7 +517,10 @@ void release2(evp2d_handle *h) {
 
 int alloc2(evp2d_handle *h, void **ptr, size_t bytes) {
   const hipError_t e = hipMalloc(ptr, std::max<size_t>(bytes, 256));
-  if (e != hipSuccess) return fail2(EVP1D_ENOMEM, "evp2d_create: hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail2(EVP1D_ENOMEM, "evp2d_create: hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+  }
   h->allocs.push_back(*ptr);
   HIP2(hipMemsetAsync(*ptr, 0, std::max<size_t>(bytes, 256), h->stream));
   return EVP1D_OK;
