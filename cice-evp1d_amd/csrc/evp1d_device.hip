@@ -1658,11 +1658,13 @@ static int fused_block_index(int b) {
   return -1;
 }
 
-// Lets fn use `bytes` of LDS where that is more than every kernel may: asked
-// for the kernels about to run, not for every variant of a new handle.
+// Lets fn use all of a CU's LDS where it needs `bytes` and that is more than
+// every kernel may: asked for the kernels about to run, not for every variant
+// of a new handle.  The limit belongs to the kernel, so it is no handle's own
+// size, which another handle's launch, from another thread, could exceed.
 static int allow_lds(const void *fn, size_t bytes) {
   if (bytes > 64 * 1024)
-    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
   return EVP1D_OK;
 }
 
