@@ -508,7 +508,8 @@ __global__ void k_fill_const(DevView d, const int32_t *klist, double2 *cstr, lon
 constexpr int kFusedMaxEntries = 2560;   // 160 KiB of LDS per workgroup (gfx950)
 constexpr int kFusedMinSub = 4;          // evp1d_run in AUTO mode: fused from this many subcycles
 // evp1d_run in AUTO mode plans tiles for a new set of skip flags at its first
-// run of this many subcycles, or at the second run; a shorter first run (a
+// run of this many subcycles, at the second run, or where the caller has set a
+// tile, an order or a depth since the last plan; a shorter first run (a
 // model step whose ice mask is new) goes over the points in class order, one
 // kernel for stress and one for stepu.  Planning takes 32 ms longer than the
 // class order at 1280x1520 and the tiles then save 57 us a subcycle (62
@@ -1078,7 +1079,8 @@ struct evp1d_handle {
   std::vector<int32_t> halo_dst_host, halo_src_host;   // caller order, -1 = fill
   bool layout_dirty = false;       // skip flags changed since the last relayout
   bool layout_tiled = false;       // the slot order was made with tiles (or none fit), not by class alone
-  long layout_runs = 0;            // evp1d_run calls since the slot order was first made for these flags
+  bool new_points = true;          // skip flags or lists changed since the last evp1d_run
+  bool tiles_asked = false;        // a tile, order or depth was set since tiles were last planned
   bool idx_dirty = false;          // slot-space lists need re-upload
   int mode = EVP1D_MODE_AUTO;
   LaunchCfg cfg_stress, cfg_stepu;
@@ -1510,6 +1512,7 @@ static int relayout_impl(evp1d_handle *h, bool tiles) {
   h->v.u_end = plan.cnt[0] + plan.cnt[1] + plan.cnt[2];
   h->layout_dirty = false;
   h->layout_tiled = tiles;
+  if (tiles) h->tiles_asked = false;
   h->idx_dirty = true;
   h->graph_dirty = true;
   return EVP1D_OK;
@@ -1520,7 +1523,6 @@ static inline int32_t slot_of(const evp1d_handle *h, int32_t q) { return q < h->
 // bring the device copy of layout, lists and halo up to date; tiles: and the
 // fused forms' tiles (else an order that is up to date stays, tiled or not)
 static int ensure(evp1d_handle *h, bool tiles = true) {
-  if (h->layout_dirty) h->layout_runs = 0;
   if (h->layout_dirty || (tiles && !h->layout_tiled)) RC_TRY(relayout(h, tiles));
   if (!h->idx_dirty) return EVP1D_OK;
   const int na = h->na;
@@ -2231,7 +2233,7 @@ static int set_index_impl(evp1d_handle *h, int k, int32_t which, const int32_t *
   if (k < 0) std::fill(ms.begin(), ms.end(), (uint8_t)1); else ms[(size_t)k] = 1;
   h->idx_set[which] = std::all_of(ms.begin(), ms.end(), [](uint8_t b) { return b != 0; });
   h->idx_dirty = true;
-  h->layout_dirty = true;   // the tiled slot order follows the lists
+  h->layout_dirty = h->new_points = true;   // the tiled slot order follows the lists
   h->tile_cache_ok = false;
   h->coords_ok = false;
   h->idx_caller_dirty[which] = true;
@@ -2253,7 +2255,7 @@ static int set_skip_impl(evp1d_handle *h, int k, int32_t which, const int32_t *f
     diff |= (uint8_t)(nb ^ skip[i]);
     skip[i] = nb;
   }
-  if (diff) h->layout_dirty = true;
+  if (diff) h->layout_dirty = h->new_points = true;
   return EVP1D_OK;
 }
 
@@ -2355,10 +2357,9 @@ int evp1d_run(evp1d_handle *h, int32_t nsub) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_run: NULL handle");
   if (nsub < 0) return fail(EVP1D_EINVAL, "evp1d_run: nsub=%d < 0", nsub);
   if (!ready(h)) return fail(EVP1D_ESTATE, "evp1d_run: neighbour lists not set");
-  const bool first = h->layout_dirty || h->layout_runs == 0;
-  RC_TRY(ensure(h, h->mode != EVP1D_MODE_AUTO || !first || nsub >= kPlanSub));
+  RC_TRY(ensure(h, h->mode != EVP1D_MODE_AUTO || !h->new_points || h->tiles_asked || nsub >= kPlanSub));
   if (nsub == 0 || h->na == 0) return EVP1D_OK;
-  ++h->layout_runs;
+  h->new_points = false;
   switch (h->mode) {
     case EVP1D_MODE_LAUNCH: return issue_subcycles(h, nsub);
     case EVP1D_MODE_PERSISTENT: return run_persistent(h, nsub);
@@ -2432,7 +2433,7 @@ int evp1d_set_tiling(evp1d_handle *h, int32_t tile_w, int32_t tile_h, int32_t bl
   if (fused_block_index(block) < 0) return fail(EVP1D_EINVAL, "evp1d_set_tiling: block must be 64, 128, 256 or 512");
   h->tile_block = block;
   if (tile_w != h->tile_w || tile_h != h->tile_h || h->tiling_auto) {
-    h->layout_dirty = true;
+    h->layout_dirty = h->tiles_asked = true;
     h->tile_cache_ok = false;
   }
   h->tiling_auto = false;
@@ -2448,7 +2449,7 @@ int evp1d_set_tile_order(evp1d_handle *h, int32_t order) {
   if (order != 0 && order != 1) return fail(EVP1D_EINVAL, "evp1d_set_tile_order: order must be 0 or 1");
   if (order != h->tile_order) {
     h->tile_order = order;
-    h->layout_dirty = true;
+    h->layout_dirty = h->tiles_asked = true;
     h->tile_cache_ok = false;
     h->graph_dirty = true;
   }
@@ -2584,7 +2585,7 @@ int evp1d_set_fused_depth(evp1d_handle *h, int32_t depth) {
   if (depth != h->fused_depth) {
     HIP_TRY(hipStreamSynchronize(h->stream));   // no queued run may still use the old tables
     h->fused_depth = depth;
-    h->layout_dirty = true;                     // plan (or drop) the pair tables
+    h->layout_dirty = h->tiles_asked = true;    // plan (or drop) the pair tables
     h->graph_dirty = true;
     if (h->tiling_auto) h->tile_cache_ok = false;   // the library's tile depends on the depth
   }

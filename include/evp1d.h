@@ -109,8 +109,10 @@ enum evp1d_mode {
                                  barrier per two subcycles, else stress and stepu over all points with a
                                  grid barrier between phases (hipLaunchCooperativeKernel) */
   EVP1D_MODE_AUTO = 3,        /* library default: FUSED when the lists tile and nsub >= 4, else GRAPH;
-                                 LAUNCH for the first run with new skip flags if it is shorter than
-                                 500 subcycles (tiles are planned at the second run, or for a long one;
+                                 LAUNCH for the first run with new skip flags or lists if it is shorter
+                                 than 500 subcycles (tiles are planned at the second run, for a long one,
+                                 or where evp1d_set_tiling, evp1d_set_tile_order, evp1d_set_fused_depth
+                                 or a tuner has changed them since the last plan;
                                  libevp1d_fma.so, whose forms round differently, plans at the first) */
   EVP1D_MODE_FUSED = 4        /* one launch per subcycle: stress and stepu per tile of points, str1..8
                                  kept on chip (hipGraph); needs lists that describe a grid */
