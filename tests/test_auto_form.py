@@ -81,3 +81,9 @@ def test_settings_that_change_later_bring_no_class_order_back(fake, st, setting)
         if setting == "halo":
             eng.set_halo(np.array([st.na + 1], np.int32), np.array([1], np.int32))
         assert _run(eng, fake, 12) == ("tiles" if setting == "depth" else "pairs")
+
+
+def test_tiles_planned_by_a_getter_are_what_the_first_run_takes(fake, st):
+    with make_engine(st, 120) as eng:
+        assert eng.get_fused_depth()["active"]
+        assert _run(eng, fake) == "pairs"
