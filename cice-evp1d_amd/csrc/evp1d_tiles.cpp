@@ -25,8 +25,6 @@ inline int point_class(uint8_t b) {
 constexpr int kDx[6] = {-1, -1, 0, 1, 1, 0};
 constexpr int kDy[6] = {0, -1, -1, 0, 1, 1};
 
-// class order with caller order inside each class (the untiled layout)
-
 // Grid coordinates of every point from the neighbour lists, one frame per
 // connected component, components placed side by side.  Returns false when
 // the lists are not those of a grid (a point reached at two positions).
@@ -138,64 +136,6 @@ static int64_t hilbert_index(int64_t n, int64_t x, int64_t y) {
   return d;
 }
 
-TileIds tile_ids(const GridCoords &c, int tile_w, int tile_h, int order) {
-  TileIds t;
-  t.tile_w = tile_w;
-  t.tile_h = tile_h;
-  t.order = order;
-  if (!c.ok) {
-    t.why = c.why;
-    return t;
-  }
-  if (tile_w < 1 || tile_h < 1) {
-    t.why = "tile size < 1";
-    return t;
-  }
-  if (order != 0 && order != 1) {
-    t.why = "tile order must be 0 or 1";
-    return t;
-  }
-  const int na = (int)c.gx.size();
-  // dense tile ids in (row of tiles, column of tiles) order, or along a
-  // Hilbert curve over the square of side hn that holds the tile grid
-  const int64_t ntx = (c.width + tile_w - 1) / tile_w, nty = (c.height + tile_h - 1) / tile_h;
-  int64_t hn = 1;
-  while (hn < ntx || hn < nty) hn *= 2;
-  const int64_t nkey = order == 1 ? hn * hn : ntx * nty;
-  auto key_of = [&](int q) {
-    const int64_t tx = c.gx[(size_t)q] / tile_w, ty = c.gy[(size_t)q] / tile_h;
-    return order == 1 ? hilbert_index(hn, tx, ty) : ty * ntx + tx;
-  };
-  t.tid.resize((size_t)na);
-  if (nkey <= 4 * (int64_t)na + 1024 && nkey <= 4 * ntx * nty + 1024) {   // a table over all tile positions
-    std::vector<int32_t> dense((size_t)nkey, -1);
-    for (int q = 0; q < na; ++q) dense[(size_t)key_of(q)] = 0;
-    int32_t n = 0;
-    for (int32_t &d : dense)
-      if (d == 0) d = n++;
-    for (int q = 0; q < na; ++q) t.tid[(size_t)q] = dense[(size_t)key_of(q)];
-    t.ntiles = n;
-  } else {   // sparse frames (many small components): sort the keys
-    std::vector<int64_t> keys((size_t)na);
-    for (int q = 0; q < na; ++q) keys[(size_t)q] = key_of(q);
-    std::sort(keys.begin(), keys.end());
-    keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
-    for (int q = 0; q < na; ++q)
-      t.tid[(size_t)q] = (int32_t)(std::lower_bound(keys.begin(), keys.end(), key_of(q)) - keys.begin());
-    t.ntiles = (int)keys.size();
-  }
-  return t;
-}
-
-TileIds tile_ids(int na, int navel, const int32_t *const idx[6], int tile_w, int tile_h) {
-  return tile_ids(grid_coords(na, navel, idx), tile_w, tile_h);
-}
-
-TilePlan plan_tiles(int na, int navel, const int32_t *const idx[6], const uint8_t *skip, int tile_w, int tile_h,
-                    int max_entries) {
-  return plan_tiles(na, navel, idx, skip, tile_ids(na, navel, idx, tile_w, tile_h), max_entries);
-}
-
 namespace {
 
 // Host threads for the planner and its check: the machine's, at most 16.
@@ -256,10 +196,12 @@ void par_chunks(int64_t n, int64_t grain, F f) {
   run_workers(T, [&](int w) { f(n * w / T, n * (w + 1) / T, w); });
 }
 
-// f(i, w) for every i in [0, n), items handed out dynamically (uneven work)
+// f(i, w) for every i in [0, n), items handed out dynamically (uneven work);
+// work: the points of them all (fewer than 2048 a thread take less time than
+// its start: a first run's planning of 64x48 0.55 ms in place of 0.99)
 template <class F>
-void par_items(int n, F f) {
-  const int T = std::max(1, std::min(plan_threads(), n / 4));
+void par_items(int n, int64_t work, F f) {
+  const int T = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(plan_threads(), n / 4), work / 2048));
   if (T <= 1) {
     for (int i = 0; i < n; ++i) f(i, 0);
     return;
@@ -270,6 +212,75 @@ void par_items(int n, F f) {
       for (int j = i; j < std::min(n, i + 8); ++j) f(j, w);
   });
 }
+
+}  // namespace
+
+TileIds tile_ids(const GridCoords &c, int tile_w, int tile_h, int order) {
+  TileIds t;
+  t.tile_w = tile_w;
+  t.tile_h = tile_h;
+  t.order = order;
+  if (!c.ok) {
+    t.why = c.why;
+    return t;
+  }
+  if (tile_w < 1 || tile_h < 1) {
+    t.why = "tile size < 1";
+    return t;
+  }
+  if (order != 0 && order != 1) {
+    t.why = "tile order must be 0 or 1";
+    return t;
+  }
+  const int na = (int)c.gx.size();
+  // dense tile ids in (row of tiles, column of tiles) order, or along a
+  // Hilbert curve over the square of side hn that holds the tile grid
+  const int64_t ntx = (c.width + tile_w - 1) / tile_w, nty = (c.height + tile_h - 1) / tile_h;
+  int64_t hn = 1;
+  while (hn < ntx || hn < nty) hn *= 2;
+  const int64_t nkey = order == 1 ? hn * hn : ntx * nty;
+  auto key_of = [&](int q) {
+    const int64_t tx = c.gx[(size_t)q] / tile_w, ty = c.gy[(size_t)q] / tile_h;
+    return order == 1 ? hilbert_index(hn, tx, ty) : ty * ntx + tx;
+  };
+  t.tid.resize((size_t)na);
+  if (nkey <= 4 * (int64_t)na + 1024 && nkey <= 4 * ntx * nty + 1024) {   // a table over all tile positions
+    std::vector<int32_t> dense((size_t)nkey, -1);
+    par_chunks(na, 1 << 14, [&](int64_t lo, int64_t hi, int) {   // every writer stores 0
+      for (int64_t q = lo; q < hi; ++q) {
+        int32_t &d = dense[(size_t)key_of((int)q)];
+        if (__atomic_load_n(&d, __ATOMIC_RELAXED) != 0) __atomic_store_n(&d, 0, __ATOMIC_RELAXED);
+      }
+    });
+    int32_t n = 0;
+    for (int32_t &d : dense)
+      if (d == 0) d = n++;
+    par_chunks(na, 1 << 14, [&](int64_t lo, int64_t hi, int) {
+      for (int64_t q = lo; q < hi; ++q) t.tid[(size_t)q] = dense[(size_t)key_of((int)q)];
+    });
+    t.ntiles = n;
+  } else {   // sparse frames (many small components): sort the keys
+    std::vector<int64_t> keys((size_t)na);
+    for (int q = 0; q < na; ++q) keys[(size_t)q] = key_of(q);
+    std::sort(keys.begin(), keys.end());
+    keys.erase(std::unique(keys.begin(), keys.end()), keys.end());
+    for (int q = 0; q < na; ++q)
+      t.tid[(size_t)q] = (int32_t)(std::lower_bound(keys.begin(), keys.end(), key_of(q)) - keys.begin());
+    t.ntiles = (int)keys.size();
+  }
+  return t;
+}
+
+TileIds tile_ids(int na, int navel, const int32_t *const idx[6], int tile_w, int tile_h) {
+  return tile_ids(grid_coords(na, navel, idx), tile_w, tile_h);
+}
+
+TilePlan plan_tiles(int na, int navel, const int32_t *const idx[6], const uint8_t *skip, int tile_w, int tile_h,
+                    int max_entries) {
+  return plan_tiles(na, navel, idx, skip, tile_ids(na, navel, idx, tile_w, tile_h), max_entries);
+}
+
+namespace {
 
 // the order by class, then caller position: per-chunk counts, then each chunk
 // places its points
@@ -385,35 +396,56 @@ TileIds pair_tiles(const GridCoords &c, int order, int *block) {
 // 17.7, 550x420 12.9 (31x17) / 11.1.  With one tile per CU nothing is lost.
 bool pair_may_crowd(const TileIds &t) { return t.tile_w == 31 && t.tile_h >= 17 && t.ntiles > kCus; }
 bool pair_uncrowd(const GridCoords &c, int na, const int32_t *const idx[6], const uint8_t *skip, TileIds &t) {
-  if (!pair_may_crowd(t) || max_level2(na, idx, skip, t) <= 512) return false;
+  if (!pair_may_crowd(t) || !crowded(na, idx, skip, t, 512)) return false;
   t = tile_ids(c, 31, 15, t.order);
   return true;
+}
+
+// counts[t]: how many of the points [0, na) f(q, add) adds to tile t with
+// add(t); per chunk, added once: one shared count for all was bound by its
+// atomic additions (19 ms of the first run of a 1280x1520 grid on 8 threads)
+template <class F>
+static std::vector<int32_t> tile_counts(int na, const TileIds &ids, F f) {
+  std::vector<int32_t> n((size_t)std::max(ids.ntiles, 1), 0);
+  par_chunks(na, 1 << 15, [&](int64_t lo, int64_t hi, int) {
+    std::vector<int32_t> mine(n.size(), 0);
+    for (int64_t q = lo; q < hi; ++q) f((int32_t)q, [&](int32_t t) { ++mine[(size_t)t]; });
+    for (size_t t = 0; t < n.size(); ++t)
+      if (mine[t]) __atomic_fetch_add(&n[t], mine[t], __ATOMIC_RELAXED);
+  });
+  return n;
+}
+
+// A tile's level-2 points are the stress points that it owns and, east and
+// north of it, at most tile_w + tile_h + 1 more: most masks are decided by the
+// owned points alone.  With tile_ids on 16 threads a first run's planning of
+// 1280x1520 takes 146 ms in place of 157, in contiguous ice 159 in place of 169.
+bool crowded(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids, int most) {
+  const std::vector<int32_t> own = tile_counts(na, ids, [&](int32_t q, auto add) {
+    if (point_class(skip[q]) <= 1) add(ids.tid[(size_t)q]);
+  });
+  const int32_t busiest = *std::max_element(own.begin(), own.end());
+  if (busiest > most) return true;
+  if (busiest + ids.tile_w + ids.tile_h + 1 <= most) return false;
+  return max_level2(na, idx, skip, ids) > most;
 }
 
 // T point q is read by the stepu points ee(q), ne(q) and se(q) (as their nw,
 // sw and sse neighbour): it is a halo entry of the other tiles among theirs.
 int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids) {
-  std::vector<int32_t> n((size_t)std::max(ids.ntiles, 1), 0);
-  // counted per chunk and added once: one shared count for all was bound by its
-  // atomic additions (19 ms of the first run of a 1280x1520 grid on 8 threads)
-  par_chunks(na, 1 << 15, [&](int64_t lo, int64_t hi, int) {
-    std::vector<int32_t> mine(n.size(), 0);
-    for (int64_t q = lo; q < hi; ++q) {
-      if (point_class(skip[q]) > 1) continue;
-      int32_t seen[4] = {ids.tid[(size_t)q], -1, -1, -1};
-      int m = 1;
-      for (int k : {0, 1, 2}) {
-        const int32_t r = idx[k][q];
-        if (r < 0 || r >= na) continue;
-        const int c = point_class(skip[r]);
-        if (c != 1 && c != 2) continue;
-        const int32_t t = ids.tid[(size_t)r];
-        if (std::find(seen, seen + m, t) == seen + m) seen[m++] = t;
-      }
-      for (int i = 0; i < m; ++i) ++mine[(size_t)seen[i]];
+  const std::vector<int32_t> n = tile_counts(na, ids, [&](int32_t q, auto add) {
+    if (point_class(skip[q]) > 1) return;
+    int32_t seen[4] = {ids.tid[(size_t)q], -1, -1, -1};
+    int m = 1;
+    for (int k : {0, 1, 2}) {
+      const int32_t r = idx[k][q];
+      if (r < 0 || r >= na) continue;
+      const int c = point_class(skip[r]);
+      if (c != 1 && c != 2) continue;
+      const int32_t t = ids.tid[(size_t)r];
+      if (std::find(seen, seen + m, t) == seen + m) seen[m++] = t;
     }
-    for (size_t t = 0; t < n.size(); ++t)
-      if (mine[t]) __atomic_fetch_add(&n[t], mine[t], __ATOMIC_RELAXED);
+    for (int i = 0; i < m; ++i) add(seen[i]);
   });
   return *std::max_element(n.begin(), n.end());
 }
@@ -495,7 +527,7 @@ TilePlan plan_tiles(int na, int navel, const int32_t *const idx[6], const uint8_
   std::vector<SlotMap> maps;
   maps.reserve((size_t)plan_threads());
   for (int w = 0; w < plan_threads(); ++w) maps.emplace_back();
-  par_items(nt, [&](int t, int w) {
+  par_items(nt, na, [&](int t, int w) {
     auto at = [&](int c, int half) { return start[((size_t)c * nt + t) * 2 + half]; };
     TileDesc &d = desc[(size_t)t];
     d = TileDesc{};
@@ -693,7 +725,7 @@ std::string check_plan(const TilePlan &p, int na, int navel, const int32_t *cons
   // every tile's table: bounds, entries and the LDS entry of every stepu read
   std::vector<std::string> err((size_t)p.tiles.size());
   std::vector<std::vector<int32_t>> emaps((size_t)plan_threads());
-  par_items((int)p.tiles.size(), [&](int t, int w) {
+  par_items((int)p.tiles.size(), na, [&](int t, int w) {
     const TileDesc &d = p.tiles[(size_t)t];
     std::string &e = err[(size_t)t];
     if (d.h0 < 0 || d.nh < 0 || (size_t)d.h0 + d.nh > p.list.size()) { e = "halo list range"; return; }
@@ -811,7 +843,7 @@ PairPlan plan_pairs(const TilePlan &p, int na, int navel, const int32_t *const i
     smaps.emplace_back();
     vmaps.emplace_back();
   }
-  par_items(nt, [&](int t, int w) {
+  par_items(nt, na, [&](int t, int w) {
     const TileDesc &d = p.tiles[(size_t)t];
     PairWork &wk = work[(size_t)t];
     SlotMap &sm = smaps[(size_t)w], &vm = vmaps[(size_t)w];
@@ -945,7 +977,7 @@ PairPlan plan_pairs(const TilePlan &p, int na, int navel, const int32_t *const i
   r.tnbr.resize(4 * nn);
   r.tsrc.resize(halo.n > 0 ? 4 * nn : 0);
   r.fix.resize(nf);
-  par_items(nt, [&](int t, int) {
+  par_items(nt, na, [&](int t, int) {
     const PairWork &wk = work[(size_t)t];
     const PairTile &pt = r.tiles[(size_t)t];
     std::copy(wk.x.begin(), wk.x.end(), r.xlist.begin() + pt.x0);
@@ -977,7 +1009,7 @@ std::string check_pairs(const PairPlan &q, const TilePlan &p, int na, int navel,
   auto slot = [&](int32_t r) { return r < na ? inv[(size_t)r] : r; };
   std::vector<std::string> err(q.tiles.size());
   std::vector<std::vector<int32_t>> smaps((size_t)plan_threads()), vmaps((size_t)plan_threads());
-  par_items((int)q.tiles.size(), [&](int t, int w) {
+  par_items((int)q.tiles.size(), na, [&](int t, int w) {
     const PairTile &pt = q.tiles[(size_t)t];
     const TileDesc &d = pt.t, &o = p.tiles[(size_t)t];
     std::string &e = err[(size_t)t];

@@ -135,6 +135,8 @@ TileIds tile_ids(int na, int navel, const int32_t *const idx[6], int tile_w, int
 // The largest number of stress points that a tile owns or evaluates as halo
 // (its level-2 entries in the pair form, one thread each) for these flags.
 int max_level2(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids);
+// max_level2 > most
+bool crowded(int na, const int32_t *const idx[6], const uint8_t *skip, const TileIds &ids, int most);
 
 // The pair form's tiles by domain size; *block: the workgroup size that one
 // subcycle per launch uses on the same tiles.
