@@ -197,11 +197,12 @@ void par_chunks(int64_t n, int64_t grain, F f) {
 }
 
 // f(i, w) for every i in [0, n), items handed out dynamically (uneven work);
-// work: the points of them all (fewer than 2048 a thread take less time than
-// its start: a first run's planning of 64x48 0.55 ms in place of 0.99)
+// work: the points of them all (fewer than 1024 a thread take less time than
+// its start: a first run's planning of 64x48 0.5 ms in place of 0.6
+// to 1.0)
 template <class F>
 void par_items(int n, int64_t work, F f) {
-  const int T = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(plan_threads(), n / 4), work / 2048));
+  const int T = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(plan_threads(), n / 4), work / 1024));
   if (T <= 1) {
     for (int i = 0; i < n; ++i) f(i, 0);
     return;
