@@ -42,6 +42,7 @@
 #include "evp1d_cache.hpp"
 #include "evp1d_hostmem.hpp"
 #include "evp1d_pair.hpp"
+#include "evp1d_par.hpp"
 #include "evp1d_point.hpp"
 #include "evp1d_tiles.hpp"
 #include "evp1d_xcd.hpp"
@@ -432,7 +433,8 @@ struct evp2d_handle {
   double2 *vel_alt = nullptr;
   // pair form: the planned 1D list of the cells and its tables
   bool pair_built = false, pair_ok = false;
-  int list_runs = 0;          // fused runs since the lists or the halo tables changed
+  long subs_done = 0;         // subcycles of fused runs since the lists or the halo tables changed
+  hipStream_t copies = nullptr;   // the plan's uploads, beside the run on `stream`
   int na = 0, nslots = 0;     // points, and with the unchanging cells that they read
   int t_end = 0, u_begin = 0, u_end = 0;
   int ptiles = 0, pblock = 0, pcap = 0, pcapv = 0, pnhalo = 0;
@@ -492,7 +494,7 @@ void free_lists2(evp2d_handle *h) {
   free_tiles2(h);
   free_pairs2(h);
   h->pair_built = false;
-  h->list_runs = 0;
+  h->subs_done = 0;
 }
 
 // Waits for the stream's copies when it goes out of scope: declared after the
@@ -511,6 +513,7 @@ void release2(evp2d_handle *h) {
   for (void *a : h->allocs) (void)hipFree(a);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
+  if (h->copies) (void)hipStreamDestroy(h->copies);
   if (h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
 }
@@ -643,16 +646,25 @@ int build_tiles2(evp2d_handle *h) {
 }
 
 // The pair form serves runs of at least kPairMinSub subcycles (it gathers and
-// scatters the state once per run) on lists that have been run before, or of
-// at least kPairFirstSub.  Its plan costs more host time than the
-// one-subcycle tables (at 1280x1520 about 40 ms more, against 26 us saved per
-// subcycle; at 800x600 10 ms against 5 us), so lists that are used for one
-// run, as when every model step has its own ice mask, are not planned.  The
-// contracted build keeps one subcycle per launch: its forms contract each in
-// its own way, and the first runs are never the pair form's.
-constexpr int kPairMinSub = 4, kPairFirstSub = 2000;
-bool wants_pair(const evp2d_handle *h, int nsub) {
-  return !EVP1D_FMA && nsub >= kPairMinSub && (h->list_runs > 0 || nsub >= kPairFirstSub);
+// scatters the state once per run) on lists that it has been planned for.  The
+// plan is host work that takes as long as about kPlanSubs subcycles of k2_fused
+// (16 threads: 45 ms against 93 us at 1280x1520, 15 against 27 at 800x600 in 2 x
+// 2 blocks, 3.5 against 5 at 200x150), and the pair form saves about a fourth of
+// each (64, 20 and 4.3 us).  So it is made beside a run, on the GPU meanwhile
+// that many of the run's subcycles, and only when it pays: lists used for one
+// run, as when every model step has its own ice mask, are planned only if that
+// run is long (kPairFirstSub: 216 -> 170 ms at 1280x1520), others when the
+// subcycles done and asked for have cost as much more as the GPU would have to
+// wait for the plan.  (Planned at the second run whatever its length, with the
+// GPU idle, 12 subcycles took 67 ms in place of 1.5 there.)  The contracted
+// build keeps one subcycle per launch: its forms contract each in their own way,
+// and the first runs are never the pair form's.
+constexpr int kPairMinSub = 4, kPlanSubs = 500, kPairFirstSub = 2000;
+bool takes_pairs(const evp2d_handle *h, int nsub) { return h->pair_ok && nsub >= kPairMinSub; }
+bool plans_pairs(const evp2d_handle *h, int nsub) {
+  if (EVP1D_FMA || h->pair_built || nsub < kPairMinSub) return false;
+  return nsub >= kPairFirstSub ||
+         (h->subs_done > 0 && h->subs_done + nsub >= 4 * (long)std::max(kPlanSubs - nsub, 0));
 }
 
 typedef void (*Pair2Fn)(PairView, PairBufs, int);
@@ -723,22 +735,39 @@ int build_pairs2(evp2d_handle *h) {
     idx[k] = nb[k].data();
   }
   std::vector<uint8_t> skip((size_t)na);
-  for (int p = 0; p < na; ++p) {
-    const long c = cell[(size_t)p], l = c % h->plane;
-    const int i = (int)(l % nxb), j = (int)(l / nxb);
-    const uint8_t m = mark[(size_t)c];
-    skip[(size_t)p] = (uint8_t)((m & kT ? 0 : 1) | (m & kU ? 0 : 2));
-    for (int k = 0; k < 6; ++k) {
-      const int ii = i + di[k], jj = j + dj[k];
-      int32_t q = dummy;
-      if (ii >= 0 && ii < nxb && jj >= 0 && jj < h->nyb) {
-        const long cc = c + dj[k] * (long)nxb + di[k];
-        q = pos[(size_t)cc];
-        if (q >= na || q < 0) q = k < 3 && (m & kT) ? ghost(cc) : dummy;   // str of other cells is zero
+  // with the cells' own coordinates, the blocks side by side
+  evp1d::GridCoords coords;
+  coords.ok = true;
+  coords.width = (int64_t)h->nblocks * (nxb + 1);
+  coords.height = h->nyb;
+  coords.gx.resize((size_t)na);
+  coords.gy.resize((size_t)na);
+  struct Read { int p, k; long cell; };   // neighbour k of point p, a cell outside the lists
+  std::vector<std::vector<Read>> reads((size_t)evp1d::plan_threads());
+  evp1d::par_chunks(na, 1 << 14, [&](int64_t lo, int64_t hi, int w) {
+    for (int64_t p = lo; p < hi; ++p) {
+      const long c = cell[(size_t)p], b = c / h->plane, l = c - b * h->plane;
+      const int j = (int)(l / nxb), i = (int)(l - (long)j * nxb);
+      const uint8_t m = mark[(size_t)c];
+      coords.gx[(size_t)p] = (int32_t)(b * (nxb + 1) + i);
+      coords.gy[(size_t)p] = (int32_t)j;
+      skip[(size_t)p] = (uint8_t)((m & kT ? 0 : 1) | (m & kU ? 0 : 2));
+      for (int k = 0; k < 6; ++k) {
+        const int ii = i + di[k], jj = j + dj[k];
+        int32_t q = dummy;   // str of cells outside the lists is zero
+        if (ii >= 0 && ii < nxb && jj >= 0 && jj < h->nyb) {
+          const long cc = c + dj[k] * (long)nxb + di[k];
+          if (pos[(size_t)cc] >= 0)
+            q = pos[(size_t)cc];
+          else if (k < 3 && (m & kT))
+            reads[(size_t)w].push_back({(int)p, k, cc});
+        }
+        nb[k][(size_t)p] = q;
       }
-      nb[k][(size_t)p] = q;
     }
-  }
+  });
+  for (const auto &r : reads)   // in the points' order
+    for (const Read &x : r) nb[x.k][(size_t)x.p] = ghost(x.cell);
   std::vector<int32_t> hdst, hsrc;   // by position; the cells that some point reads
   for (size_t k = 0; k < hd.size(); ++k) {
     const int32_t d = pos[(size_t)hd[k]];
@@ -747,18 +776,6 @@ int build_pairs2(evp2d_handle *h) {
     hsrc.push_back(hs[k] < 0 ? -1 : ghost(hs[k]));
   }
   const int nslots = (int)cell.size();
-  // the cells' own coordinates, the blocks side by side
-  evp1d::GridCoords coords;
-  coords.ok = true;
-  coords.width = (int64_t)h->nblocks * (nxb + 1);
-  coords.height = h->nyb;
-  coords.gx.resize((size_t)na);
-  coords.gy.resize((size_t)na);
-  for (int p = 0; p < na; ++p) {
-    const long c = cell[(size_t)p], l = c % h->plane;
-    coords.gx[(size_t)p] = (int32_t)((c / h->plane) * (nxb + 1) + l % nxb);
-    coords.gy[(size_t)p] = (int32_t)(l / nxb);
-  }
   int block1 = 0;
   evp1d::TileIds ids = evp1d::pair_tiles(coords, 0, &block1);
   if (ids.ntiles == 0) return EVP1D_OK;
@@ -786,7 +803,8 @@ int build_pairs2(evp2d_handle *h) {
   std::vector<int32_t> scell((size_t)nslots);
   for (int s = 0; s < nslots; ++s) scell[(size_t)s] = cell[(size_t)(s < na ? plan.perm[(size_t)s] : s)];
   const std::vector<int> zero(1, 0);
-  const CopiesDone copies{h->stream};
+  if (!h->copies) HIP2(hipStreamCreateWithFlags(&h->copies, hipStreamNonBlocking));
+  const CopiesDone copies{h->copies};
   auto get = [&](auto **dst, const void *src, size_t bytes) -> int {
     void *p = nullptr;
     if (hipMalloc(&p, std::max<size_t>(bytes, 256)) != hipSuccess) {
@@ -794,7 +812,7 @@ int build_pairs2(evp2d_handle *h) {
       return fail2(EVP1D_ENOMEM, "evp2d pair plan: hipMalloc(%zu)", bytes);
     }
     h->pbufs.push_back(p);
-    if (src && bytes) HIP2(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, h->stream));
+    if (src && bytes) HIP2(hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, h->copies));
     *dst = static_cast<std::remove_reference_t<decltype(*dst)>>(p);
     return EVP1D_OK;
   };
@@ -877,22 +895,19 @@ int ensure2_impl(evp2d_handle *h) {
   return EVP1D_OK;
 }
 
-// the tables of the form that a run of nsub subcycles takes
-int ensure_form2(evp2d_handle *h, int nsub) {
-  if (wants_pair(h, nsub) && !h->pair_built) {
-    const int rc = evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); });
-    if (rc) free_pairs2(h);
-    if (rc != EVP1D_ENOMEM) RC2(rc);   // one subcycle per launch needs less
-  }
-  const bool pair = wants_pair(h, nsub) && h->pair_ok;
-  if ((!pair || nsub % 2 == 1) && !h->tiles_built) {
+// the tables of one subcycle per launch
+int ensure_tiles2(evp2d_handle *h) {
+  if (!h->tiles_built) {
     const int rc = evp1d::no_throw("evp2d tiles", [h] { return build_tiles2(h); });
     if (rc) free_tiles2(h);
     RC2(rc);
   }
-  if ((!pair || nsub % 2 == 1) && !h->vel_alt)
-    HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
+  if (!h->vel_alt) HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
   return EVP1D_OK;
+}
+// the tables of the form that a run of nsub subcycles takes
+int ensure_form2(evp2d_handle *h, int nsub) {
+  return takes_pairs(h, nsub) && nsub % 2 == 0 ? EVP1D_OK : ensure_tiles2(h);
 }
 
 int launch_stress2(evp2d_handle *h) {
@@ -994,7 +1009,7 @@ int issue_fused2(evp2d_handle *h, int nsub) {
 // halo copies that some point reads are made by slot; after the run the halo
 // update of the block arrays sets the other halo cells too.
 int issue_run2(evp2d_handle *h, int nsub) {
-  if (!wants_pair(h, nsub) || !h->pair_ok) return issue_fused2(h, nsub);
+  if (!takes_pairs(h, nsub)) return issue_fused2(h, nsub);
   if (nsub % 2 == 1) RC2(issue_fused2(h, 1));
   const View2 &v = h->v;
   PairView f{};
@@ -1056,6 +1071,24 @@ int issue_run2(evp2d_handle *h, int nsub) {
                        (const double2 *)h->pvel[cur], h->pcell, h->u_begin, h->u_end);
   HIP2(hipGetLastError());
   return launch_halo2(h);
+}
+
+// A run of nsub subcycles with the pair form's plan made beside it: the first
+// ones, as many as the plan takes, run with k2_fused while the host plans, the
+// rest in the pair form.  Where the plan fails for lack of memory one subcycle
+// per launch stays the form of these lists.  Passes of 1000 subcycles on the
+// same lists at 1280x1520: 93 ms (and 31 for the lists' first tables), 79 with
+// the plan, then 64.
+int run_and_plan2(evp2d_handle *h, int nsub) {
+  RC2(ensure_tiles2(h));
+  int first = std::min(nsub, kPlanSubs);
+  first += (nsub - first) % 2;   // the pair form takes an even rest
+  RC2(issue_fused2(h, first));
+  h->graph_dirty = true;         // captured before the lists were planned
+  const int rc = evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); });
+  if (rc) free_pairs2(h);
+  if (nsub > first) RC2(issue_run2(h, nsub - first));
+  return rc == EVP1D_ENOMEM ? EVP1D_OK : rc;
 }
 
 // field id -> where it lives
@@ -1311,7 +1344,11 @@ int evp2d_run(evp2d_handle *h, int32_t nsub) {
   if (nsub == 0) return EVP1D_OK;
   RC2(ensure2(h));
   const bool fused = h->mode == EVP2D_MODE_FUSED;
-  if (fused && !h->pair_built && wants_pair(h, nsub)) h->graph_dirty = true;   // captured before the lists were planned
+  if (fused && plans_pairs(h, nsub)) {
+    RC2(run_and_plan2(h, nsub));
+    h->subs_done += nsub;
+    return EVP1D_OK;
+  }
   if (h->graph_dirty || h->graph_nsub != nsub || !h->exec) {
     drop_graph2(h);
     if (fused) RC2(ensure_form2(h, nsub));
@@ -1330,7 +1367,7 @@ int evp2d_run(evp2d_handle *h, int32_t nsub) {
     h->graph_dirty = false;
   }
   HIP2(hipGraphLaunch(h->exec, h->stream));
-  if (fused && h->list_runs < 1) ++h->list_runs;
+  if (fused) h->subs_done += nsub;
   return EVP1D_OK;
 }
 
@@ -1363,7 +1400,7 @@ int evp2d_set_cache_hints(evp2d_handle *h, int32_t hints) {
 int evp2d_get_cache_hints(evp2d_handle *h, int32_t *hints, int32_t *active) {
   if (!h) return fail2(EVP1D_EINVAL, "evp2d_get_cache_hints: NULL handle");
   RC2(ensure2(h));
-  if (h->mode == EVP2D_MODE_FUSED && active) RC2(ensure_form2(h, kPairMinSub));   // the form that runs use now
+  if (h->mode == EVP2D_MODE_FUSED && active) RC2(ensure_form2(h, kPairMinSub));   // the form that runs take now
   if (hints) *hints = h->cache_hints;
   if (active)
     *active = h->mode == EVP2D_MODE_FUSED && (h->pair_ok ? pair_hints2(h) : h->ntiles > 0 && hints2(h)) ? 1 : 0;

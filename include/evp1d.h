@@ -476,15 +476,18 @@ int evp2d_get_field(evp2d_handle *h, int32_t field, double *a, int64_t n);
 int evp2d_run(evp2d_handle *h, int32_t nsub);
 /* How evp2d_run runs the subcycles.  EVP2D_MODE_FUSED (default): two per
  * launch with the 1D engine's pair form (evp1d_set_fused_depth), on the cells
- * of the lists as a 1D list with the halo update as its copy list, when the
- * same lists are run again (their plan takes host time) or for 2000
- * subcycles and more; else, in libevp1d_fma.so (whose forms round
+ * of the lists as a 1D list with the halo update as its copy list, once the
+ * lists are planned for it; else, in libevp1d_fma.so (whose forms round
  * differently), and where the pair tables do not fit or stepu writes a cell
  * of the halo, one per launch: stress and stepu of one 32 x 8
  * tile of cells per workgroup with str1..8 in LDS (the T cells of the column
- * east and the row north of the tile evaluated again).  Velocities and
- * stresses alternate between two buffers.  EVP2D_MODE_PLAIN runs the two
- * kernels one after the other, as the reference does.  Results are
+ * east and the row north of the tile evaluated again).  The plan takes host
+ * time, about that of 500 subcycles on the GPU; it is made inside a run, while
+ * the GPU works on the run's first subcycles: in a run of 2000 or more, or in a
+ * later run on the same lists once the subcycles done and asked for pay for it
+ * (1000 at a time: the second run; 12 at a time: after 1900 subcycles).
+ * Velocities and stresses alternate between two buffers.  EVP2D_MODE_PLAIN runs
+ * the two kernels one after the other, as the reference does.  Results are
  * identical.                                                                */
 enum evp2d_mode { EVP2D_MODE_PLAIN = 0, EVP2D_MODE_FUSED = 1 };
 int evp2d_set_mode(evp2d_handle *h, int32_t mode);
