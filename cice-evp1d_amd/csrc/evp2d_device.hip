@@ -848,9 +848,6 @@ int build_pairs2(evp2d_handle *h) {
   h->nslots = nslots;
   h->pnhalo = (int)hdst.size();
   h->ptiles = (int)q.tiles.size();
-  for (const auto &kind : kPair2Fns[b])
-    for (Pair2Fn fn : kind)
-      HIP2(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
   h->pair_ok = true;
   return EVP1D_OK;
 }
@@ -905,8 +902,22 @@ int ensure_tiles2(evp2d_handle *h) {
   if (!h->vel_alt) HIP2(hipMalloc((void **)&h->vel_alt, (size_t)h->n * sizeof(double2)));
   return EVP1D_OK;
 }
-// the tables of the form that a run of nsub subcycles takes
+// Whether the pair form uses the cache hints, as for the 1D list (there the
+// stress constants are 56 B, here 80).
+bool pair_hints2(const evp2d_handle *h) {
+  if (h->cache_hints >= 0) return h->cache_hints != 0;
+  const double reread = 152.0 * (h->u_end - h->u_begin) + 16.0 * h->nslots;
+  return hints_pay(reread, reread + 272.0 * h->t_end);
+}
+Pair2Fn pair_fn2(const evp2d_handle *h) {
+  return kPair2Fns[pair_block_index(h->pblock)][h->pnhalo > 0 ? 1 : 0][pair_hints2(h) ? 1 : 0];
+}
+// The tables of the form that a run of nsub subcycles takes, and the LDS of its
+// kernel where that is more than every kernel may use: asking it for all four
+// kernels of a workgroup size made the first plan of a process 6 ms longer.
 int ensure_form2(evp2d_handle *h, int nsub) {
+  if (takes_pairs(h, nsub) && pair_lds(h->pcap, h->pcapv) > 64 * 1024)
+    HIP2(hipFuncSetAttribute((const void *)pair_fn2(h), hipFuncAttributeMaxDynamicSharedMemorySize, kPairMaxLds));
   return takes_pairs(h, nsub) && nsub % 2 == 0 ? EVP1D_OK : ensure_tiles2(h);
 }
 
@@ -956,13 +967,6 @@ bool hints2(const evp2d_handle *h) {
   if (h->cache_hints >= 0) return h->cache_hints != 0;
   const double reread = 100.0 * h->et + 124.0 * h->eu + 32.0 * h->n;
   return hints_pay(reread, reread + 192.0 * h->no);
-}
-// The pair form's, as for the 1D list (there the stress constants are 56 B,
-// here 80).
-bool pair_hints2(const evp2d_handle *h) {
-  if (h->cache_hints >= 0) return h->cache_hints != 0;
-  const double reread = 152.0 * (h->u_end - h->u_begin) + 16.0 * h->nslots;
-  return hints_pay(reread, reread + 272.0 * h->t_end);
 }
 
 // nsub fused subcycles.  The velocities start in the handle's buffer (X),
@@ -1044,9 +1048,7 @@ int issue_run2(evp2d_handle *h, int nsub) {
     hipLaunchKernelGGL(k2_pack_sig, dim3(blocks2(h->t_end)), dim3(kB2), 0, h->stream, (const double *)v.sig, h->n,
                        h->pcell, h->psig[0], (long)h->t_end);
   HIP2(hipGetLastError());
-  int b = 0;
-  while (kPairBlocks[b] != h->pblock) ++b;
-  const Pair2Fn fn = kPair2Fns[b][h->pnhalo > 0 ? 1 : 0][pair_hints2(h) ? 1 : 0];
+  const Pair2Fn fn = pair_fn2(h);
   const size_t lds = pair_lds(h->pcap, h->pcapv);
   int cur = 0;
   const int L = nsub / 2;
@@ -1087,7 +1089,10 @@ int run_and_plan2(evp2d_handle *h, int nsub) {
   h->graph_dirty = true;         // captured before the lists were planned
   const int rc = evp1d::no_throw("evp2d pair plan", [h] { return build_pairs2(h); });
   if (rc) free_pairs2(h);
-  if (nsub > first) RC2(issue_run2(h, nsub - first));
+  if (nsub > first) {
+    RC2(ensure_form2(h, nsub - first));
+    RC2(issue_run2(h, nsub - first));
+  }
   return rc == EVP1D_ENOMEM ? EVP1D_OK : rc;
 }
 
