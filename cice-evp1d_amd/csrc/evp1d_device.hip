@@ -511,12 +511,19 @@ constexpr int kFusedMinSub = 4;          // evp1d_run in AUTO mode: fused from t
 // run of this many subcycles, at the second run, or where the caller has set a
 // tile, an order or a depth since the last plan; a shorter first run (a
 // model step whose ice mask is new) goes over the points in class order, one
-// kernel for stress and one for stepu.  Planning takes 32 ms longer than the
-// class order at 1280x1520 and the tiles then save 57 us a subcycle (62
-// against 119): even at 560 subcycles, and at 550 for 2560x3040 (150 ms, 270
-// us), 500 for 64x48 (1.3 ms, 2.5 us), 1200 for 400x300 and 700x500 (5.5 and
-// 10 ms, 4.6 and 7.8 us).  A step of 240 subcycles at 1280x1520 with new
-// flags, fields in and out of 2D arrays: 65 -> 45 ms.
+// kernel for stress and one for stepu.  Planning takes 35 ms longer than the
+// class order at 1280x1520 and the tiles then save 52 us a subcycle (65
+// against 118): even at 660 subcycles, and at 490 for 2560x3040 (131 ms, 265
+// us), 310 for 64x48 (0.7 ms, 2.3 us), 750 to 1050 from 200x150 to 733x517 (4
+// to 8 ms, 4.8 to 8.8 us).  Between 500 and those a first run takes up to a
+// third longer than in class order, and later runs with its flags have the tiles.
+// A step of 240 subcycles at 1280x1520 with new flags, fields in and out of 2D
+// arrays: 65 -> 45 ms.
+// Where the last two sets of flags were each replaced before or each after this
+// many subcycles, the next is taken to be like them: not planned before it has
+// had as many, or at its first run.  Steps of two runs of 120 with new flags,
+// planned at the second run / so: 1280x1520 65 / 40 ms, 700x500 15 / 8.7,
+// 400x300 8.3 / 4.5.
 // The contracted build plans at the first run: there each form contracts in
 // its own way, and a state that goes on from a run in another form drifts from
 // the one it would have had (1e-13 after a run of 241 subcycles, up to 1e-7
@@ -1080,6 +1087,8 @@ struct evp1d_handle {
   bool layout_dirty = false;       // skip flags changed since the last relayout
   bool layout_tiled = false;       // the slot order was made with tiles (or none fit), not by class alone
   bool new_points = true;          // skip flags or lists changed since the last evp1d_run
+  long set_subs = 0;               // subcycles of the evp1d_run calls with these flags and lists
+  int habit = 0;                   // sets before these in a row that had kPlanSub subcycles (+) or fewer (-)
   bool tiles_asked = false;        // a tile, order or depth was set since tiles were last planned
   bool idx_dirty = false;          // slot-space lists need re-upload
   int mode = EVP1D_MODE_AUTO;
@@ -2357,9 +2366,17 @@ int evp1d_run(evp1d_handle *h, int32_t nsub) {
   if (!h) return fail(EVP1D_EINVAL, "evp1d_run: NULL handle");
   if (nsub < 0) return fail(EVP1D_EINVAL, "evp1d_run: nsub=%d < 0", nsub);
   if (!ready(h)) return fail(EVP1D_ESTATE, "evp1d_run: neighbour lists not set");
-  RC_TRY(ensure(h, h->mode != EVP1D_MODE_AUTO || !h->new_points || h->tiles_asked || nsub >= kPlanSub));
+  if (h->new_points && h->set_subs > 0) {
+    const bool enough = h->set_subs >= kPlanSub;
+    h->habit = std::max(-2, std::min(enough ? std::max(h->habit, 0) + 1 : std::min(h->habit, 0) - 1, 2));
+    h->set_subs = 0;
+  }
+  const bool tiles = h->mode != EVP1D_MODE_AUTO || h->tiles_asked || h->set_subs + nsub >= kPlanSub ||
+                     h->habit == 2 || (!h->new_points && h->habit > -2);
+  RC_TRY(ensure(h, tiles));
   if (nsub == 0 || h->na == 0) return EVP1D_OK;
   h->new_points = false;
+  h->set_subs += nsub;
   switch (h->mode) {
     case EVP1D_MODE_LAUNCH: return issue_subcycles(h, nsub);
     case EVP1D_MODE_PERSISTENT: return run_persistent(h, nsub);
@@ -2369,7 +2386,7 @@ int evp1d_run(evp1d_handle *h, int32_t nsub) {
     case EVP1D_MODE_GRAPH: return run_graph(h, nsub, false);
     case EVP1D_MODE_AUTO:
     default:
-      // these flags' first, short run: a captured graph would serve it only
+      // these flags' short run: a captured graph would serve it only
       if (!h->layout_tiled) return issue_subcycles(h, nsub);
       // the fused form copies the state once per run (two buffers), which
       // only pays off over several subcycles

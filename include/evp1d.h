@@ -112,7 +112,9 @@ enum evp1d_mode {
                                  LAUNCH for the first run with new skip flags or lists if it is shorter
                                  than 500 subcycles (tiles are planned at the second run, for a long one,
                                  or where evp1d_set_tiling, evp1d_set_tile_order, evp1d_set_fused_depth
-                                 or a tuner has changed them since the last plan;
+                                 or a tuner has changed them since the last plan; where the last two sets
+                                 of flags each had fewer than 500 subcycles, not before the new one has
+                                 had 500, and at its first run where each had more;
                                  libevp1d_fma.so, whose forms round differently, plans at the first) */
   EVP1D_MODE_FUSED = 4        /* one launch per subcycle: stress and stepu per tile of points, str1..8
                                  kept on chip (hipGraph); needs lists that describe a grid */

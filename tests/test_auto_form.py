@@ -87,3 +87,30 @@ def test_tiles_planned_by_a_getter_are_what_the_first_run_takes(fake, st):
     with make_engine(st, 120) as eng:
         assert eng.get_fused_depth()["active"]
         assert _run(eng, fake) == "pairs"
+
+
+def _sets(eng, fake, st, runs, sets):
+    """Forms of the runs of each of `sets` model steps, each with flags of its own."""
+    forms = []
+    for k in range(sets):
+        flags = st.skipT.copy()
+        flags[k] ^= 1
+        eng.set_skip("skipT", flags)
+        forms.append([_run(eng, fake, n) for n in runs])
+    return forms
+
+
+def test_steps_of_several_short_runs(fake, st):
+    with make_engine(st, 120) as eng:
+        once, never = ["class order", "pairs"], ["class order", "class order"]
+        assert _sets(eng, fake, st, [120, 120], 5) == [once, once, never, never, never]
+        assert [_run(eng, fake, 120) for _ in range(4)] == ["class order", "class order", "pairs", "pairs"]
+        # a set that had enough for a plan: the second run of the next one plans again
+        assert _sets(eng, fake, st, [120, 120], 1) == [once]
+
+
+def test_steps_of_several_runs_long_enough_together(fake, st):
+    with make_engine(st, 120) as eng:
+        second, first = ["class order", "pairs"], ["pairs", "pairs"]
+        assert _sets(eng, fake, st, [300, 200], 4) == [second, second, first, first]
+        assert _sets(eng, fake, st, [120, 120], 2) == [first, second]
