@@ -240,7 +240,6 @@ __device__ __forceinline__ void pair_tile(const PairView &f, PairBufs bf, int la
     if (TRAJ && k < nUo) out2<NT>(f.tr_mid + (q - f.u_begin), vt[k]);
   }
   // level 2, stress of entry me: memory inputs loaded before the barrier
-  // (velocities that are no U1 entry never change, kNoEntry: from memory)
   // (velocities that are no U1 entry never change, kNoEntry: from memory;
   // a ghost on the copy list whose source is no U1 entry: kFixBase + j, the
   // source's unchanging velocity or zero)

@@ -332,10 +332,11 @@ __global__ __launch_bounds__(kB2F) void k2_fused(View2 v, Fused2 f, int last) {
 // tile), with the neighbours at the cell offsets and the halo update as its
 // copy list, so the planner, the tiles and the kernel are the 1D engine's.
 // What changes during a run lives by slot: velocities and stresses, gathered
-// from the block arrays before the run and scattered after it.  As in the 1D
-// list the kernel is bound by the latency of its phases at 16 waves per CU,
-// with half the bytes of k2_fused: 1280x1520 in one block, 1000 subcycles,
-// 88 -> 65 us per subcycle; 800x600 in 2 x 2 blocks, 120 subcycles, 26.7 ->
+// from the block arrays before the run and scattered after it.  As the 1D
+// list's, the kernel moves its bytes close to the streaming rate (689 MB a
+// launch at 5.3 of 5.67 TB/s), with what the loads of 16 waves per CU keep in
+// flight, and two thirds of k2_fused's per subcycle: 1280x1520 in one block,
+// 91 -> 64.5 us per subcycle; 800x600 in 2 x 2 blocks, 120 subcycles, 26.7 ->
 // 20.6 us, where the halo update was four launches per two subcycles, and is
 // none after the second launch of a run: the tables name a halo cell's source
 // in its place (0.9 us a subcycle less than one copy per launch).

@@ -250,7 +250,9 @@ int evp1d_get_tuning(const evp1d_handle *h, int32_t *stress_block, int32_t *stre
  * on 256 if at least 512, else 16x8 on 128 (XCD-aware order).
  * evp1d_get_tiling reports the tiling and the number of tiles (0 when the
  * lists do not describe a grid: the fused form is then unavailable).
- * Results never depend on the tiling.                                       */
+ * Results of libevp1d.so never depend on the tiling.  In libevp1d_fma.so each
+ * kernel variant contracts in its own way: a tile that takes another variant
+ * can change the last bits (relative 3e-17 at 733x517).                     */
 int evp1d_set_tiling(evp1d_handle *h, int32_t tile_w, int32_t tile_h, int32_t block, int32_t xcd);
 int evp1d_get_tiling(evp1d_handle *h, int32_t *tile_w, int32_t *tile_h, int32_t *block, int32_t *xcd,
                      int32_t *ntiles);
@@ -376,8 +378,8 @@ int evp1d_loss_noalloc(evp1d_handle *h, const double *u_target, const double *v_
  * from the stored state.  seg = 0 (default): ceil(nsub / nsnap), made even in
  * the pair form when nsub is even, which stores every unit start and
  * recomputes each unit once, when that trajectory fits in free device memory
- * beside the stored states, else 1.  The gradient is the same bit for bit for
- * every seg and nsnap.                                                      */
+ * beside the stored states, else 1.  In libevp1d.so the gradient is the same
+ * bit for bit for every seg and nsnap.                                      */
 int evp1d_set_adjoint_segment(evp1d_handle *h, int32_t seg);
 int evp1d_get_adjoint_segment(evp1d_handle *h, int32_t *seg);
 /* Device memory that gradient and tangent calls keep with the handle (no
